@@ -24,8 +24,11 @@ struct Levels {
 
 // Scratch for two-stage reductions.
 struct Work {
-    double* part = nullptr;  // [1024][64]
+    double* part = nullptr;  // [kPartSize]
 };
+
+// 1024 workgroups' partials of the 2 KMAX projection values of one step
+constexpr size_t kPartSize = (size_t)1024 * 2 * KMAX;
 
 struct GmresScalars;
 
@@ -132,7 +135,7 @@ struct FgmresArgs {
 int reduceBlocks(int nC);
 // Full 5x5 off-diagonal blocks (sliced layout) from generator storage.
 void launchExpandBlocks(const MeshView& m, int fp32, const void* gen, void* out, hipStream_t st);
-void launchProjectionPasses(const MeshView& m, int vecFp32, int ch, const void* w, const void* V, int nv,
+void launchProjectionPasses(const MeshView& m, int vecFp32, int ch, int mgs, const void* w, const void* V, int nv,
                             double* part, hipStream_t st);
 
 void launchUpdate(const MeshView& m, const Phys& ph, const StateView& s, const double* dW, int mode,

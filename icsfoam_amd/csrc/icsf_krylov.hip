@@ -609,114 +609,70 @@ __global__ void __launch_bounds__(256) k_norm2(int nC, const TV* __restrict__ x,
     blockReduceStore<1>(v, part);
 }
 
-// CGS projection partials: <w, V_j> for j < nv (nv <= 64, chunked by 16).
-// The basis vectors are streamed with non-temporal loads here and in the
-// update and combine kernels: each is read once per pass and the passes
-// between two reads of one vector move far more than L2 holds.
-template <typename TV, int CH>
-__global__ void __launch_bounds__(256) k_multidot(int nC, const TV* __restrict__ w, const TV* __restrict__ Vb,
-                                                  size_t vstride, int j0, int nv, double* __restrict__ part) {
-    double v[CH];
+// Projection partials of one Arnoldi step: <w, V_j> for j < nv = i + 1, and
+// with WY (modified Gram-Schmidt) <v_i, V_k> for k < i from the same loads,
+// blockIdx.y = a chunk of CH basis vectors.  Value q's partials are
+// contiguous (part + q * gridDim.x): projections q = j, Gram values
+// q = KMAX + k.  The basis vectors are streamed with non-temporal loads here
+// and in the update and combine kernels: each is read once per pass and the
+// passes between two reads of one vector move far more than L2 holds.
+template <typename TV, int CH, bool WY>
+__global__ void __launch_bounds__(256) k_project(int nC, const TV* __restrict__ w, const TV* __restrict__ Vb,
+                                                 size_t vstride, int nv, double* __restrict__ part) {
+    constexpr int NA = WY ? 2 * CH : CH;
+    const int j0 = blockIdx.y * CH;
+    const TV* vi = Vb + (size_t)(nv - 1) * vstride;
+    double v[NA];
 #pragma unroll
-    for (int k = 0; k < CH; ++k) v[k] = 0;
+    for (int k = 0; k < NA; ++k) v[k] = 0;
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nC; c += gridDim.x * blockDim.x) {
-        TV wv[5];
+        TV wv[5], vv[5];
 #pragma unroll
-        for (int q = 0; q < 5; ++q) wv[q] = w[(size_t)q * nC + c];
+        for (int q = 0; q < 5; ++q) {
+            wv[q] = w[(size_t)q * nC + c];
+            if (WY) vv[q] = vi[(size_t)q * nC + c];
+        }
 #pragma unroll
         for (int k = 0; k < CH; ++k) {
-            if (k < nv) {
+            if (j0 + k < nv) {
                 const TV* vj = Vb + (size_t)(j0 + k) * vstride;
-                double s = 0;
+                double s = 0, g = 0;
 #pragma unroll
-                for (int q = 0; q < 5; ++q) s += (double)(wv[q] * __builtin_nontemporal_load(vj + (size_t)q * nC + c));
+                for (int q = 0; q < 5; ++q) {
+                    const TV x = __builtin_nontemporal_load(vj + (size_t)q * nC + c);
+                    s += (double)(wv[q] * x);
+                    if (WY) g += (double)(vv[q] * x);
+                }
                 v[k] += s;
+                if (WY) v[CH + k] += g;
             }
         }
     }
-    blockReduceStore<CH>(v, part);
-}
-
-// CGS projections of one pass over w: ch (8, 16 or 32) basis vectors.
-template <typename TV>
-void launchMultidot(int ch, int nbk, int nC, const TV* w, const TV* V, size_t vs, int j0, int nv, double* part,
-                    hipStream_t st) {
-    if (ch == 8) k_multidot<TV, 8><<<nbk, 256, 0, st>>>(nC, w, V, vs, j0, nv, part);
-    else if (ch == 32) k_multidot<TV, 32><<<nbk, 256, 0, st>>>(nC, w, V, vs, j0, nv, part);
-    else k_multidot<TV, 16><<<nbk, 256, 0, st>>>(nC, w, V, vs, j0, nv, part);
-}
-
-// w -= sum_j h_j V_j (j < nv), then ||w||^2 partials
-template <typename TV>
-__global__ void __launch_bounds__(256) k_cgs_update(int nC, TV* __restrict__ w, const TV* __restrict__ Vb,
-                                                    size_t vstride, int nv, const double* __restrict__ h,
-                                                    double* __restrict__ part) {
-    double v[1] = {0};
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nC; c += gridDim.x * blockDim.x) {
-        // five independent chains (one per component), basis vectors in
-        // order j = 0..nv-1 on each; four basis vectors' loads in flight
-        TV a[5];
+    __shared__ double sh[4][NA];
+    const int lane = threadIdx.x & 63, wvi = threadIdx.x >> 6;
 #pragma unroll
-        for (int q = 0; q < 5; ++q) a[q] = w[(size_t)q * nC + c];
-        int j = 0;
-        for (; j + 4 <= nv; j += 4) {
-            TV x[4][5];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int q = 0; q < 5; ++q)
-                    x[u][q] = __builtin_nontemporal_load(Vb + (size_t)(j + u) * vstride + (size_t)q * nC + c);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const TV hj = (TV)h[j + u];
-#pragma unroll
-                for (int q = 0; q < 5; ++q) a[q] -= hj * x[u][q];
-            }
-        }
-        for (; j < nv; ++j) {
-            const TV hj = (TV)h[j];
-#pragma unroll
-            for (int q = 0; q < 5; ++q) a[q] -= hj * Vb[(size_t)j * vstride + (size_t)q * nC + c];
-        }
-#pragma unroll
-        for (int q = 0; q < 5; ++q) {
-            w[(size_t)q * nC + c] = a[q];
-            v[0] += (double)a[q] * (double)a[q];
-        }
+    for (int k = 0; k < NA; ++k) {
+        const double t = waveSum(v[k]);
+        if (lane == 0) sh[wvi][k] = t;
     }
-    blockReduceStore<1>(v, part);
+    __syncthreads();
+    if (threadIdx.x < NA) {
+        const int k = threadIdx.x, j = j0 + (k < CH ? k : k - CH);
+        if (j < nv)
+            part[(size_t)(k < CH ? j : KMAX + j) * gridDim.x + blockIdx.x] =
+                ((sh[0][k] + sh[1][k]) + sh[2][k]) + sh[3][k];
+    }
 }
 
-// MGS step: (optionally) w -= h * V_prev, then partials of <w, V_next>
-// (5 per-variable partial sums, combined in the reference's order on reduce)
-template <typename TV>
-__global__ void __launch_bounds__(256) k_mgs_step(int nC, TV* __restrict__ w, const TV* __restrict__ Vprev,
-                                                  const double* __restrict__ hprev, const TV* __restrict__ Vnext,
-                                                  int wantNorm, double* __restrict__ part) {
-    double v[3] = {0, 0, 0};
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nC; c += gridDim.x * blockDim.x) {
-        TV a[5];
-#pragma unroll
-        for (int q = 0; q < 5; ++q) {
-            a[q] = w[(size_t)q * nC + c];
-            if (Vprev) {
-                a[q] -= (TV)(*hprev) * Vprev[(size_t)q * nC + c];
-                w[(size_t)q * nC + c] = a[q];
-            }
-        }
-        if (Vnext) {
-            v[0] += (double)(a[0] * Vnext[c]);
-            v[1] += (double)(a[1] * Vnext[(size_t)nC + c]);
-            v[2] += (double)(a[2] * Vnext[2 * (size_t)nC + c] + a[3] * Vnext[3 * (size_t)nC + c] +
-                             a[4] * Vnext[4 * (size_t)nC + c]);
-        }
-        if (wantNorm) {
-            v[0] += (double)(a[0] * a[0]);
-            v[1] += (double)(a[1] * a[1]);
-            v[2] += (double)(a[2] * a[2] + a[3] * a[3] + a[4] * a[4]);
-        }
-    }
-    blockReduceStore<3>(v, part);
+// All projections of one Arnoldi step, ch (8, 16 or 32) basis vectors per
+// workgroup.
+template <typename TV, bool WY>
+void launchProject(int ch, int nbk, int nC, const TV* w, const TV* V, size_t vs, int nv, double* part,
+                   hipStream_t st) {
+    const dim3 g(nbk, (nv + ch - 1) / ch);
+    if (ch == 8) k_project<TV, 8, WY><<<g, 256, 0, st>>>(nC, w, V, vs, nv, part);
+    else if (ch == 32) k_project<TV, 32, WY><<<g, 256, 0, st>>>(nC, w, V, vs, nv, part);
+    else k_project<TV, 16, WY><<<g, 256, 0, st>>>(nC, w, V, vs, nv, part);
 }
 
 // x = y - avg (component-wise); dW = 0 afterwards is done by memset.
@@ -766,13 +722,15 @@ __global__ void __launch_bounds__(256) k_update_sol(int nC, TX* __restrict__ dW,
 // ------------------------------------------------------------ GMRES state --
 // Scalars of one GMRES(m) cycle kept on the device (no host round trips).
 struct GmresScalars {
-    double H[KMAX][KMAX];
-    double cs[KMAX], sn[KMAX], bh[KMAX + 1], yh[KMAX];
+    double H[KMAX][KMAX];   // projections of column i: H[j][i], j <= i
+    double hn[KMAX + 1];    // ||r|| of the cycle's start, then ||w_i|| after the orthogonalisation
+    double T[KMAX][KMAX];   // modified Gram-Schmidt: unit lower triangular, (I + L)^-1 (orthCoeffs)
+    double s[2 * KMAX];     // reduced projections (and Gram values) of the current step
+    double yh[KMAX];
     double beta;
     double sNF[2], vNF;
     double res[10];   // sInit[2] vInit[3] sFinal[2] vFinal[3]
     double red[64];   // scratch reduction results
-    double hcol[KMAX];  // contiguous copy of the current Hessenberg column
 };
 
 namespace {
@@ -803,94 +761,155 @@ __global__ void k_gm_init(GmresScalars* g) {
     for (int k = 0; k < 5; ++k) g->res[5 + k] = g->res[k];
 }
 
-// beta = ||r|| at the start of a cycle
-__global__ void k_gm_beta0(GmresScalars* g, int nDirs) {
-    if (threadIdx.x != 0) return;
-    g->beta = sqrt(g->red[0]);
-    for (int i = 0; i <= nDirs; ++i) g->bh[i] = 0;
-    g->bh[0] = g->beta;
-}
-
-// Apply the previous rotations to column i of H, form the new rotation and
-// update bh (gmres.C:999-1027); beta2 = ||w||^2 after the orthogonalisation.
-// The block's threads stage column i and the previous rotations in LDS, so
-// that the chain of dependent updates run by one thread waits on LDS, not
-// on device memory.  Called by all threads of the block.
-__device__ void givensBlock(GmresScalars* g, int i, double beta2) {
-    __shared__ double hc[KMAX], cc[KMAX], ss[KMAX];
-    for (int t = threadIdx.x; t <= i; t += blockDim.x) hc[t] = g->H[t][i];
-    for (int t = threadIdx.x; t < i; t += blockDim.x) {
-        cc[t] = g->cs[t];
-        ss[t] = g->sn[t];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const double beta = sqrt(beta2);
-        for (int j = 0; j < i; ++j) {
-            const double Hji = hc[j];
-            hc[j] = cc[j] * Hji - ss[j] * hc[j + 1];
-            hc[j + 1] = ss[j] * Hji + cc[j] * hc[j + 1];
-        }
-        double ci, si;
-        givensRot(hc[i], beta, ci, si);
-        g->cs[i] = ci;
-        g->sn[i] = si;
-        const double bhi = g->bh[i];
-        const double bhn = g->bh[i + 1];
-        g->bh[i] = ci * bhi - si * bhn;
-        g->bh[i + 1] = si * bhi + ci * bhn;
-        hc[i] = ci * hc[i] - si * beta;
-        g->beta = beta;
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t <= i; t += blockDim.x) g->H[t][i] = hc[t];
-}
-
-// CGS projections of one multidot pass (partial rows of ch values): value
-// k = blockIdx.x (grid nv) is stored as H[j0+k][i] and hcol[j0+k].
-__global__ void __launch_bounds__(256) k_reduce_col(const double* __restrict__ part, int nb, int ch,
-                                                    GmresScalars* g, int i, int j0) {
-    const int k = blockIdx.x;
-    const double s = sumPartials(part, nb, ch, k);
-    if (threadIdx.x == 0) {
-        g->red[k] = s;
-        g->H[j0 + k][i] = s;
-        g->hcol[j0 + k] = s;
-    }
-}
-
-// ||w||^2 of the CGS update pass, then the Givens step (one block).
-__global__ void __launch_bounds__(256) k_reduce_givens(const double* __restrict__ part, int nb, GmresScalars* g,
-                                                       int i) {
+// beta = ||r|| (slot 0, a cycle's start) or ||w_i|| (slot i + 1) from the
+// norm partials (one block).
+__global__ void __launch_bounds__(256) k_reduce_norm(const double* __restrict__ part, int nb, GmresScalars* g,
+                                                     int slot) {
     const double s = sumPartials(part, nb, 1, 0);
-    if (threadIdx.x == 0) g->red[0] = s;
-    givensBlock(g, i, s);
-}
-
-// MGS step j of column i: the three per-variable partial sums of <w, V_j>
-// (j <= i, stored as H[j][i]) or of ||w||^2 (j = i+1, then the Givens
-// step), combined in the reference's order (one block).
-__global__ void __launch_bounds__(256) k_reduce_mgs(const double* __restrict__ part, int nb, GmresScalars* g, int i,
-                                                    int j) {
-    double s[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) s[k] = sumPartials(part, nb, 3, k);
-    const double hs = (0.0 + s[0] + s[1]) + s[2];
     if (threadIdx.x == 0) {
-        for (int k = 0; k < 3; ++k) g->red[k] = s[k];
-        if (j <= i) g->H[j][i] = hs;
+        const double beta = sqrt(s);
+        g->beta = beta;
+        g->hn[slot] = beta;
     }
-    if (j > i) givensBlock(g, i, hs);
 }
 
-__global__ void k_gm_backsub(GmresScalars* g, int n) {
-    if (threadIdx.x != 0) return;
+// Sums of the projection partials, one block per value: projections
+// (blockIdx.x < nv), then the Gram values.
+__global__ void __launch_bounds__(256) k_reduce_proj(const double* __restrict__ part, int nb, GmresScalars* g,
+                                                     int nv) {
+    const int q = (int)blockIdx.x < nv ? (int)blockIdx.x : KMAX + (int)blockIdx.x - nv;
+    const double s = sumPartials(part + (size_t)q * nb, nb, 1, 0);
+    if (threadIdx.x == 0) g->s[q] = s;
+}
+
+// Coefficients h (LDS, KMAX) with which w loses its projections on v_0..v_i,
+// from the reduced sums s_j = <w, V_j>; called by all threads of a block.
+// Classical Gram-Schmidt: h = s.  Modified Gram-Schmidt subtracts h_j v_j one
+// after the other, h_j = <w - sum_{k<j} h_k v_k, v_j>, which is the forward
+// substitution (I + L) h = s with L_jk = <v_j, v_k>, k < j (the inverse
+// compact WY form of the product of the projectors): one pass over the
+// basis instead of i + 1, and one reduction.  T = (I + L)^-1 of the earlier
+// rows is kept, so the substitution is a product without a serial chain;
+// row i of T follows from L_i, the Gram values that came with s.  Block 0
+// stores column i of H and row i of T.
+template <bool WY>
+__device__ void orthCoeffs(GmresScalars* g, int i, double* h) {
+    __shared__ double s[KMAX], l[KMAX];
+    const int t = threadIdx.x;
+    if (t <= i) s[t] = g->s[t];
+    if (WY && t < i) l[t] = g->s[KMAX + t];
+    __syncthreads();
+    if (WY) {
+        double a = 0;
+        if (t < i)
+            for (int k = 0; k <= t; ++k) a += g->T[t][k] * s[k];
+        if (t < i) h[t] = a;
+        __syncthreads();
+        if (t == i) {
+            a = s[i];
+            for (int k = 0; k < i; ++k) a -= l[k] * h[k];
+            h[i] = a;
+        }
+        if (blockIdx.x == 0 && t <= i) {
+            double r = t == i ? 1.0 : 0.0;
+            for (int k = t; k < i; ++k) r -= l[k] * g->T[k][t];
+            g->T[i][t] = r;
+        }
+    } else if (t <= i) h[t] = s[t];
+    __syncthreads();
+    if (blockIdx.x == 0 && t <= i) g->H[t][i] = h[t];
+}
+
+// w -= sum_j h_j V_j (j <= i), then ||w||^2 partials
+template <typename TV, bool WY>
+__global__ void __launch_bounds__(256) k_orth_update(int nC, TV* __restrict__ w, const TV* __restrict__ Vb,
+                                                     size_t vstride, GmresScalars* g, int i,
+                                                     double* __restrict__ part) {
+    __shared__ double h[KMAX];
+    orthCoeffs<WY>(g, i, h);
+    const int nv = i + 1;
+    double v[1] = {0};
+    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nC; c += gridDim.x * blockDim.x) {
+        // five independent chains (one per component), basis vectors in
+        // order j = 0..nv-1 on each; four basis vectors' loads in flight
+        TV a[5];
+#pragma unroll
+        for (int q = 0; q < 5; ++q) a[q] = w[(size_t)q * nC + c];
+        int j = 0;
+        for (; j + 4 <= nv; j += 4) {
+            TV x[4][5];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int q = 0; q < 5; ++q)
+                    x[u][q] = __builtin_nontemporal_load(Vb + (size_t)(j + u) * vstride + (size_t)q * nC + c);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const TV hj = (TV)h[j + u];
+#pragma unroll
+                for (int q = 0; q < 5; ++q) a[q] -= hj * x[u][q];
+            }
+        }
+        for (; j < nv; ++j) {
+            const TV hj = (TV)h[j];
+#pragma unroll
+            for (int q = 0; q < 5; ++q) a[q] -= hj * Vb[(size_t)j * vstride + (size_t)q * nC + c];
+        }
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+            w[(size_t)q * nC + c] = a[q];
+            v[0] += (double)a[q] * (double)a[q];
+        }
+    }
+    blockReduceStore<1>(v, part);
+}
+
+// End of a cycle (one wavefront, lane = column): the Givens rotations of the
+// n columns of H with sub-diagonal hn (gmres.C:999-1027) and the back
+// substitution into yh.  Step k's rotation is formed by lane k and applied
+// to all later columns at once, from LDS: 30 directions take 30 short steps
+// instead of the 435 dependent column updates of one thread.
+__global__ void __launch_bounds__(64) k_gm_finish(GmresScalars* g, int n) {
+    __shared__ double Hs[KMAX + 1][KMAX];
+    __shared__ double bh[KMAX + 1], rot[2];
+    const int t = threadIdx.x;
+    if (t < n) {
+        for (int j = 0; j <= t; ++j) Hs[j][t] = g->H[j][t];
+        Hs[t + 1][t] = g->hn[t + 1];
+        bh[t + 1] = 0;
+    }
+    if (t == 0) bh[0] = g->hn[0];
+    __syncthreads();
+    for (int k = 0; k < n; ++k) {
+        if (t == k) {
+            double c, s;
+            const double beta = Hs[k + 1][k];
+            givensRot(Hs[k][k], beta, c, s);
+            Hs[k][k] = c * Hs[k][k] - s * beta;
+            const double b0 = bh[k], b1 = bh[k + 1];
+            bh[k] = c * b0 - s * b1;
+            bh[k + 1] = s * b0 + c * b1;
+            rot[0] = c;
+            rot[1] = s;
+        }
+        __syncthreads();
+        if (t > k && t < n) {
+            const double a = Hs[k][t], b = Hs[k + 1][t];
+            Hs[k][t] = rot[0] * a - rot[1] * b;
+            Hs[k + 1][t] = rot[1] * a + rot[0] * b;
+        }
+        __syncthreads();
+    }
     for (int i = n - 1; i >= 0; --i) {
-        double s = g->bh[i];
-        for (int j = i + 1; j < n; ++j) s -= g->H[i][j] * g->yh[j];
-        double hd = g->H[i][i];
-        hd = hd >= 0 ? hd + kVSMALL : hd - kVSMALL;
-        g->yh[i] = s / hd;
+        if (t == i) {
+            double hd = Hs[i][i];
+            hd = hd >= 0 ? hd + kVSMALL : hd - kVSMALL;
+            rot[0] = bh[i] / hd;
+            g->yh[i] = rot[0];
+        }
+        __syncthreads();
+        if (t < i) bh[t] -= Hs[t][i] * rot[0];
+        __syncthreads();
     }
 }
 
@@ -907,16 +926,18 @@ __global__ void k_gm_final(GmresScalars* g, int emptyDir) {
 // --------------------------------------------------------------- host side --
 static inline int nb(size_t n, int b) { return (int)((n + b - 1) / b); }
 
-// The CGS projection passes of one Arnoldi step against nv basis vectors,
-// ch vectors per pass (autotuner timing).
-void launchProjectionPasses(const MeshView& m, int vecFp32, int ch, const void* w, const void* V, int nv,
+// The projection pass of one Arnoldi step against nv basis vectors, ch
+// vectors per workgroup (autotuner timing).
+void launchProjectionPasses(const MeshView& m, int vecFp32, int ch, int mgs, const void* w, const void* V, int nv,
                             double* part, hipStream_t st) {
     const int nC = m.nC, nbk = reduceBlocks(nC);
     const size_t vs = (size_t)5 * nC;
-    for (int j0 = 0; j0 < nv; j0 += ch) {
-        const int n = (nv - j0) < ch ? (nv - j0) : ch;
-        if (vecFp32) launchMultidot<float>(ch, nbk, nC, (const float*)w, (const float*)V, vs, j0, n, part, st);
-        else launchMultidot<double>(ch, nbk, nC, (const double*)w, (const double*)V, vs, j0, n, part, st);
+    if (vecFp32) {
+        if (mgs) launchProject<float, true>(ch, nbk, nC, (const float*)w, (const float*)V, vs, nv, part, st);
+        else launchProject<float, false>(ch, nbk, nC, (const float*)w, (const float*)V, vs, nv, part, st);
+    } else {
+        if (mgs) launchProject<double, true>(ch, nbk, nC, (const double*)w, (const double*)V, vs, nv, part, st);
+        else launchProject<double, false>(ch, nbk, nC, (const double*)w, (const double*)V, vs, nv, part, st);
     }
 }
 
@@ -1043,6 +1064,31 @@ void launchJacobiApply(int nC, int blkFp32, int vecFp32, const void* dinv, void*
     else k_jacobi_apply<double, double><<<nb(nC, 256), 256, 0, st>>>(nC, (const double*)dinv, (double*)r);
 }
 
+// Orthogonalisation of w against v_0..v_i (V): projections, their reduction,
+// the update with ||w||, and its reduction (beta).  Four launches for both
+// Gram-Schmidt forms; modified Gram-Schmidt step by step took 2 (i + 2)
+// launches and 4 (i + 1) vector passes where this takes 2 i + 6 (200x50x1
+// cells, GMRES(30): 990 of the cycle's 1110 launches).  Pseudo-steps with
+// modified Gram-Schmidt, FP64: 200x50x1 3.83 -> 1.34 ms, 53x42x39 viscous
+// 5.69 -> 2.86 ms; classical, 64^3: 5.89 -> 5.39 ms (one projection launch
+// for all chunks, the Givens chain once per cycle).
+template <typename TV>
+static void orthStep(const MeshView& m, int orth, int nC, TV* w, const TV* V, int i, GmresScalars* g, double* part,
+                     hipStream_t st) {
+    const int nbk = reduceBlocks(nC);
+    const size_t vs = (size_t)5 * nC;
+    if (orth == 0) {
+        launchProject<TV, true>(m.mdCh, nbk, nC, w, V, vs, i + 1, part, st);
+        k_reduce_proj<<<2 * i + 1, 256, 0, st>>>(part, nbk, g, i + 1);
+        k_orth_update<TV, true><<<nbk, 256, 0, st>>>(nC, w, V, vs, g, i, part);
+    } else {
+        launchProject<TV, false>(m.mdCh, nbk, nC, w, V, vs, i + 1, part, st);
+        k_reduce_proj<<<i + 1, 256, 0, st>>>(part, nbk, g, i + 1);
+        k_orth_update<TV, false><<<nbk, 256, 0, st>>>(nC, w, V, vs, g, i, part);
+    }
+    k_reduce_norm<<<1, 256, 0, st>>>(part, nbk, g, i + 1);
+}
+
 // --------------------------------------------------------- GMRES driver --
 template <typename TV>
 void gmresCycleT(const GmresArgs& a, hipStream_t st) {
@@ -1054,7 +1100,6 @@ void gmresCycleT(const GmresArgs& a, hipStream_t st) {
     TV* r2 = (TV*)a.r2;  // SpMV output (ping-pong with r)
     TV* V = (TV*)a.V;
     GmresScalars* g = a.g;
-    double* red = g->red;
     auto mark = [&](int k, int b) {
         if (a.mark) a.mark(k, b);
     };
@@ -1068,8 +1113,7 @@ void gmresCycleT(const GmresArgs& a, hipStream_t st) {
     // r <- P^-1 r; beta = ||r||
     precond(r);
     k_norm2<TV><<<nbk, 256, 0, st>>>(nC, r, a.wk->part);
-    k_reduce_final<<<1, 256, 0, st>>>(a.wk->part, nbk, 1, red);
-    k_gm_beta0<<<1, 64, 0, st>>>(g, a.nDirs);
+    k_reduce_norm<<<1, 256, 0, st>>>(a.wk->part, nbk, g, 0);
     for (int i = 0; i < a.nDirs; ++i) {
         TV* vi = V + (size_t)i * vs;
         // v_i = r / beta ; w = A v_i (into the other buffer: the SpMV gathers
@@ -1095,29 +1139,10 @@ void gmresCycleT(const GmresArgs& a, hipStream_t st) {
         }
         if (!fused) precond(r);
         mark(TK_ORTH, 1);
-        if (a.orth == 0) {
-            // modified Gram-Schmidt, reference order
-            for (int j = 0; j <= i + 1; ++j) {
-                const TV* vprev = j > 0 ? V + (size_t)(j - 1) * vs : nullptr;
-                const TV* vnext = j <= i ? V + (size_t)j * vs : nullptr;
-                const double* hprev = j > 0 ? &g->H[j - 1][i] : nullptr;
-                k_mgs_step<TV><<<nbk, 256, 0, st>>>(nC, r, vprev, hprev, vnext, j == i + 1, a.wk->part);
-                k_reduce_mgs<<<1, 256, 0, st>>>(a.wk->part, nbk, g, i, j);
-            }
-        } else {
-            // classical Gram-Schmidt: one projection pass + one update pass
-            const int ch = m.mdCh;
-            for (int j0 = 0; j0 <= i; j0 += ch) {
-                const int nv = (i + 1 - j0) < ch ? (i + 1 - j0) : ch;
-                launchMultidot<TV>(ch, nbk, nC, r, V, vs, j0, nv, a.wk->part, st);
-                k_reduce_col<<<nv, 256, 0, st>>>(a.wk->part, nbk, ch, g, i, j0);
-            }
-            k_cgs_update<TV><<<nbk, 256, 0, st>>>(nC, r, V, vs, i + 1, g->hcol, a.wk->part);
-            k_reduce_givens<<<1, 256, 0, st>>>(a.wk->part, nbk, g, i);
-        }
+        orthStep<TV>(m, a.orth, nC, r, V, i, g, a.wk->part, st);
         mark(TK_ORTH, 0);
     }
-    k_gm_backsub<<<1, 64, 0, st>>>(g, a.nDirs);
+    k_gm_finish<<<1, 64, 0, st>>>(g, a.nDirs);
 }
 
 }  // namespace icsf
@@ -1350,10 +1375,8 @@ void fgmresCycle(const FgmresArgs& a, hipStream_t st) {
     double* V = (double*)a.V;
     double* Z = (double*)a.Z;
     GmresScalars* g = a.g;
-    double* red = g->red;
     k_norm2<double><<<nbk, 256, 0, st>>>(nC, r, a.wk->part);
-    k_reduce_final<<<1, 256, 0, st>>>(a.wk->part, nbk, 1, red);
-    k_gm_beta0<<<1, 64, 0, st>>>(g, a.nDirs);
+    k_reduce_norm<<<1, 256, 0, st>>>(a.wk->part, nbk, g, 0);
     for (int i = 0; i < a.nDirs; ++i) {
         double* vi = V + (size_t)i * vs;
         double* zi = Z + (size_t)i * vs;
@@ -1366,27 +1389,10 @@ void fgmresCycle(const FgmresArgs& a, hipStream_t st) {
         else launchSpmv(m, a.blkFp32, 0, a.blk, a.dg, zi, nullptr, nullptr, r, st);
         if (a.mark) a.mark(TK_OTHER, 0);
         if (a.mark) a.mark(TK_ORTH, 1);
-        if (a.orth == 0) {
-            for (int j = 0; j <= i + 1; ++j) {
-                const double* vprev = j > 0 ? V + (size_t)(j - 1) * vs : nullptr;
-                const double* vnext = j <= i ? V + (size_t)j * vs : nullptr;
-                const double* hprev = j > 0 ? &g->H[j - 1][i] : nullptr;
-                k_mgs_step<double><<<nbk, 256, 0, st>>>(nC, r, vprev, hprev, vnext, j == i + 1, a.wk->part);
-                k_reduce_mgs<<<1, 256, 0, st>>>(a.wk->part, nbk, g, i, j);
-            }
-        } else {
-            const int ch = m.mdCh;
-            for (int j0 = 0; j0 <= i; j0 += ch) {
-                const int nv = (i + 1 - j0) < ch ? (i + 1 - j0) : ch;
-                launchMultidot<double>(ch, nbk, nC, r, V, vs, j0, nv, a.wk->part, st);
-                k_reduce_col<<<nv, 256, 0, st>>>(a.wk->part, nbk, ch, g, i, j0);
-            }
-            k_cgs_update<double><<<nbk, 256, 0, st>>>(nC, r, V, vs, i + 1, g->hcol, a.wk->part);
-            k_reduce_givens<<<1, 256, 0, st>>>(a.wk->part, nbk, g, i);
-        }
+        orthStep<double>(m, a.orth, nC, r, V, i, g, a.wk->part, st);
         if (a.mark) a.mark(TK_ORTH, 0);
     }
-    k_gm_backsub<<<1, 64, 0, st>>>(g, a.nDirs);
+    k_gm_finish<<<1, 64, 0, st>>>(g, a.nDirs);
 }
 
 // z = sum_i y_i V_i from zero (inner solve result), FP32 or FP64 vectors.

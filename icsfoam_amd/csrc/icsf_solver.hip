@@ -762,9 +762,9 @@ int autotune(icsf_case* c) {
         }, 2);
         const void* V = v32 ? (const void*)c->V32 : (const void*)c->V;
         const int nv = v32 ? c->innerDirs : c->nDirs;
-        if (c->orth == 1 && V && nv > 0)
+        if (V && nv > 0)
             pick(m.mdCh, std::vector<int>{8, 16, 32},
-                 [&] { launchProjectionPasses(m, v32, m.mdCh, x, V, nv, c->wk.part, c->st); });
+                 [&] { launchProjectionPasses(m, v32, m.mdCh, c->orth == 0, x, V, nv, c->wk.part, c->st); });
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
@@ -1760,7 +1760,7 @@ int createCase(icsf_mesh* mesh, const char* thermo, const char* schemes, const c
         HIPCHK(hipMemset(C->g, 0, gmresScalarsBytes()));
         HIPCHK(hipMemset(C->g2, 0, gmresScalarsBytes()));
     }
-    RC(B.alloc(C->wk.part, (size_t)1024 * 64));
+    RC(B.alloc(C->wk.part, kPartSize));
     HIPCHK(hipStreamSynchronize(C->st));
     *out = C.release();
     return ICSF_OK;
@@ -2662,7 +2662,7 @@ int icsf_hb_create(icsf_mesh* mesh, const char* thermo, const char* schemes, con
     RC(B.alloc(H->dres, 10 * (size_t)HB_MAXO));
     RC(B.alloc(H->derr, 1));
     HIPCHK(hipMemset(H->derr, 0, sizeof(int)));
-    RC(B.alloc(H->wk.part, (size_t)1024 * 64));
+    RC(B.alloc(H->wk.part, kPartSize));
     {
         char* p;
         RC(B.alloc(p, gmresScalarsBytes())); H->g = (GmresScalars*)p;
