@@ -20,6 +20,8 @@ struct Levels {
     // two levels each way, forward level 1 == backward level 0 (a two-colour
     // numbering: every neighbour of a level-1 cell is a level-0 cell)
     bool twoColour = false;
+    // two-colour levels that are the cell ranges [0, n0) and [n0, nC)
+    bool colourMajor = false;
 };
 
 // Scratch for two-stage reductions.
@@ -48,6 +50,7 @@ struct GmresArgs {
     void* r;          // residual / work vector, [5][nC]
     void* r2;         // second work vector (SpMV output), [5][nC]
     void* V;          // Krylov basis, nDirs vectors of [5][nC]
+    void* t;          // work vector of the fused operator, [5][nC]
     // optional timing marks: mark(kernelClass, begin?1:0)
     std::function<void(int, int)> mark;
     // Batched (harmonic-balance) systems: vectors of 5*nVec entries and
@@ -58,8 +61,7 @@ struct GmresArgs {
     std::function<void(const void*, const double*, void*, void*)> op;
     std::function<void(void*)> pre;
     // fuse the Arnoldi SpMV with the LU-SGS sweeps when the level structure
-    // allows it (same algorithm; the forward-sweep terms of a row are summed
-    // in three partial sums instead of one running difference)
+    // allows it (same algorithm; a row's terms summed in another order)
     bool fuse = false;
     // batched systems: fused operator + preconditioner (returns false when
     // not applicable; op and pre are then used)
@@ -166,10 +168,11 @@ void launchSpmv(const MeshView& m, int blkFp32, int vecFp32, const void* blk, co
                 const double* scal, void* vout, void* y, hipStream_t st);
 void launchLusgs(const MeshView& m, const Levels& L, int blkFp32, int vecFp32, const void* blk, const double* rD,
                  void* r, hipStream_t st);
-// y = LU-SGS(A (x/scal)) in three passes on a two-colour level structure
-// (false: not applicable, nothing launched).
+// y = LU-SGS(A (x/scal)) in three passes on a two-colour level structure, t
+// a work vector (false: not applicable, nothing launched).
 bool launchSpmvLusgs(const MeshView& m, const Levels& L, int blkFp32, int vecFp32, const void* blk, const void* dg,
-                     const double* rD, const void* x, const double* scal, void* vout, void* y, hipStream_t st);
+                     const double* rD, const void* x, const double* scal, void* vout, void* t, void* y,
+                     hipStream_t st);
 void launchJacobiSetup(int nC, int blkFp32, const void* dg, void* dinv, hipStream_t st);
 void launchJacobiApply(int nC, int blkFp32, int vecFp32, const void* dinv, void* r, hipStream_t st);
 
@@ -196,9 +199,9 @@ void launchSpmvHB(const MeshView& m, const HBBlocks& hb, int vecFp32, const void
 // t = A (W - avg) and b; final residuals from r = b - A dW (r holds A dW on
 // entry).
 // y = LU-SGS(A_HB (x/scal)) in three passes on a two-colour level
-// structure (false: not applicable, nothing launched).
+// structure, t a work vector (false: not applicable, nothing launched).
 bool launchSpmvLusgsHB(const MeshView& m, const Levels& L, const HBBlocks& hb, int vecFp32, const double* rD,
-                       const void* x, const double* scal, void* vout, void* y, hipStream_t st);
+                       const void* x, const double* scal, void* vout, void* t, void* y, hipStream_t st);
 // LU-SGS of all HB instances (per-instance sweeps, shared diagonal rD).
 void launchLusgsHB(const MeshView& m, const Levels& L, const HBBlocks& hb, int vecFp32, const double* rD, void* r,
                    hipStream_t st);

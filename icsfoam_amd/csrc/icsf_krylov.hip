@@ -29,12 +29,7 @@ __device__ __forceinline__ double ld(const T* p, size_t i) { return (double)p[i]
 // One block row of y = A (x/scal): the diagonal block, then the
 // off-diagonal slots in column order, three partial sums per row (scalar
 // rho column, scalar rhoE column, vector rhoU columns) combined as the
-// blockFvMatrix sub-block sums (coupledMatrix.C:66-123).  With FWD, the
-// slots are all lower neighbours p of a colour-1 row and the forward
-// LU-SGS terms L_cp (rD_p y_p) are accumulated from the same block loads
-// (three partial sums per row as well); the row result is then
-// rD_c (y_c - fwd), i.e. the forward and the first backward level of the
-// LU-SGS sweep of a two-colour level structure.
+// blockFvMatrix sub-block sums (coupledMatrix.C:66-123).
 // Off-diagonal block of sliced-ELL slot sk for the row in lane `lane`, in
 // arithmetic type A: read from full storage, or generated from the slot's
 // NGEN generators in the storage precision (the same bits as the block the
@@ -93,11 +88,10 @@ __device__ __forceinline__ void spmvCyclic(const MeshView& m, const TB* __restri
     }
 }
 
-template <typename TB, typename TV, bool FWD, bool GEN>
+template <typename TB, typename TV, bool GEN>
 __device__ __forceinline__ void spmvRow(const MeshView& m, const TB* __restrict__ blk, const TB* __restrict__ dg,
                                         const TV* __restrict__ x, const double* __restrict__ scal,
-                                        TV* __restrict__ vout, TV* __restrict__ y, const double* __restrict__ rD,
-                                        int c) {
+                                        TV* __restrict__ vout, TV* __restrict__ y, int c) {
     const size_t nC = m.nC;
     typedef TV A;
     const A beta = scal ? (A)(*scal) : (A)1;
@@ -112,7 +106,6 @@ __device__ __forceinline__ void spmvRow(const MeshView& m, const TB* __restrict_
 #pragma unroll
         for (int k = 0; k < 5; ++k) stnt(vout + (size_t)k * nC + c, xc[k]);
     A acc[5][3];
-    A fw[5][3];
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
         const A b0 = (A)__builtin_nontemporal_load(dg + diagOff(c, 5 * i)),
@@ -123,7 +116,6 @@ __device__ __forceinline__ void spmvRow(const MeshView& m, const TB* __restrict_
         acc[i][0] = b0 * xc[0];
         acc[i][1] = b1 * xc[1];
         acc[i][2] = b2 * xc[2] + b3 * xc[3] + b4 * xc[4];
-        if (FWD) fw[i][0] = fw[i][1] = fw[i][2] = (A)0;
     }
     const int sl = c >> 6, lane = c & 63;
     const int len = m.rowLen[c];
@@ -131,14 +123,9 @@ __device__ __forceinline__ void spmvRow(const MeshView& m, const TB* __restrict_
     for (int k = 0; k < len; ++k) {
         const size_t slot = (base + k) * 64 + lane;
         const int j = ldnt(m.col + slot);
-        A xj[5], d[5];
+        A xj[5];
 #pragma unroll
         for (int q = 0; q < 5; ++q) xj[q] = X(q, j);
-        if (FWD) {
-            const A rd = (A)rD[j];
-#pragma unroll
-            for (int q = 0; q < 5; ++q) d[q] = rd * y[(size_t)q * nC + j];
-        }
         A bk[NB];
         slotBlock<TB, A, GEN, true>(m, blk, base + k, lane, bk);
 #pragma unroll
@@ -149,28 +136,14 @@ __device__ __forceinline__ void spmvRow(const MeshView& m, const TB* __restrict_
             acc[i][1] += b1 * xj[1];
             const A dd = b2 * xj[2] + b3 * xj[3] + b4 * xj[4];
             acc[i][2] += dd;
-            if (FWD) {
-                fw[i][0] += b0 * d[0];
-                fw[i][1] += b1 * d[1];
-                const A de = b2 * d[2] + b3 * d[3] + b4 * d[4];
-                fw[i][2] += de;
-            }
         }
     }
     if (m.nCyc > 0) spmvCyclic<TB, A>(m, blk, c, X, acc);
-    A rdc = (A)1;
-    if (FWD) rdc = (A)rD[c];
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
         A r = (A)0 + acc[i][0];
         r = r + acc[i][1];
         r = r + acc[i][2];
-        if (FWD) {
-            r = r - fw[i][0];
-            r = r - fw[i][1];
-            r = r - fw[i][2];
-            r = rdc * r;
-        }
         y[(size_t)i * nC + c] = r;
     }
 }
@@ -181,19 +154,7 @@ __global__ void __launch_bounds__(256, W) k_spmv(MeshView m, const TB* __restric
                                               TV* __restrict__ vout, TV* __restrict__ y) {
     const int c = xcdBlock() * blockDim.x + threadIdx.x;
     if (c >= m.nC) return;
-    spmvRow<TB, TV, false, GEN>(m, blk, dg, x, scal, vout, y, nullptr, c);
-}
-
-// SpMV of the rows in a cell list; FWD: fused forward sweep (see spmvRow).
-template <typename TB, typename TV, bool FWD, bool GEN, int W = 1>
-__global__ void __launch_bounds__(256, W) k_spmv_cells(MeshView m, const TB* __restrict__ blk,
-                                                    const TB* __restrict__ dg, const TV* __restrict__ x,
-                                                    const double* __restrict__ scal, TV* __restrict__ vout,
-                                                    TV* __restrict__ y, const double* __restrict__ rD,
-                                                    const int* __restrict__ cells, int n) {
-    const int t = xcdBlock() * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    spmvRow<TB, TV, FWD, GEN>(m, blk, dg, x, scal, vout, y, rD, ldnt(cells + t));
+    spmvRow<TB, TV, GEN>(m, blk, dg, x, scal, vout, y, c);
 }
 
 // Harmonic-balance SpMV: row cell c of instance J = blockIdx.y.  The own
@@ -203,13 +164,10 @@ __global__ void __launch_bounds__(256, W) k_spmv_cells(MeshView m, const TB* __r
 // instances 0..nO-1 (own rho, rhoE blocks at K = J) and then the own
 // vector column; vector rows add the own scalar columns and then the vector
 // columns of instances 0..nO-1 (own block at K = J).
-// With FWD (colour-1 rows of a two-colour numbering): the forward LU-SGS
-// terms of the own instance are accumulated from the same block loads and
-// the row result is rD_c (y_c - fwd), as in spmvRow.
-template <typename TB, typename TV, bool FWD, bool GEN>
+template <typename TB, typename TV, bool GEN>
 __device__ __forceinline__ void spmvRowHB(const MeshView& m, const HBBlocks& hb, int J, const TV* __restrict__ x,
                                           const double* __restrict__ scal, TV* __restrict__ vout,
-                                          TV* __restrict__ y, const double* __restrict__ rD, int c) {
+                                          TV* __restrict__ y, int c) {
     typedef TV A;
     const size_t nC = m.nC;
     const size_t vs = 5 * nC;
@@ -220,14 +178,13 @@ __device__ __forceinline__ void spmvRowHB(const MeshView& m, const HBBlocks& hb,
         const A v = x[(size_t)K * vs + (size_t)k * nC + j];
         return scal ? v / beta : v;
     };
-    const TV* yJ = y + (size_t)J * vs;
     A xc[5];
 #pragma unroll
     for (int k = 0; k < 5; ++k) xc[k] = X(J, k, c);
     if (vout)
 #pragma unroll
         for (int k = 0; k < 5; ++k) vout[(size_t)J * vs + (size_t)k * nC + c] = xc[k];
-    A acc[5][3], fw[5][3];
+    A acc[5][3];
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
         const A b0 = (A)__builtin_nontemporal_load(dg + diagOff(c, 5 * i)),
@@ -238,7 +195,6 @@ __device__ __forceinline__ void spmvRowHB(const MeshView& m, const HBBlocks& hb,
         acc[i][0] = b0 * xc[0];
         acc[i][1] = b1 * xc[1];
         acc[i][2] = b2 * xc[2] + b3 * xc[3] + b4 * xc[4];
-        if (FWD) fw[i][0] = fw[i][1] = fw[i][2] = (A)0;
     }
     const int sl = c >> 6, lane = c & 63;
     const int len = m.rowLen[c];
@@ -246,14 +202,9 @@ __device__ __forceinline__ void spmvRowHB(const MeshView& m, const HBBlocks& hb,
     for (int k = 0; k < len; ++k) {
         const size_t slot = (base + k) * 64 + lane;
         const int j = ldnt(m.col + slot);
-        A xj[5], d[5];
+        A xj[5];
 #pragma unroll
         for (int q = 0; q < 5; ++q) xj[q] = X(J, q, j);
-        if (FWD) {
-            const A rd = (A)rD[j];
-#pragma unroll
-            for (int q = 0; q < 5; ++q) d[q] = rd * yJ[(size_t)q * nC + j];
-        }
         A bk[NB];
         slotBlock<TB, A, GEN, true>(m, blk, base + k, lane, bk);
 #pragma unroll
@@ -264,12 +215,6 @@ __device__ __forceinline__ void spmvRowHB(const MeshView& m, const HBBlocks& hb,
             acc[i][1] += b1 * xj[1];
             const A dd = b2 * xj[2] + b3 * xj[3] + b4 * xj[4];
             acc[i][2] += dd;
-            if (FWD) {
-                fw[i][0] += b0 * d[0];
-                fw[i][1] += b1 * d[1];
-                const A de = b2 * d[2] + b3 * d[3] + b4 * d[4];
-                fw[i][2] += de;
-            }
         }
     }
     if (m.nCyc > 0) spmvCyclic<TB, A>(m, blk, c, [&](int k, int j) { return X(J, k, j); }, acc);
@@ -301,19 +246,8 @@ __device__ __forceinline__ void spmvRowHB(const MeshView& m, const HBBlocks& hb,
         }
         out[i] = r;
     }
-    A rdc = (A)1;
-    if (FWD) rdc = (A)rD[c];
 #pragma unroll
-    for (int i = 0; i < 5; ++i) {
-        A r = out[i];
-        if (FWD) {
-            r = r - fw[i][0];
-            r = r - fw[i][1];
-            r = r - fw[i][2];
-            r = rdc * r;
-        }
-        y[(size_t)J * vs + (size_t)i * nC + c] = r;
-    }
+    for (int i = 0; i < 5; ++i) y[(size_t)J * vs + (size_t)i * nC + c] = out[i];
 }
 
 template <typename TB, typename TV, bool GEN>
@@ -322,18 +256,191 @@ __global__ void __launch_bounds__(256) k_spmv_hb(MeshView m, HBBlocks hb, const 
                                                  TV* __restrict__ y) {
     const int c = xcdBlock() * blockDim.x + threadIdx.x;
     if (c >= m.nC) return;
-    spmvRowHB<TB, TV, false, GEN>(m, hb, blockIdx.y, x, scal, vout, y, nullptr, c);
+    spmvRowHB<TB, TV, GEN>(m, hb, blockIdx.y, x, scal, vout, y, c);
 }
 
-// HB rows of a cell list (blockIdx.y = instance); FWD: fused forward sweep.
-template <typename TB, typename TV, bool FWD, bool GEN>
-__global__ void __launch_bounds__(256) k_spmv_hb_cells(MeshView m, HBBlocks hb, const TV* __restrict__ x,
-                                                       const double* __restrict__ scal, TV* __restrict__ vout,
-                                                       TV* __restrict__ y, const double* __restrict__ rD,
-                                                       const int* __restrict__ cells, int n) {
-    const int t = xcdBlock() * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    spmvRowHB<TB, TV, FWD, GEN>(m, hb, blockIdx.y, x, scal, vout, y, rD, cells[t]);
+// ------------------------------------ Arnoldi operator, two colours -------
+// y = LU-SGS(A x), x = w/beta, on a two-level dependency graph: colour-0 rows
+// have upper neighbours only (all colour 1), colour-1 rows lower ones only.
+// With A = [D0 U; L D1] and the preconditioner ((1/rD + L) rD (1/rD + U))^-1:
+//   phase 0 (colour-0 rows): z0 = D0 x0 + U x1,  t0 = x0 - rD0 z0
+//   phase 1 (colour-1 rows): y1 = rD1 (D1 x1 + L x0 - L rD0 z0)
+//                               = rD1 (D1 x1 + L t0)
+//   phase 2 (colour-0 rows): y0 = rD0 (z0 - U y1)
+// What bounds it: the generators or blocks streamed once per phase and the
+// neighbour gathers beside them.  t0 (its own buffer) makes the product and
+// the forward sweep of phase 1 one block product of one gathered vector: 5
+// gathers per slot instead of 11 (x, y and rD) and half of its arithmetic;
+// the 1/beta scaling is applied to row sums, 5 divisions per row instead of
+// 5 per slot.  Phases 0 / 1 / 2 at 104x96x96, FP32 generators: 35 / 41 / 33
+// us (36 / 52 / 38 us with x, y and rD gathered and the blocks formed);
+// 64^3, FP64: 20 / 22 / 18 us (20 / 27 / 20 us).
+
+// acc += B x of slot sk.  FP32 generators: the flux Jacobian is applied
+// without forming its 25 entries (h A(U, E, n) x - (v + sv + mo) x, about 70
+// operations instead of 190, and 15 registers less); FP64 forms the block,
+// so that generator and block storage give the same bits.
+template <typename TB, bool GEN>
+__device__ __forceinline__ void slotApply(const MeshView& m, const TB (&g)[GEN ? NGEN : NB], TB mo, const TB x[5],
+                                          TB acc[5]) {
+    if constexpr (GEN && sizeof(TB) == 4) {
+        const TB ux = g[0], uy = g[1], uz = g[2], E = g[3], nx = g[4], ny = g[5], nz = g[6], h = g[7];
+        const TB gm = (TB)m.gamma, a2 = gm - (TB)1;
+        const TB th = (TB)0.5 * a2 * fmaf(ux, ux, fmaf(uy, uy, uz * uz));
+        const TB a1 = gm * E - th;
+        const TB pu = fmaf(ux, nx, fmaf(uy, ny, uz * nz));
+        const TB mn = fmaf(nx, x[2], fmaf(ny, x[3], nz * x[4]));
+        const TB um = fmaf(ux, x[2], fmaf(uy, x[3], uz * x[4]));
+        const TB k = fmaf(th, x[0], a2 * (x[1] - um));
+        const TB s = fmaf(-pu, x[0], mn);
+        const TB d = g[8] + g[9] + mo;
+        acc[0] = fmaf(h, mn, fmaf(-d, x[0], acc[0]));
+        acc[1] = fmaf(h, fmaf(a1, s, pu * (k + x[1])), fmaf(-d, x[1], acc[1]));
+        acc[2] = fmaf(h, fmaf(nx, k, fmaf(ux, s, pu * x[2])), fmaf(-d, x[2], acc[2]));
+        acc[3] = fmaf(h, fmaf(ny, k, fmaf(uy, s, pu * x[3])), fmaf(-d, x[3], acc[3]));
+        acc[4] = fmaf(h, fmaf(nz, k, fmaf(uz, s, pu * x[4])), fmaf(-d, x[4], acc[4]));
+    } else {
+        TB t[NB];
+        if constexpr (GEN) blockFromGen<TB>(g, (TB)m.gamma, t, mo, m.genMo != nullptr);
+        else
+#pragma unroll
+            for (int e = 0; e < NB; ++e) t[e] = g[e];
+#pragma unroll
+        for (int i = 0; i < 5; ++i)
+#pragma unroll
+            for (int q = 0; q < 5; ++q) acc[i] = __builtin_fma(t[5 * i + q], x[q], acc[i]);
+    }
+}
+
+// acc += sum over the row's slots of B_k v[col_k] (v: [5][nC]).  UN slots'
+// columns, generators and gathers are in flight together.  NT: the slot data
+// loaded non-temporally.
+template <typename TB, bool GEN, bool NT, int UN>
+__device__ __forceinline__ void rowApply(const MeshView& m, const TB* __restrict__ blk, const TB* __restrict__ v,
+                                         int c, TB acc[5]) {
+    constexpr int NE = GEN ? NGEN : NB;
+    const size_t nC = m.nC;
+    const int lane = c & 63, len = m.rowLen[c];
+    const size_t base = (size_t)m.slicePtr[c >> 6];
+    const TB* gm = (const TB*)m.genMo;
+    for (int k = 0; k < len; k += UN) {
+        int j[UN];
+        TB g[UN][NE], mo[UN], x[UN][5];
+#pragma unroll
+        for (int u = 0; u < UN; ++u) j[u] = k + u < len ? ldnt(m.col + (base + k + u) * 64 + lane) : -1;
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+            const size_t sk = base + (k + u < len ? k + u : k);
+#pragma unroll
+            for (int e = 0; e < NE; ++e) {
+                const TB* q = blk + (sk * NE + e) * 64 + lane;
+                g[u][e] = NT ? ldnt(q) : *q;
+            }
+            mo[u] = (TB)0;
+            if (GEN && gm) mo[u] = NT ? ldnt(gm + sk * 64 + lane) : gm[sk * 64 + lane];
+        }
+#pragma unroll
+        for (int u = 0; u < UN; ++u)
+#pragma unroll
+            for (int q = 0; q < 5; ++q) x[u][q] = v[(size_t)q * nC + (j[u] < 0 ? c : j[u])];
+#pragma unroll
+        for (int u = 0; u < UN; ++u)
+            if (j[u] >= 0) slotApply<TB, GEN>(m, g[u], mo[u], x[u], acc);
+    }
+}
+
+// One phase of the operator for a row per thread: rows c0 + [0, n), or a
+// cell list.  HB: instance blockIdx.y, with its cross-instance terms
+// (V_c D_JK) x_K of the other instances.  W: waves per SIMD the registers
+// must allow.
+template <typename TB, bool GEN, int PH, bool HB, int UN, int W>
+__global__ void __launch_bounds__(256, W) k_op(MeshView m, HBBlocks hb, const TB* __restrict__ blk_,
+                                               const TB* __restrict__ dg_, const TB* __restrict__ w_,
+                                               const double* __restrict__ scal, TB* __restrict__ vout,
+                                               TB* __restrict__ t_, TB* __restrict__ y_,
+                                               const double* __restrict__ rD, const int* __restrict__ cells, int c0,
+                                               int n) {
+    const int i0 = xcdBlock() * blockDim.x + threadIdx.x;
+    if (i0 >= n) return;
+    const int c = cells ? ldnt(cells + i0) : c0 + i0;
+    const size_t nC = m.nC;
+    const int J = HB ? blockIdx.y : 0;
+    const size_t off = HB ? (size_t)J * 5 * nC : 0;
+    const TB* blk = HB ? (const TB*)hb.blk[J] : blk_;
+    const TB* dg = HB ? (const TB*)hb.dg[J] : dg_;
+    TB* y = y_ + off;
+    TB* t = t_ + off;
+    const TB rd = (TB)rD[c];
+    TB acc[5];
+    if constexpr (PH == 2) {
+        TB z[5];
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+            z[q] = y[(size_t)q * nC + c];
+            acc[q] = (TB)0;
+        }
+        rowApply<TB, GEN, false, UN>(m, blk, y, c, acc);
+#pragma unroll
+        for (int q = 0; q < 5; ++q) y[(size_t)q * nC + c] = rd * (z[q] - acc[q]);
+        return;
+    }
+    const TB* w = w_ + off;
+    const TB beta = scal ? (TB)(*scal) : (TB)1;
+    TB x[5];
+#pragma unroll
+    for (int q = 0; q < 5; ++q) x[q] = w[(size_t)q * nC + c];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        acc[i] = (TB)0;
+#pragma unroll
+        for (int q = 0; q < 5; ++q) acc[i] = __builtin_fma(ldnt(dg + diagOff(c, 5 * i + q)), x[q], acc[i]);
+    }
+    if (m.nCyc > 0) {
+        // interface blocks on the far cells' rows of w, forwardT applied
+        TB a3[5][3];
+#pragma unroll
+        for (int i = 0; i < 5; ++i) a3[i][0] = a3[i][1] = a3[i][2] = (TB)0;
+        spmvCyclic<TB, TB>(m, blk, c, [&](int k, int j) { return w[(size_t)k * nC + j]; }, a3);
+#pragma unroll
+        for (int i = 0; i < 5; ++i) acc[i] += a3[i][0] + a3[i][1] + a3[i][2];
+    }
+    if (HB) {
+        const double Vc = m.V[c];
+        for (int K = 0; K < hb.nO; ++K) {
+            if (K == J) continue;
+            const TB d = (TB)(Vc * hb.D[J * hb.nO + K]);
+#pragma unroll
+            for (int q = 0; q < 5; ++q) acc[q] = __builtin_fma(d, w_[((size_t)K * 5 + q) * nC + c], acc[q]);
+        }
+    }
+    if constexpr (PH == 0) {
+        // sums of w, then scaled
+        rowApply<TB, GEN, true, UN>(m, blk, w, c, acc);
+        if (scal)
+#pragma unroll
+            for (int q = 0; q < 5; ++q) {
+                acc[q] /= beta;
+                x[q] /= beta;
+            }
+#pragma unroll
+        for (int q = 0; q < 5; ++q) {
+            y[(size_t)q * nC + c] = acc[q];
+            t[(size_t)q * nC + c] = x[q] - rd * acc[q];
+        }
+    } else {
+        if (scal)
+#pragma unroll
+            for (int q = 0; q < 5; ++q) {
+                acc[q] /= beta;
+                x[q] /= beta;
+            }
+        rowApply<TB, GEN, true, UN>(m, blk, t, c, acc);
+#pragma unroll
+        for (int q = 0; q < 5; ++q) y[(size_t)q * nC + c] = rd * acc[q];
+    }
+    if (vout)
+#pragma unroll
+        for (int q = 0; q < 5; ++q) stnt(vout + off + (size_t)q * nC + c, x[q]);
 }
 
 // ------------------------------------------------------------- LU-SGS -----
@@ -988,36 +1095,56 @@ void launchSpmv(const MeshView& m, int blkFp32, int vecFp32, const void* blk, co
     else spmv<double, double>(m, blk, dg, x, scal, vout, y, st);
 }
 
-template <typename TB, typename TV, bool GEN, int W>
-static void spmvLusgsG(const MeshView& m, const Levels& L, const void* blk, const void* dg, const double* rD,
-                       const void* x, const double* scal, void* vout, void* y, hipStream_t st) {
+// The three phases on a two-colour level structure.  Below kOpLatencyRows
+// rows per launch (about one wavefront per SIMD) a launch lasts as long as
+// one row's chain of dependent loads, and the loads of two slots (FP64) or six
+// (FP32, a third of the registers) are issued together; above, more
+// registers cost waves.  Pseudo-step, one slot / together: FP64 36^3 1.745 /
+// 1.643 ms, 64^3 4.43 / 4.48 ms; mixed 48^3 1.90 / 1.74 ms, 64^3 3.08 /
+// 3.12 ms.
+constexpr size_t kOpLatencyRows = 65536;
+
+template <typename TB, bool GEN, bool HB, int UN, int W>
+static void opPhases(const MeshView& m, const Levels& L, const HBBlocks& hb, const void* blk, const void* dg,
+                     const double* rD, const void* x, const double* scal, void* vout, void* t, void* y, int bs,
+                     hipStream_t st) {
     const int n0 = L.fwdPtrHost[1], n1 = L.fwdPtrHost[2] - n0;
-    const TB* B = (const TB*)blk;
-    const TB* G = (const TB*)dg;
-    const int bs = m.bsOp;
-    k_spmv_cells<TB, TV, false, GEN, W><<<xcdGrid(n0, bs), bs, 0, st>>>(m, B, G, (const TV*)x, scal, (TV*)vout,
-                                                                        (TV*)y, rD, L.fwdCells, n0);
-    k_spmv_cells<TB, TV, true, GEN, W><<<xcdGrid(n1, bs), bs, 0, st>>>(m, B, G, (const TV*)x, scal, (TV*)vout,
-                                                                       (TV*)y, rD, L.fwdCells + n0, n1);
     const int s0 = L.bwdPtrHost[1], nbw = L.bwdPtrHost[2] - s0;
-    k_lusgs_bwd<TB, TV, GEN, W><<<xcdGrid(nbw, bs), bs, 0, st>>>(m, B, rD, (TV*)y, L.bwdCells + s0, nbw);
+    const int nO = HB ? hb.nO : 1;
+    // colour-major numberings: the levels are cell ranges, no list
+    const int *l0 = L.colourMajor ? nullptr : L.fwdCells, *l1 = L.colourMajor ? nullptr : L.fwdCells + n0;
+    const int* l2 = L.colourMajor ? nullptr : L.bwdCells + s0;
+    const TB *B = (const TB*)blk, *G = (const TB*)dg, *X = (const TB*)x;
+    TB *V = (TB*)vout, *T = (TB*)t, *Y = (TB*)y;
+    k_op<TB, GEN, 0, HB, UN, W><<<dim3(xcdGrid(n0, bs), nO), bs, 0, st>>>(m, hb, B, G, X, scal, V, T, Y, rD, l0, 0, n0);
+    k_op<TB, GEN, 1, HB, UN, W><<<dim3(xcdGrid(n1, bs), nO), bs, 0, st>>>(m, hb, B, G, X, scal, V, T, Y, rD, l1, n0, n1);
+    k_op<TB, GEN, 2, HB, UN, W><<<dim3(xcdGrid(nbw, bs), nO), bs, 0, st>>>(m, hb, B, G, X, scal, V, T, Y, rD, l2, 0, nbw);
 }
 
-template <typename TB, typename TV>
-static void spmvLusgsT(const MeshView& m, const Levels& L, const void* blk, const void* dg, const double* rD,
-                       const void* x, const double* scal, void* vout, void* y, hipStream_t st) {
-    if (m.blkGen && m.occOp) spmvLusgsG<TB, TV, true, 4>(m, L, blk, dg, rD, x, scal, vout, y, st);
-    else if (m.blkGen) spmvLusgsG<TB, TV, true, 1>(m, L, blk, dg, rD, x, scal, vout, y, st);
-    else spmvLusgsG<TB, TV, false, 1>(m, L, blk, dg, rD, x, scal, vout, y, st);
+template <typename TB, bool HB>
+static void opLaunch(const MeshView& m, const Levels& L, const HBBlocks& hb, const void* blk, const void* dg,
+                     const double* rD, const void* x, const double* scal, void* vout, void* t, void* y, int bs,
+                     hipStream_t st) {
+    const bool few = (size_t)L.fwdPtrHost[1] * (HB ? hb.nO : 1) <= kOpLatencyRows;
+    if (!m.blkGen) opPhases<TB, false, HB, 1, 1>(m, L, hb, blk, dg, rD, x, scal, vout, t, y, bs, st);
+    else if (few) opPhases<TB, true, HB, sizeof(TB) == 4 ? 6 : 2, 1>(m, L, hb, blk, dg, rD, x, scal, vout, t, y, bs, st);
+    else {
+        // register budgets: FP32 fits 8 waves per SIMD (64 VGPRs), FP64 4
+        if constexpr (!HB)
+            if (m.occOp)
+                return opPhases<TB, true, HB, 1, sizeof(TB) == 4 ? 8 : 4>(m, L, hb, blk, dg, rD, x, scal, vout, t, y,
+                                                                         bs, st);
+        opPhases<TB, true, HB, 1, 1>(m, L, hb, blk, dg, rD, x, scal, vout, t, y, bs, st);
+    }
 }
 
 bool launchSpmvLusgs(const MeshView& m, const Levels& L, int blkFp32, int vecFp32, const void* blk, const void* dg,
-                     const double* rD, const void* x, const double* scal, void* vout, void* y, hipStream_t st) {
-    if (!L.twoColour) return false;
-    if (blkFp32 && vecFp32) spmvLusgsT<float, float>(m, L, blk, dg, rD, x, scal, vout, y, st);
-    else if (blkFp32) spmvLusgsT<float, double>(m, L, blk, dg, rD, x, scal, vout, y, st);
-    else if (vecFp32) spmvLusgsT<double, float>(m, L, blk, dg, rD, x, scal, vout, y, st);
-    else spmvLusgsT<double, double>(m, L, blk, dg, rD, x, scal, vout, y, st);
+                     const double* rD, const void* x, const double* scal, void* vout, void* t, void* y,
+                     hipStream_t st) {
+    if (!L.twoColour || blkFp32 != vecFp32) return false;
+    const HBBlocks none{};
+    if (vecFp32) opLaunch<float, false>(m, L, none, blk, dg, rD, x, scal, vout, t, y, m.bsOp, st);
+    else opLaunch<double, false>(m, L, none, blk, dg, rD, x, scal, vout, t, y, m.bsOp, st);
     return true;
 }
 
@@ -1125,8 +1252,8 @@ void gmresCycleT(const GmresArgs& a, hipStream_t st) {
         bool fused = false;
         if (a.opPre) fused = a.opPre(r, &g->beta, vi, r2);
         else if (!a.op && !a.pre && a.precond == 0 && a.fuse)
-            fused = launchSpmvLusgs(m, *a.lev, a.blkFp32, sizeof(TV) == 4, a.blk, a.dg, a.rD, r, &g->beta, vi, r2,
-                                    st);
+            fused = launchSpmvLusgs(m, *a.lev, a.blkFp32, sizeof(TV) == 4, a.blk, a.dg, a.rD, r, &g->beta, vi,
+                                    a.t, r2, st);
         if (!fused) {
             if (a.op) a.op(r, &g->beta, vi, r2);
             else launchSpmv(m, a.blkFp32, sizeof(TV) == 4, a.blk, a.dg, r, &g->beta, vi, r2, st);
@@ -1290,33 +1417,11 @@ void launchLusgsHB(const MeshView& m, const Levels& L, const HBBlocks& hb, int v
     else lusgsHBT<double, double>(m, L, hb, rD, r, st);
 }
 
-template <typename TB, typename TV, bool GEN>
-void spmvLusgsHBG(const MeshView& m, const Levels& L, const HBBlocks& hb, const double* rD, const void* x,
-                  const double* scal, void* vout, void* y, hipStream_t st) {
-    const int n0 = L.fwdPtrHost[1], n1 = L.fwdPtrHost[2] - n0;
-    k_spmv_hb_cells<TB, TV, false, GEN><<<dim3(xcdGrid(n0, 256), hb.nO), 256, 0, st>>>(
-        m, hb, (const TV*)x, scal, (TV*)vout, (TV*)y, rD, L.fwdCells, n0);
-    k_spmv_hb_cells<TB, TV, true, GEN><<<dim3(xcdGrid(n1, 256), hb.nO), 256, 0, st>>>(
-        m, hb, (const TV*)x, scal, (TV*)vout, (TV*)y, rD, L.fwdCells + n0, n1);
-    const int s0 = L.bwdPtrHost[1], nbw = L.bwdPtrHost[2] - s0;
-    k_lusgs_hb<TB, TV, false, GEN><<<dim3(xcdGrid(nbw, 256), hb.nO), 256, 0, st>>>(m, hb, rD, (TV*)y,
-                                                                                  L.bwdCells + s0, nbw);
-}
-
-template <typename TB, typename TV>
-void spmvLusgsHBT(const MeshView& m, const Levels& L, const HBBlocks& hb, const double* rD, const void* x,
-                  const double* scal, void* vout, void* y, hipStream_t st) {
-    if (m.blkGen) spmvLusgsHBG<TB, TV, true>(m, L, hb, rD, x, scal, vout, y, st);
-    else spmvLusgsHBG<TB, TV, false>(m, L, hb, rD, x, scal, vout, y, st);
-}
-
 bool launchSpmvLusgsHB(const MeshView& m, const Levels& L, const HBBlocks& hb, int vecFp32, const double* rD,
-                       const void* x, const double* scal, void* vout, void* y, hipStream_t st) {
-    if (!L.twoColour) return false;
-    if (hb.fp32 && vecFp32) spmvLusgsHBT<float, float>(m, L, hb, rD, x, scal, vout, y, st);
-    else if (hb.fp32) spmvLusgsHBT<float, double>(m, L, hb, rD, x, scal, vout, y, st);
-    else if (vecFp32) spmvLusgsHBT<double, float>(m, L, hb, rD, x, scal, vout, y, st);
-    else spmvLusgsHBT<double, double>(m, L, hb, rD, x, scal, vout, y, st);
+                       const void* x, const double* scal, void* vout, void* t, void* y, hipStream_t st) {
+    if (!L.twoColour || hb.fp32 != vecFp32) return false;
+    if (vecFp32) opLaunch<float, true>(m, L, hb, nullptr, nullptr, rD, x, scal, vout, t, y, 256, st);
+    else opLaunch<double, true>(m, L, hb, nullptr, nullptr, rD, x, scal, vout, t, y, 256, st);
     return true;
 }
 

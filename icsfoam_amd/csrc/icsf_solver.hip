@@ -639,7 +639,7 @@ int gmresSolve(icsf_case* c, const double* W, const double* b, int& nIter) {
     nIter = 0;
     for (;;) {
         GmresArgs a{&c->mv, &c->mesh->lev, &c->wk, c->g, c->nDirs, c->precond, c->orth, c->blkFp32,
-                    c->blk, c->dg, c->rD, c->dinv, c->r, c->t2, c->V};
+                    c->blk, c->dg, c->rD, c->dinv, c->r, c->t2, c->V, c->t1};
         a.mark = [c](int k, int b) { markClass(c, k, b); };
         a.fuse = c->fuse;
         gmresCycle(a, 0, c->st);
@@ -755,7 +755,7 @@ int autotune(icsf_case* c) {
         int occDummy = 0;
         pick2(m.bsOp, m.blkGen ? m.occOp : occDummy, [&] {
             if (!(c->fuse && launchSpmvLusgs(m, c->mesh->lev, c->blkFp32, v32, c->blk, c->dg, c->rD, x, nullptr,
-                                             nullptr, y, c->st))) {
+                                             nullptr, c->dW, y, c->st))) {
                 launchSpmv(m, c->blkFp32, v32, c->blk, c->dg, x, nullptr, nullptr, y, c->st);
                 launchLusgs(m, c->mesh->lev, c->blkFp32, v32, c->blk, c->rD, y, c->st);
             }
@@ -864,7 +864,7 @@ int fgmresSolve(icsf_case* c, const double* W, const double* b, int& nIter) {
             launchConvert(vs, 0, v, c->r32, c->st);
             if (c->innerDirs > 0) {
                 GmresArgs a{&c->mv, &c->mesh->lev, &c->wk, c->g2, c->innerDirs, c->precond, c->orth, c->blkFp32,
-                            c->blk, c->dg, c->rD, c->dinv, c->r32, c->r32b, c->V32};
+                            c->blk, c->dg, c->rD, c->dinv, c->r32, c->r32b, c->V32, c->t1};
                 a.mark = [c](int k, int b) { markClass(c, k, b); };
                 a.fuse = c->fuse;
                 gmresCycle(a, 1, c->st);
@@ -1202,7 +1202,7 @@ int hbSolve(icsf_hb* h, const double* b, int& nIter) {
     nIter = 0;
     for (;;) {
         GmresArgs a{&m, &h->mesh->lev, &h->wk, h->g, h->nDirs, 0, h->orth, 0, nullptr, nullptr, h->rD, nullptr,
-                    h->r, h->r2, h->V};
+                    h->r, h->r2, h->V, h->t1};
         a.nVec = m.nC * h->nO;
         a.op = [h, &m](const void* x, const double* scal, void* vout, void* y) {
             launchSpmvHB(m, h->hbb, 0, x, scal, vout, y, h->st);
@@ -1210,7 +1210,7 @@ int hbSolve(icsf_hb* h, const double* b, int& nIter) {
         a.pre = [h](void* v) { hbLusgs(h, v); };
         if (h->fuse)
             a.opPre = [h, &m](const void* x, const double* scal, void* vout, void* y) {
-                return launchSpmvLusgsHB(m, h->mesh->lev, h->hbb, 0, h->rD, x, scal, vout, y, h->st);
+                return launchSpmvLusgsHB(m, h->mesh->lev, h->hbb, 0, h->rD, x, scal, vout, h->t1, y, h->st);
             };
         gmresCycle(a, 0, h->st);
         launchUpdateSolution((size_t)m.nC * h->nO, h->dW, h->V, vA, h->nDirs, h->g, h->st);
@@ -1259,7 +1259,7 @@ int hbSolveMixed(icsf_hb* h, const double* b, int& nIter) {
             return;
         }
         GmresArgs a{&m, &h->mesh->lev, &h->wk, h->g2, h->innerDirs, 0, h->orth, 1, nullptr, nullptr, h->rD,
-                    nullptr, h->r32, h->r32b, h->V32};
+                    nullptr, h->r32, h->r32b, h->V32, h->t1};
         a.nVec = nVec;
         a.op = [h, &m](const void* x, const double* scal, void* vout, void* y) {
             launchSpmvHB(m, h->hbb, 1, x, scal, vout, y, h->st);
@@ -1267,7 +1267,7 @@ int hbSolveMixed(icsf_hb* h, const double* b, int& nIter) {
         a.pre = [h](void* v) { hbLusgs(h, v, 1); };
         if (h->fuse)
             a.opPre = [h, &m](const void* x, const double* scal, void* vout, void* y) {
-                return launchSpmvLusgsHB(m, h->mesh->lev, h->hbb, 1, h->rD, x, scal, vout, y, h->st);
+                return launchSpmvLusgsHB(m, h->mesh->lev, h->hbb, 1, h->rD, x, scal, vout, h->t1, y, h->st);
             };
         gmresCycle(a, 1, h->st);
         launchCombine(nVec, 1, h->V32, h->innerDirs, h->g2, h->r32, h->st);
@@ -1555,6 +1555,8 @@ int icsf_mesh_create(int nPoints, const double* points, int nFaces, const int* f
     bucket(bl, nbw, L.bwdPtrHost, bc);
     L.twoColour = nf == 2 && nbw == 2 && L.fwdPtrHost[1] == L.bwdPtrHost[2] - L.bwdPtrHost[1] &&
                   std::equal(fc.begin() + L.fwdPtrHost[1], fc.end(), bc.begin());
+    L.colourMajor = L.twoColour;
+    for (int i = 0; L.colourMajor && i < h.nCells; ++i) L.colourMajor = fc[i] == i;
     DevBuf& B = M->buf;
     MeshView& v = M->view;
     v.nC = h.nCells;
