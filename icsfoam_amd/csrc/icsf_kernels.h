@@ -22,11 +22,31 @@ struct Levels {
     bool twoColour = false;
     // two-colour levels that are the cell ranges [0, n0) and [n0, nC)
     bool colourMajor = false;
+    // dataflow sweep (null when the levels are swept by a launch each): the
+    // cells of each level in chunks of a wavefront (-1 pads a level's last
+    // chunk), the level of each chunk, the chunks of each level (forward,
+    // then backward levels), all on the device
+    int nFwdChunks = 0, nBwdChunks = 0;
+    int *chunkCells = nullptr, *chunkLevel = nullptr, *levelChunks = nullptr;
 };
+// Largest average number of cells per level swept in one dataflow launch: a
+// launch per level costs the same up to there (its latency), while the
+// dataflow's uncached loads add up.  Pseudo-step with a launch per level / in
+// one launch: 813 cells per level 11.5 / 7.5 ms, 2600 101 / 60 ms, 3800 14.4 /
+// 10.3 ms, 13800 26.0 / 23.7 ms in FP64 but 20.3 / 20.7 ms mixed.
+constexpr int kSweepLevelCells = 8192;
+// Fewest levels (forward and backward together) for it: the 28 059-cell LS89
+// mesh coloured (4 + 4 levels) steps in 2.36 ms with its 7 launches per
+// application and 2.43 ms in one, 17 + 17 levels are well ahead (above).
+constexpr int kSweepMinLevels = 24;
 
-// Scratch for two-stage reductions.
+// Scratch for two-stage reductions, and of the dataflow sweep: the forward
+// and the final values [5][nC], the levels' finished chunks and the next chunk
+// to draw, the case's error flags (swF null: none).
 struct Work {
     double* part = nullptr;  // [kPartSize]
+    void *swF = nullptr, *swO = nullptr;
+    int *swDone = nullptr, *err = nullptr;
 };
 
 // 1024 workgroups' partials of the 2 KMAX projection values of one step
@@ -166,8 +186,8 @@ void launchCellSumsJacobian(const MeshView& m, const Phys& ph, const StateView& 
 
 void launchSpmv(const MeshView& m, int blkFp32, int vecFp32, const void* blk, const void* dg, const void* x,
                 const double* scal, void* vout, void* y, hipStream_t st);
-void launchLusgs(const MeshView& m, const Levels& L, int blkFp32, int vecFp32, const void* blk, const double* rD,
-                 void* r, hipStream_t st);
+void launchLusgs(const MeshView& m, const Levels& L, const Work& wk, int blkFp32, int vecFp32, const void* blk,
+                 const double* rD, void* r, hipStream_t st);
 // y = LU-SGS(A (x/scal)) in three passes on a two-colour level structure, t
 // a work vector (false: not applicable, nothing launched).
 bool launchSpmvLusgs(const MeshView& m, const Levels& L, int blkFp32, int vecFp32, const void* blk, const void* dg,

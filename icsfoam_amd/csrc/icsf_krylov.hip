@@ -549,6 +549,200 @@ __global__ void __launch_bounds__(256) k_lusgs_hb(MeshView m, HBBlocks hb, const
     else lusgsBwdRow<TB, TV, GEN>(m, (const TB*)hb.blk[J], rD, rJ, cells[t]);
 }
 
+// LU-SGS of a numbering with many dependency levels (RCM or file order: a
+// hundred and more each way) in one launch.  A launch per level costs 5 to 7
+// us whatever the level holds; here a level costs one store-to-load round
+// trip between wavefronts, about 2 us.  The cells of a level form chunks of
+// one wavefront; the wavefronts draw the chunks in level order, forward
+// levels first, from one counter, and wait for the values their rows read:
+//   - forward results f and final results o start as a sentinel (a signalling
+//     NaN pattern, which arithmetic does not return), are stored once with
+//     agent-scope relaxed atomics and read with the same until they differ
+//     from it: each value is its own flag, so nothing depends on the order in
+//     which different values become visible;
+//   - before that, a wavefront waits on the finished-chunk count of the level
+//     two before its own, one load at a time, so that wavefronts far from the
+//     front do not load the rows' values over and over.  The counts only pace
+//     the loads.
+// A row reads only rows of earlier levels, i.e. of lower chunks.  A chunk is
+// drawn by a running wavefront, which finishes the chunks it drew in order,
+// so the lowest unfinished chunk always runs, however few of the wavefronts
+// the GPU has room for.  Every wait gives up after kSweepSpins loads (seconds; the longest
+// sweep takes milliseconds) and sets ERR_FLAG_SWEEP, as does every later one.
+// Same operations and order per row as lusgsFwdRow / lusgsBwdRow.
+constexpr int kSweepSpins = 1 << 21;
+
+__device__ __forceinline__ unsigned long long sweepSentinel(double) { return 0x7FF4DEADBEEF5A5Aull; }
+__device__ __forceinline__ unsigned sweepSentinel(float) { return 0x7FA5A5A5u; }
+__device__ __forceinline__ unsigned long long sweepBits(double v) { return __double_as_longlong(v); }
+__device__ __forceinline__ unsigned sweepBits(float v) { return __float_as_uint(v); }
+template <typename TV>
+__device__ __forceinline__ TV sweepLoad(const TV* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename TV>
+__device__ __forceinline__ void sweepStore(TV* p, TV v) {
+    if (sweepBits(v) == sweepSentinel(v)) v = (TV)__builtin_nan("");
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// done: the finished chunks of each level, then the next chunk to draw
+template <typename TV>
+__global__ void k_sweep_init(size_t n, int nLev, TV* __restrict__ f, TV* __restrict__ o, int* __restrict__ done) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    TV v;
+    const auto s = sweepSentinel((TV)0);
+    __builtin_memcpy(&v, &s, sizeof(TV));
+    if (i < n) f[i] = o[i] = v;
+    if (i <= (size_t)nLev) done[i] = 0;
+}
+
+template <typename TB, typename TV, bool GEN>
+__global__ void __launch_bounds__(64) k_sweep(MeshView m, const TB* __restrict__ blk, const double* __restrict__ rD,
+                                               TV* r, TV* f, TV* o, const int* __restrict__ chunkCells,
+                                               const int* __restrict__ chunkLevel,
+                                               const int* __restrict__ levelChunks, int nFwd, int nChunks,
+                                               int nFwdLevels, int* done, int* next, int* err) {
+    constexpr int UN = 3;  // slots whose blocks and values are in flight together
+    typedef TV A;
+    const size_t nC = m.nC;
+    const int lane = threadIdx.x & 63;
+    const auto sent = sweepSentinel((TV)0);
+    int spins = 0;
+    // the values at q (5 of them nC apart) of every lane with on set
+    auto wait5 = [&](const TV* q, bool on, A (&v)[5]) {
+        bool ready = !on;
+        for (;;) {
+            if (!ready) {
+                ready = true;
+#pragma unroll
+                for (int z = 0; z < 5; ++z) {
+                    const TV x = sweepLoad(q + (size_t)z * nC);
+                    v[z] = (A)x;
+                    ready = ready && sweepBits(x) != sent;
+                }
+            }
+            if (__all(ready)) return true;
+            if (++spins > kSweepSpins) return false;
+        }
+    };
+    auto draw = [&]() {
+        int i = 0;
+        if (lane == 0) i = __hip_atomic_fetch_add(next, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return __builtin_amdgcn_readfirstlane(i);
+    };
+    for (int ch = draw(); ch < nChunks; ch = draw()) {
+        const bool bwd = ch >= nFwd;
+        const int lev = chunkLevel[ch];                        // within its sweep
+        const int lg = bwd ? nFwdLevels + lev : lev;           // over both
+        const int c = chunkCells[(size_t)ch * 64 + lane];
+        const bool on = c >= 0;
+        const int cc = on ? c : 0;
+        const int sl = cc >> 6, ln = cc & 63;
+        const size_t base = (size_t)m.slicePtr[sl];
+        const int nl = m.nLower[cc], len = m.rowLen[cc];
+        const int n = on ? (bwd ? len - nl : nl) : 0;
+        const A rdc = (A)rD[cc];
+        bool ok = true, begun = false;
+        A acc[5];
+        // the pacing wait, then the row's own value (forward: r; backward: f)
+        auto begin = [&]() {
+            begun = true;
+            if (lev >= 2) {
+                const int want = levelChunks[lg - 2];
+                while (__builtin_amdgcn_readfirstlane(
+                           __hip_atomic_load(done + lg - 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) < want) {
+                    if (++spins > kSweepSpins) { ok = false; return; }
+                    __builtin_amdgcn_s_sleep(8);
+                }
+            }
+            if (bwd) ok = wait5(f + cc, on, acc);
+            else
+#pragma unroll
+                for (int q = 0; q < 5; ++q) acc[q] = (A)r[(size_t)q * nC + cc];
+        };
+        const TV* src = bwd ? o : f;
+        for (int k = 0; ok && __any(k < n); k += UN) {
+            // forward: lower slots upwards; backward: upper slots downwards.
+            // The blocks are formed before the wait (the empty asm keeps
+            // them from being moved behind it): after it a slot costs its
+            // product only
+            constexpr int NE = GEN ? NGEN : NB;
+            TB b[UN][NB];
+            A rd[UN];
+            int p[UN];
+            A d[UN][5];
+#pragma unroll
+            for (int u = 0; u < UN; ++u) {
+                const bool has = k + u < n;
+                const size_t sk = base + (has ? (bwd ? len - 1 - (k + u) : k + u) : 0);
+                p[u] = has ? m.col[sk * 64 + ln] : cc;
+                rd[u] = bwd ? (A)1 : (A)rD[p[u]];
+                TB g[NE];
+#pragma unroll
+                for (int e = 0; e < NE; ++e) g[e] = has ? blk[(sk * NE + e) * 64 + ln] : (TB)0;
+                const TB mo = GEN && m.genMo && has ? ((const TB*)m.genMo)[sk * 64 + ln] : (TB)0;
+                if constexpr (GEN) blockFromGen<TB>(g, (TB)m.gamma, b[u], mo, m.genMo != nullptr);
+                else
+#pragma unroll
+                    for (int e = 0; e < NB; ++e) b[u][e] = g[e];
+#pragma unroll
+                for (int e = 0; e < NB; ++e) asm volatile("" : "+v"(b[u][e]));
+            }
+            if (!begun) begin();
+            // the slots' values, those not there yet loaded again
+            unsigned miss = 0;
+#pragma unroll
+            for (int u = 0; u < UN; ++u) miss |= ok && k + u < n ? 1u << u : 0u;
+            while (__any(miss)) {
+#pragma unroll
+                for (int u = 0; u < UN; ++u)
+                    if (miss & (1u << u)) {
+                        bool got = true;
+#pragma unroll
+                        for (int z = 0; z < 5; ++z) {
+                            const TV x = sweepLoad(src + (size_t)z * nC + p[u]);
+                            d[u][z] = (A)x;
+                            got = got && sweepBits(x) != sent;
+                        }
+                        if (got) miss &= ~(1u << u);
+                    }
+                if (++spins > kSweepSpins) { ok = false; break; }
+            }
+#pragma unroll
+            for (int u = 0; u < UN; ++u) {
+                if (k + u >= n) continue;
+                if (!bwd)
+#pragma unroll
+                    for (int z = 0; z < 5; ++z) d[u][z] = rd[u] * d[u][z];
+#pragma unroll
+                for (int i = 0; i < 5; ++i) {
+                    const A b0 = (A)b[u][5 * i], b1 = (A)b[u][5 * i + 1];
+                    const A b2 = (A)b[u][5 * i + 2], b3 = (A)b[u][5 * i + 3], b4 = (A)b[u][5 * i + 4];
+                    acc[i] -= b0 * d[u][0];
+                    acc[i] -= b1 * d[u][1];
+                    const A dd = b2 * d[u][2] + b3 * d[u][3] + b4 * d[u][4];
+                    acc[i] -= dd;
+                }
+            }
+        }
+        if (!begun) begin();
+        if (!ok) {
+            if (lane == 0) atomicOr(err, ERR_FLAG_SWEEP);
+            return;
+        }
+        if (on)
+#pragma unroll
+            for (int q = 0; q < 5; ++q) {
+                const A v = bwd ? rdc * acc[q] : acc[q];
+                sweepStore((bwd ? o : f) + (size_t)q * nC + c, (TV)v);
+                // r[c] was read by the forward chunk whose f[c] this wave has
+                if (bwd) r[(size_t)q * nC + c] = (TV)v;
+            }
+        if (lane == 0) __hip_atomic_fetch_add(done + lg, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
 // ------------------------------------------------------- block-Jacobi -----
 // 5x5 inverse of each diagonal block by LU with partial pivoting.
 template <typename TB>
@@ -1164,19 +1358,42 @@ static void lusgsG(const MeshView& m, const Levels& L, const void* blk, const do
     }
 }
 
+// The dataflow sweep, one wavefront per workgroup.  Per application, forward
+// and backward: 48x24x24 in RCM order (82 levels each way) 1110 us as 164
+// launches -> 540 us; 200x50x1 in file order (249 levels) 3200 -> 1010 us;
+// 128x64x64 in RCM order (201 levels) 3200 -> 1850 us.  256 wavefronts: with 512
+// the 72x64x56 and 128x64x64 boxes take 7 and 12 % longer (their loads
+// queue behind each other's), smaller ones the same; chunks of 32 rows 10 to
+// 25 % longer (more counts and draws).
+constexpr int kSweepWaves = 256;
+template <typename TB, typename TV, bool GEN>
+static void sweepG(const MeshView& m, const Levels& L, const Work& wk, const void* blk, const double* rD, void* r,
+                   hipStream_t st) {
+    const int nCh = L.nFwdChunks + L.nBwdChunks, nLev = L.nFwd + L.nBwd;
+    const size_t n = (size_t)5 * m.nC;
+    k_sweep_init<TV><<<nb(n, 256), 256, 0, st>>>(n, nLev, (TV*)wk.swF, (TV*)wk.swO, wk.swDone);
+    const int nWg = nCh < kSweepWaves ? nCh : kSweepWaves;
+    k_sweep<TB, TV, GEN><<<nWg, 64, 0, st>>>(m, (const TB*)blk, rD, (TV*)r, (TV*)wk.swF, (TV*)wk.swO, L.chunkCells,
+                                             L.chunkLevel, L.levelChunks, L.nFwdChunks, nCh, L.nFwd, wk.swDone,
+                                             wk.swDone + nLev, wk.err);
+}
+
 template <typename TB, typename TV>
-static void lusgsT(const MeshView& m, const Levels& L, const void* blk, const double* rD, void* r, hipStream_t st) {
-    if (m.blkGen && m.occOp) lusgsG<TB, TV, true, 4>(m, L, blk, rD, r, st);
+static void lusgsT(const MeshView& m, const Levels& L, const Work& wk, const void* blk, const double* rD, void* r,
+                   hipStream_t st) {
+    if (wk.swF && m.blkGen) sweepG<TB, TV, true>(m, L, wk, blk, rD, r, st);
+    else if (wk.swF) sweepG<TB, TV, false>(m, L, wk, blk, rD, r, st);
+    else if (m.blkGen && m.occOp) lusgsG<TB, TV, true, 4>(m, L, blk, rD, r, st);
     else if (m.blkGen) lusgsG<TB, TV, true, 1>(m, L, blk, rD, r, st);
     else lusgsG<TB, TV, false, 1>(m, L, blk, rD, r, st);
 }
 
-void launchLusgs(const MeshView& m, const Levels& L, int blkFp32, int vecFp32, const void* blk, const double* rD,
-                 void* r, hipStream_t st) {
-    if (blkFp32 && vecFp32) lusgsT<float, float>(m, L, blk, rD, r, st);
-    else if (blkFp32) lusgsT<float, double>(m, L, blk, rD, r, st);
-    else if (vecFp32) lusgsT<double, float>(m, L, blk, rD, r, st);
-    else lusgsT<double, double>(m, L, blk, rD, r, st);
+void launchLusgs(const MeshView& m, const Levels& L, const Work& wk, int blkFp32, int vecFp32, const void* blk,
+                 const double* rD, void* r, hipStream_t st) {
+    if (blkFp32 && vecFp32) lusgsT<float, float>(m, L, wk, blk, rD, r, st);
+    else if (blkFp32) lusgsT<float, double>(m, L, wk, blk, rD, r, st);
+    else if (vecFp32) lusgsT<double, float>(m, L, wk, blk, rD, r, st);
+    else lusgsT<double, double>(m, L, wk, blk, rD, r, st);
 }
 
 void launchJacobiSetup(int nC, int blkFp32, const void* dg, void* dinv, hipStream_t st) {
@@ -1233,7 +1450,7 @@ void gmresCycleT(const GmresArgs& a, hipStream_t st) {
     auto precond = [&](TV* v) {
         mark(TK_PRECOND, 1);
         if (a.pre) a.pre(v);
-        else if (a.precond == 0) launchLusgs(m, *a.lev, a.blkFp32, sizeof(TV) == 4, a.blk, a.rD, v, st);
+        else if (a.precond == 0) launchLusgs(m, *a.lev, *a.wk, a.blkFp32, sizeof(TV) == 4, a.blk, a.rD, v, st);
         else if (a.precond == 1) launchJacobiApply(nC, a.blkFp32, sizeof(TV) == 4, a.dinv, v, st);
         mark(TK_PRECOND, 0);
     };

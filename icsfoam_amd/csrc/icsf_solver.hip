@@ -443,6 +443,7 @@ int takeDeviceErrors(hipStream_t st, const std::vector<int*>& flags) {
         any |= e;
     }
     if (any & ERR_FLAG_NONFINITE) return fail(ICSF_ERR_NONFINITE, "non-finite conserved state after the update");
+    if (any & ERR_FLAG_SWEEP) return fail(ICSF_ERR_HIP, "LU-SGS sweep: a wait ended at its limit");
     if (any & ERR_FLAG_DIAG) return fail(ICSF_ERR_ZERO_DIAG, "All diagonals of coupledMatrix are zero.");
     return ICSF_OK;
 }
@@ -621,7 +622,7 @@ int jacobianStage(icsf_case* c, bool cellSums = false) {
 
 void applyPrecond(icsf_case* c, int vecFp32, void* v) {
     Timed t(c, TK_PRECOND);
-    if (c->precond == 0) launchLusgs(c->mv, c->mesh->lev, c->blkFp32, vecFp32, c->blk, c->rD, v, c->st);
+    if (c->precond == 0) launchLusgs(c->mv, c->mesh->lev, c->wk, c->blkFp32, vecFp32, c->blk, c->rD, v, c->st);
     else if (c->precond == 1) launchJacobiApply(c->mv.nC, c->blkFp32, vecFp32, c->dinv, v, c->st);
 }
 
@@ -757,7 +758,7 @@ int autotune(icsf_case* c) {
             if (!(c->fuse && launchSpmvLusgs(m, c->mesh->lev, c->blkFp32, v32, c->blk, c->dg, c->rD, x, nullptr,
                                              nullptr, c->dW, y, c->st))) {
                 launchSpmv(m, c->blkFp32, v32, c->blk, c->dg, x, nullptr, nullptr, y, c->st);
-                launchLusgs(m, c->mesh->lev, c->blkFp32, v32, c->blk, c->rD, y, c->st);
+                launchLusgs(m, c->mesh->lev, c->wk, c->blkFp32, v32, c->blk, c->rD, y, c->st);
             }
         }, 2);
         const void* V = v32 ? (const void*)c->V32 : (const void*)c->V;
@@ -1603,6 +1604,24 @@ int icsf_mesh_create(int nPoints, const double* points, int nFaces, const int* f
     }
     RC(B.upload(L.fwdCells, fc.data(), fc.size()));
     RC(B.upload(L.bwdCells, bc.data(), bc.size()));
+    if (nf + nbw >= kSweepMinLevels && (size_t)2 * h.nCells <= (size_t)kSweepLevelCells * (nf + nbw)) {
+        std::vector<int> cells, level, count;
+        auto chunks = [&](const std::vector<int>& ptr, const std::vector<int>& list, int n) {
+            for (int l = 0; l < n; ++l) {
+                const int nCh = (ptr[l + 1] - ptr[l] + 63) / 64;
+                for (int i = ptr[l]; i < ptr[l] + 64 * nCh; ++i) cells.push_back(i < ptr[l + 1] ? list[i] : -1);
+                level.insert(level.end(), nCh, l);
+                count.push_back(nCh);
+            }
+        };
+        chunks(L.fwdPtrHost, fc, nf);
+        L.nFwdChunks = (int)level.size();
+        chunks(L.bwdPtrHost, bc, nbw);
+        L.nBwdChunks = (int)level.size() - L.nFwdChunks;
+        RC(B.upload(L.chunkCells, cells.data(), cells.size()));
+        RC(B.upload(L.chunkLevel, level.data(), level.size()));
+        RC(B.upload(L.levelChunks, count.data(), count.size()));
+    }
     v.own = own; v.nei = nei; v.Sf = Sf; v.magSf = magSf; v.Cf = Cf; v.w = w; v.dc = dc; v.nodc = nodc;
     v.corr = corr; v.C = C; v.V = V; v.cfOff = cfOff; v.cf = cf; v.bKind = bKind;
     v.nSlices = M->sell.nSlices; v.slicePtr = slicePtr; v.col = col; v.rowLen = rowLen; v.nLower = nLower;
@@ -1763,6 +1782,15 @@ int createCase(icsf_mesh* mesh, const char* thermo, const char* schemes, const c
         HIPCHK(hipMemset(C->g2, 0, gmresScalarsBytes()));
     }
     RC(B.alloc(C->wk.part, kPartSize));
+    if (mesh->lev.chunkCells && C->precond == 0) {
+        double *f, *o;
+        RC(B.alloc(f, vs));
+        RC(B.alloc(o, vs));
+        RC(B.alloc(C->wk.swDone, mesh->lev.nFwd + mesh->lev.nBwd + 1));
+        C->wk.swF = f;
+        C->wk.swO = o;
+        C->wk.err = C->derr;
+    }
     HIPCHK(hipStreamSynchronize(C->st));
     *out = C.release();
     return ICSF_OK;
@@ -2423,7 +2451,7 @@ int icsf_precondition(icsf_case* c, double* r) {
     applyPrecond(c, 0, c->t1);
     HIPCHK(hipMemcpyAsync(r, c->t1, vs * 8, hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
-    return ICSF_OK;
+    return takeDeviceErrors(c->st, {c->derr});
 }
 
 int icsf_solve_for_incr(icsf_case* c, const double* W, const double* b, double* dW, double* residuals,

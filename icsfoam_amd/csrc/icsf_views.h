@@ -162,7 +162,8 @@ struct StateView {
 enum { CTL_CORR = 0, CTL_CONV = 1, CTL_FIN = 2, CTL_RUN = 3, CTL_EN = 4, CTL_FIRST = 5, NCTL = 8 };
 
 // bits of the device error flags
-enum { ERR_FLAG_DIAG = 1, ERR_FLAG_NONFINITE = 2 };
+// (ERR_FLAG_SWEEP: a wait of the dataflow sweep ended at its limit)
+enum { ERR_FLAG_DIAG = 1, ERR_FLAG_NONFINITE = 2, ERR_FLAG_SWEEP = 4 };
 
 // Buffers of the residual adjoint (vector-Jacobian product).
 struct AdjView {
