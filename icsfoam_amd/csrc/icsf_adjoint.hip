@@ -13,23 +13,25 @@
 // The reconstruction is recomputed, not taped: the forward pass re-runs the
 // boundary and gradient kernels (keeping the unlimited gradients and the
 // limiter values), then the reverse kernels pull adjoints without atomics:
-//   k_adj_face   one thread per face: AUSM+up or Roe reverse (each one
-//                forward evaluation and one backward sweep) or HLLC (one
-//                dual-number pass per face value), adjoint of
-//                the face values (owner/neighbour side) and of Sf, Cf
-//                (flux part)
+//   k_adj_face   one thread per face: the scheme's reverse (one forward
+//                evaluation and one backward sweep), adjoint of the face
+//                values (owner/neighbour side) and, with the geometry
+//                adjoint, of Sf, Cf (flux part)
 //   k_adj_visc   one thread per face (viscous cases): adjoint of the
 //                viscous face terms
-//   k_adj_cell   one thread per cell: adjoint of the limited gradients, of
-//                the limiter (its active face and max/min neighbour) and of
-//                the Gauss gradient sum divided by V
+//   k_adj_cell   one thread per cell and half of its fields: adjoint of the
+//                limited gradients, of the limiter (its active face and
+//                max/min neighbour) and of the Gauss gradient sum divided by V
 //   k_adj_gauss  one thread per face: Gauss-gradient face values, boundary
-//                values -> owner primitives, limiter pulls into Cf
-//   k_adj_state  one thread per cell: cell-value adjoints -> E, H, c* ->
-//                rho, U, e, T, p -> W
+//                values -> owner primitives, Gauss and limiter pulls into Sf
+//                and Cf; without the geometry adjoint the boundary faces only
+//   k_adj_state  one thread per cell: cell-value adjoints (without the
+//                geometry adjoint the Gauss face values formed here) -> E, H,
+//                c* -> rho, U, e, T, p -> W
 // Branches follow the primal value: max(a, b) takes b only if b > a,
 // min(a, b) takes b only if b < a, and the limiter's min over faces keeps
 // the first face that attains it.
+#include "icsf_hllc_rev.h"
 #include "icsf_kernels.h"
 #include "icsf_recon.h"
 #include "icsf_roe_rev.h"
@@ -46,104 +48,6 @@ namespace {
 // VSMALL)).
 DF bool used(int flux, int k) {
     return flux == FLUX_ROE ? k != F_CS : (flux == FLUX_HLLC ? true : k != F_E);
-}
-
-// ---- HLLC: forward-mode passes of the face flux on dual numbers (value
-// and one tangent), one per input, contracted with the flux adjoint
-struct Dn {
-    double v, d;
-};
-DF Dn operator+(Dn a, Dn b) { return Dn{a.v + b.v, a.d + b.d}; }
-DF Dn operator-(Dn a, Dn b) { return Dn{a.v - b.v, a.d - b.d}; }
-DF Dn operator*(Dn a, Dn b) { return Dn{a.v * b.v, a.d * b.v + a.v * b.d}; }
-DF Dn operator/(Dn a, Dn b) {
-    const double q = a.v / b.v;
-    return Dn{q, (a.d - q * b.d) / b.v};
-}
-DF Dn dsqrt(Dn a) {
-    const double r = sqrt(a.v);
-    return Dn{r, r > 0.0 ? a.d / (2.0 * r) : 0.0};
-}
-DF Dn dfabs(Dn a) { return a.v < 0.0 ? Dn{-a.v, -a.d} : a; }
-DF Dn dmin(Dn a, Dn b) { return b.v < a.v ? b : a; }  // std::min(a, b)
-DF Dn dmax(Dn a, Dn b) { return a.v < b.v ? b : a; }  // std::max(a, b)
-DF Dn cst(double x) { return Dn{x, 0.0}; }
-struct V3n {
-    Dn x, y, z;
-};
-DF V3n operator+(V3n a, V3n b) { return V3n{a.x + b.x, a.y + b.y, a.z + b.z}; }
-DF V3n operator*(Dn s, V3n a) { return V3n{s * a.x, s * a.y, s * a.z}; }
-DF V3n operator*(V3n a, Dn s) { return V3n{a.x * s, a.y * s, a.z * s}; }
-DF V3n operator/(V3n a, Dn s) { return V3n{a.x / s, a.y / s, a.z / s}; }
-DF Dn dotn(V3n a, V3n b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
-
-// hllcFace() (icsf_flux.h, hllcFluxScheme.C:76-221) on dual numbers, no
-// frame velocity; br: the switches (Sl, Sr choices, the signs of Sl, Sr,
-// Sm, the fabs argument).
-DF void hllcDual(double gIv, V3n S, Dn magS, Dn rl, Dn rr, Dn pl, Dn pr, V3n Ul, V3n Ur, Dn cl, Dn cr, Dn El,
-                 Dn Er, Dn Hl, Dn Hr, Dn& phi, V3n& phiU, Dn& phiE, int* br) {
-    const Dn gI = cst(gIv), one = cst(1.0);
-    const V3n n = S / magS;
-    const Dn coefR = dsqrt(dmax(cst(kVSMALL), rr) / dmax(cst(kVSMALL), rl));
-    const V3n uAvg = (coefR * Ur + Ul) / (coefR + one);
-    const Dn HAvg = (coefR * Hr + Hl) / (coefR + one);
-    const Dn arg = (gI - one) * (HAvg - cst(0.5) * dotn(uAvg, uAvg));
-    const Dn cAvg = dsqrt(dfabs(arg));
-    const Dn ul = dotn(Ul, n), ur = dotn(Ur, n), ua = dotn(uAvg, n);
-    const Dn Sl = dmin(ul - cl, ua - cAvg);
-    const Dn Sr = dmax(ur + cr, ua + cAvg);
-    const Dn Sm = (rr * ur * (Sr - ur) - rl * ul * (Sl - ul) + pl - pr) / (rr * (Sr - ur) - rl * (Sl - ul));
-    const Dn cSl = cst(Sl.v > 0 ? 1.0 : 0.0), cSr = cst(Sr.v < 0 ? 1.0 : 0.0), cSm = cst(Sm.v > 0 ? 1.0 : 0.0);
-    if (br)
-        *br = (int)((ua - cAvg).v < (ul - cl).v) | (int)((ur + cr).v < (ua + cAvg).v) << 1 | (int)(Sl.v > 0) << 2 |
-              (int)(Sr.v < 0) << 3 | (int)(Sm.v > 0) << 4 | (int)(arg.v < 0) << 5;
-    const Dn cSlm = (one - cSl) * cSm, cSmr = (one - cSm) * (one - cSr);
-    const Dn frl = Sm / (Sl - Sm) * ((Sl - ul) * rl);
-    const Dn frr = Sm / (Sr - Sm) * ((Sr - ur) * rr);
-    phi = (cSl * rl * ul + cSlm * frl + cSmr * frr + cSr * rr * ur) * magS;
-    const Dn psl = rl * (ul - Sl) * (ul - Sm) + pl;
-    const Dn psr = rr * (ur - Sr) * (ur - Sm) + pr;
-    const V3n rUsl = one / (Sl - Sm) * ((Sl - ul) * rl * Ul + (psl - pl) * n);
-    const V3n rUsr = one / (Sr - Sm) * ((Sr - ur) * rr * Ur + (psr - pr) * n);
-    const V3n fUl = Sm * rUsl + psl * n;
-    const V3n fUr = Sm * rUsr + psr * n;
-    phiU = (cSl * (rl * ul * Ul + pl * n) + cSlm * fUl + cSmr * fUr + cSr * (rr * ur * Ur + pr * n)) * magS;
-    const Dn rEsl = one / (Sl - Sm) * ((Sl - ul) * (rl * El) - pl * ul + psl * Sm);
-    const Dn rEsr = one / (Sr - Sm) * ((Sr - ur) * (rr * Er) - pr * ur + psr * Sm);
-    const Dn fEl = Sm * (rEsl + psl);
-    const Dn fEr = Sm * (rEsr + psr);
-    phiE = (cSl * rl * Hl * ul + cSlm * fEl + cSmr * fEr + cSr * rr * Hr * ur) * magS;
-}
-
-// Reverse of the HLLC face flux: one dual pass per face value (owner side
-// L, neighbour side R, fields F_RHO..F_CS) and, with geom, per Sf
-// component; each input's adjoint is the flux adjoint contracted with
-// that pass's tangent.
-DF void hllcFaceRev(double gI, V3 S, const double* L, const double* R, double bphi, V3 bphiU, double bphiE,
-                    double* bL, double* bR, V3& bS, int* branches, bool geom) {
-    const int nIn = geom ? 2 * NFLD + 3 : 2 * NFLD;
-    double bs[3] = {0, 0, 0};
-    for (int i = 0; i < nIn; ++i) {
-        Dn l[NFLD], r[NFLD];
-#pragma unroll
-        for (int k = 0; k < NFLD; ++k) {
-            l[k] = Dn{L[k], i == k ? 1.0 : 0.0};
-            r[k] = Dn{R[k], i == NFLD + k ? 1.0 : 0.0};
-        }
-        const V3n Sd{Dn{S.x, i == 2 * NFLD ? 1.0 : 0.0}, Dn{S.y, i == 2 * NFLD + 1 ? 1.0 : 0.0},
-                     Dn{S.z, i == 2 * NFLD + 2 ? 1.0 : 0.0}};
-        const Dn magS = dsqrt(dotn(Sd, Sd));
-        Dn ph, pe;
-        V3n pu;
-        hllcDual(gI, Sd, magS, l[F_RHO], r[F_RHO], l[F_P], r[F_P], V3n{l[F_UX], l[F_UY], l[F_UZ]},
-                 V3n{r[F_UX], r[F_UY], r[F_UZ]}, l[F_CS], r[F_CS], l[F_E], r[F_E], l[F_H], r[F_H], ph, pu, pe,
-                 i == 0 ? branches : nullptr);
-        const double t = bphi * ph.d + (bphiU.x * pu.x.d + bphiU.y * pu.y.d + bphiU.z * pu.z.d) + bphiE * pe.d;
-        if (i < NFLD) bL[i] = t;
-        else if (i < 2 * NFLD) bR[i - NFLD] = t;
-        else bs[i - 2 * NFLD] = t;
-    }
-    bS = V3{bs[0], bs[1], bs[2]};
 }
 
 // Reverse of ausmFace(): adjoints of the owner-side (L) and neighbour-side
@@ -290,18 +194,26 @@ DF void ausmFaceAdj(bool lowMach, V3 S, double magS, const double* L, const doub
 }
 
 // Face pass: adjoint of the face flux from v (b_owner gets -F, b_neighbour
-// +F), AUSM+up reverse, reconstruction reverse into Cf.
+// +F), the scheme's reverse, and with geom the flux part of the Sf and Cf
+// adjoints (reconstruction into Cf).  Bound by its gathers (both cells'
+// field and gradient rows), which are read as 128-bit rows; the rows are read
+// again for Cf rather than held through the reverse.  AUSM+up with geometry
+// at 96^3: 510 us read entry by entry -> 372 us; HLLC at 61x57x50: 375 us with
+// a dual-number pass per face value -> 62 us with the hand-written reverse.
 template <int SCH>
 __global__ void __launch_bounds__(256) k_adj_face(MeshView m, Phys ph, StateView s, AdjView a,
                                                   const double* __restrict__ v, double* __restrict__ gS,
                                                   double* __restrict__ gC, bool geom) {
     const int f = xcdBlock() * blockDim.x + threadIdx.x;
     if (f >= m.nF) return;
+    double out[2 * NFLD];
+#pragma unroll
+    for (int k = 0; k < 2 * NFLD; ++k) out[k] = 0.0;
     double* lr = a.fLR + (size_t)f * 2 * NFLD;
     if (f >= m.nI && m.bKind[f - m.nI] == PK_EMPTY) {
-#pragma unroll
-        for (int k = 0; k < 2 * NFLD; ++k) lr[k] = 0.0;
-        for (int d = 0; d < 3; ++d) { gS[3 * (size_t)f + d] = 0.0; gC[3 * (size_t)f + d] = 0.0; }
+        stRow(lr, out);
+        if (geom)
+            for (int d = 0; d < 3; ++d) { gS[3 * (size_t)f + d] = 0.0; gC[3 * (size_t)f + d] = 0.0; }
         if (a.fbr) a.fbr[f] = 0;
         return;
     }
@@ -314,21 +226,21 @@ __global__ void __launch_bounds__(256) k_adj_face(MeshView m, Phys ph, StateView
     for (int q = 0; q < 5; ++q) bf[q] = internal ? v[q * nC + n] - v[q * nC + o] : -v[q * nC + o];
     double L[NFLD], R[NFLD];
     if (internal) {
-#pragma unroll
-        for (int k = 0; k < NFLD; ++k)
-            if (used(ph.flux, k)) recon(m, s, ph.recon, f, o, n, k, L[k], R[k]);
-            else L[k] = R[k] = 0.0;
+        double fo[NFLD], fn[NFLD];
+        ldRow(s.fld + (size_t)o * NFLD, fo);
+        ldRow(s.fld + (size_t)n * NFLD, fn);
+        reconRows(m, s, ph.recon, SCH == FLUX_ROE ? NFLD - 1 : NFLD, f, o, n, fo, fn, L, R);
     } else {
-        const double* bv = s.bfld + (size_t)(f - m.nI) * NFLD;
+        ldRow(s.bfld + (size_t)(f - m.nI) * NFLD, L);
 #pragma unroll
-        for (int k = 0; k < NFLD; ++k) L[k] = R[k] = bv[k];
+        for (int k = 0; k < NFLD; ++k) R[k] = L[k];
     }
     const V3 S = ld3(m.Sf + 3 * (size_t)f);
     double bL[NFLD], bR[NFLD];
     V3 bS;
     if constexpr (SCH == FLUX_HLLC) {
         hllcFaceRev(ph.gamma, S, L, R, bf[0], V3{bf[2], bf[3], bf[4]}, bf[1], bL, bR, bS,
-                    a.fbr ? a.fbr + f : nullptr, geom);
+                    a.fbr ? a.fbr + f : nullptr);
         // on a boundary face both sides are the boundary state, where every
         // branch gives the physical flux: no switch of the derivative
         if (a.fbr && !internal) a.fbr[f] = 0;
@@ -349,22 +261,23 @@ __global__ void __launch_bounds__(256) k_adj_face(MeshView m, Phys ph, StateView
         // U.n)
         if (a.fbr && !internal) a.fbr[f] &= ~((1 << 2) | (1 << 9));
     }
+#pragma unroll
+    for (int k = 0; k < NFLD; ++k) {
+        out[k] = internal ? bL[k] : bL[k] + bR[k];
+        out[NFLD + k] = internal ? bR[k] : 0.0;
+    }
+    stRow(lr, out);
+    if (!geom) return;
     V3 bC{0, 0, 0};
-    if (internal) {
+    if (internal && ph.recon == 1) {
+        double go[3 * NFLD], gn[3 * NFLD];
+        ldRow(s.grd + (size_t)o * NFLD * 3, go);
+        ldRow(s.grd + (size_t)n * NFLD * 3, gn);
 #pragma unroll
-        for (int k = 0; k < NFLD; ++k) { lr[k] = bL[k]; lr[NFLD + k] = bR[k]; }
-        if (ph.recon == 1) {
-#pragma unroll
-            for (int k = 0; k < NFLD; ++k) {
-                if (!used(ph.flux, k)) continue;
-                const V3 go = ld3(s.grd + ((size_t)o * NFLD + k) * 3);
-                const V3 gn = ld3(s.grd + ((size_t)n * NFLD + k) * 3);
-                bC = bC + bL[k] * go + bR[k] * gn;
-            }
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < NFLD; ++k) { lr[k] = bL[k] + bR[k]; lr[NFLD + k] = 0.0; }
+        for (int k = 0; k < NFLD; ++k)
+            if (used(SCH, k))
+                bC = bC + bL[k] * V3{go[3 * k], go[3 * k + 1], go[3 * k + 2]} +
+                     bR[k] * V3{gn[3 * k], gn[3 * k + 1], gn[3 * k + 2]};
     }
     gS[3 * (size_t)f] = bS.x; gS[3 * (size_t)f + 1] = bS.y; gS[3 * (size_t)f + 2] = bS.z;
     gC[3 * (size_t)f] = bC.x; gC[3 * (size_t)f + 1] = bC.y; gC[3 * (size_t)f + 2] = bC.z;
@@ -488,14 +401,20 @@ __global__ void __launch_bounds__(256) k_adj_visc(MeshView m, Phys ph, StateView
 // Cell pass: the adjoint of the limited gradients and of the cell values
 // (linearUpwind), then the limiter reverse (recomputing each field's
 // max/min neighbour and the face that set its limiter), then the
-// Gauss-gradient adjoint divided by V.  All fields are carried together,
-// so the cell's faces are walked twice (once for the face adjoints and the
-// max/min, once for the limiter faces) whatever the number of fields; per
-// field the operations and their order are those of the forward kernels.
-template <bool VISC>
-__global__ void __launch_bounds__(256) k_adj_cell(MeshView m, Phys ph, StateView s, AdjView a) {
-    const int c = xcdBlock() * blockDim.x + threadIdx.x;
-    if (c >= m.nC) return;
+// Gauss-gradient adjoint divided by V.  The fields are independent here, so a
+// thread carries NK of them, from K0, through both walks over the cell's
+// faces (face adjoints and max/min, then the limiter faces); per field the
+// operations and their order are those of the forward kernels.  With all
+// eight the walks' state left one wavefront per SIMD: 96^3 AUSM+up 621 -> 468
+// us, 48^3 viscous Roe 110 -> 91 us.  Both halves of a cell belong to one
+// workgroup, so that the rows they share stay in its caches (halves in
+// separate workgroups: 739 us).
+constexpr int NKC = NFLD / 2;
+constexpr int kAdjCellBlock = 128;
+template <bool VISC, int K0>
+__device__ __forceinline__ void adjCellBody(const MeshView& m, const Phys& ph, const StateView& s, const AdjView& a,
+                                            int c) {
+    constexpr int NK = NKC;
     const int e0 = m.cfOff[c], e1 = m.cfOff[c + 1];
     const V3 Cc = ld3(m.C + 3 * (size_t)c);
     const double Vc = m.V[c];
@@ -504,20 +423,22 @@ __global__ void __launch_bounds__(256) k_adj_cell(MeshView m, Phys ph, StateView
     // records pass (a.fbr set): the limiter's active face and max/min
     // element are found for every field, whatever the adjoint seed
     const bool records = a.fbr != nullptr;
-    double qd[NFLD], mx[NFLD], mn[NFLD], vcr[NFLD];
-    V3 gl[NFLD];
-    int imx[NFLD], imn[NFLD];
-    ldRow(s.fld + (size_t)c * NFLD, vcr);
+    double qd[NK], mx[NK], mn[NK], vcr[NK];
+    V3 gl[NK];
+    int imx[NK], imn[NK];
+    ldRow(s.fld + (size_t)c * NFLD + K0, vcr);
 #pragma unroll
-    for (int k = 0; k < NFLD; ++k) {
-        qd[k] = 0.0;
-        gl[k] = V3{0, 0, 0};
-        mx[k] = mn[k] = vcr[k];
-        imx[k] = imn[k] = -1;
+    for (int i = 0; i < NK; ++i) {
+        qd[i] = 0.0;
+        gl[i] = V3{0, 0, 0};
+        mx[i] = mn[i] = vcr[i];
+        imx[i] = imn[i] = -1;
     }
-    // viscous: adjoint of the cell's Gauss grad(U) (zu, row-major) and
-    // grad(e) sums from the viscous face pass
-    constexpr bool visc = VISC;
+    // viscous: adjoint of the cell's Gauss grad(U) columns of this half's
+    // velocity components (zu, row-major) and of grad(e) (the last half),
+    // from the viscous face pass
+    constexpr bool GE = VISC && K0 + NK == NFLD;
+    auto isU = [](int k) { return VISC && k >= F_UX && k <= F_UZ; };
     double zu[9];
     V3 ges{0, 0, 0};
 #pragma unroll
@@ -535,25 +456,30 @@ __global__ void __launch_bounds__(256) k_adj_cell(MeshView m, Phys ph, StateView
                               : ld3(m.Cf + 3 * (size_t)f)) - Cc;
         const double* vo;
         int id;
-        if (visc) {
+        if (VISC) {
             // grad(U) and grad(e) sum adjoints: the first 12 entries of the row
             double vz[VS_GE + 3];
             ldRow(a.vis + (size_t)f * NVIS, vz);
             const double wt = f < m.nI ? (j >= nLo ? m.w[f] : 1.0 - m.w[f]) : 1.0;
 #pragma unroll
-            for (int i = 0; i < 9; ++i) zu[i] += wt * vz[VS_Z + i];
-            ges = ges + wt * V3{vz[VS_GE], vz[VS_GE + 1], vz[VS_GE + 2]};
+            for (int i = 0; i < NK; ++i) {
+                if (!isU(K0 + i)) continue;
+                const int u = K0 + i - F_UX;
+#pragma unroll
+                for (int r = 0; r < 3; ++r) zu[3 * r + u] += wt * vz[VS_Z + 3 * r + u];
+            }
+            if (GE) ges = ges + wt * V3{vz[VS_GE], vz[VS_GE + 1], vz[VS_GE + 2]};
         }
         if (f < m.nI) {
             const bool isOwn = j >= nLo;
-            double lr[NFLD];
-            ldRow(a.fLR + (size_t)f * 2 * NFLD + (isOwn ? 0 : NFLD), lr);
+            double lr[NK];
+            ldRow(a.fLR + (size_t)f * 2 * NFLD + (isOwn ? 0 : NFLD) + K0, lr);
 #pragma unroll
-            for (int k = 0; k < NFLD; ++k) {
-                if (!used(ph.flux, k)) continue;
-                const double av = lr[k];
-                qd[k] += av;
-                if (rec) gl[k] = gl[k] + av * d;
+            for (int i = 0; i < NK; ++i) {
+                if (!used(ph.flux, K0 + i)) continue;
+                const double av = lr[i];
+                qd[i] += av;
+                if (rec) gl[i] = gl[i] + av * d;
             }
             id = m.col[sk];
             vo = s.fld + (size_t)id * NFLD;
@@ -563,135 +489,215 @@ __global__ void __launch_bounds__(256) k_adj_cell(MeshView m, Phys ph, StateView
             vo = s.bfld + (size_t)b * NFLD;
         }
         if (limit) {
-            double vr[NFLD];
-            ldRow(vo, vr);
+            double vr[NK];
+            ldRow(vo + K0, vr);
 #pragma unroll
-            for (int k = 0; k < NFLD; ++k) {
-                if (!used(ph.flux, k)) continue;
-                const double v = vr[k];
+            for (int i = 0; i < NK; ++i) {
+                if (!used(ph.flux, K0 + i)) continue;
+                const double v = vr[i];
                 // records pass: a candidate within rounding of the current
                 // max/min does not displace it.  Such ties are two equal
                 // functions of the state computed two ways (H of a cell and
                 // of its zeroGradient outlet face: E + p/rho with p/rho = R T
                 // on both sides), whose order follows the rounding, so that
                 // any step flips them while the derivative does not change.
-                const double tx = records ? 1e-12 * fabs(mx[k]) : 0.0;
-                const double tn = records ? 1e-12 * fabs(mn[k]) : 0.0;
-                if (mx[k] + tx < v) { mx[k] = v; imx[k] = id; }
-                if (v < mn[k] - tn) { mn[k] = v; imn[k] = id; }
+                const double tx = records ? 1e-12 * fabs(mx[i]) : 0.0;
+                const double tn = records ? 1e-12 * fabs(mn[i]) : 0.0;
+                if (mx[i] + tx < v) { mx[i] = v; imx[i] = id; }
+                if (v < mn[i] - tn) { mn[i] = v; imn[i] = id; }
             }
         }
     }
-    V3 g[NFLD], gb[NFLD];
-    double limb[NFLD];
+    V3 g[NK], gb[NK];
+    double limb[NK];
     bool any = false;
-    double gunr[3 * NFLD], limr[NFLD];
+    double gunr[3 * NK], limr[NK];
     if (rec) {
-        ldRow(a.gun + (size_t)c * NFLD * 3, gunr);
-        ldRow(a.lim + (size_t)c * NFLD, limr);
+        ldRow(a.gun + ((size_t)c * NFLD + K0) * 3, gunr);
+        ldRow(a.lim + (size_t)c * NFLD + K0, limr);
     }
 #pragma unroll
-    for (int k = 0; k < NFLD; ++k) {
-        g[k] = gb[k] = V3{0, 0, 0};
-        limb[k] = 0.0;
-        if (!used(ph.flux, k) || !rec) continue;
-        g[k] = V3{gunr[3 * k], gunr[3 * k + 1], gunr[3 * k + 2]};
-        gb[k] = limr[k] * gl[k];
-        limb[k] = dot(gl[k], g[k]);
-        if (limit && (limb[k] != 0.0 || records)) any = true;
+    for (int i = 0; i < NK; ++i) {
+        g[i] = gb[i] = V3{0, 0, 0};
+        limb[i] = 0.0;
+        if (!used(ph.flux, K0 + i) || !rec) continue;
+        g[i] = V3{gunr[3 * i], gunr[3 * i + 1], gunr[3 * i + 2]};
+        gb[i] = limr[i] * gl[i];
+        limb[i] = dot(gl[i], g[i]);
+        if (limit && (limb[i] != 0.0 || records)) any = true;
     }
-    int fs[NFLD], br[NFLD];
-    double lm[NFLD], rs[NFLD], es[NFLD], mxD[NFLD], mnD[NFLD];
+    int fs[NK], br[NK];
+    double lm[NK], rs[NK], es[NK], mxD[NK], mnD[NK];
 #pragma unroll
-    for (int k = 0; k < NFLD; ++k) {
-        fs[k] = -1; br[k] = 0; lm[k] = 1.0; rs[k] = 1.0; es[k] = 0.0;
-        mxD[k] = mx[k] - vcr[k];
-        mnD[k] = mn[k] - vcr[k];
+    for (int i = 0; i < NK; ++i) {
+        fs[i] = -1; br[i] = 0; lm[i] = 1.0; rs[i] = 1.0; es[i] = 0.0;
+        mxD[i] = mx[i] - vcr[i];
+        mnD[i] = mn[i] - vcr[i];
     }
     if (any) {
         for (int q = e0; q < e1; ++q) {
             const int f = m.cf[q];
-            const V3 d = ld3(m.Cf + 3 * (size_t)f) - Cc;
+            const int j = q - e0;
+            const size_t sk = rslot + 64 * (size_t)j;
+            const V3 d = (j < len ? V3{m.sgeo[sgOff(sk, SG_CX)], m.sgeo[sgOff(sk, SG_CX + 1)],
+                                       m.sgeo[sgOff(sk, SG_CX + 2)]}
+                                  : ld3(m.Cf + 3 * (size_t)f)) - Cc;
 #pragma unroll
-            for (int k = 0; k < NFLD; ++k) {
-                if (!used(ph.flux, k) || (limb[k] == 0.0 && !records)) continue;
-                const double ext = dot(d, g[k]);
+            for (int i = 0; i < NK; ++i) {
+                if (!used(ph.flux, K0 + i) || (limb[i] == 0.0 && !records)) continue;
+                const double ext = dot(d, g[i]);
                 double r = 1;
                 int bq = 0;
-                if (ext > kSMALL) { r = mxD[k] / ext; bq = 1; }
-                else if (ext < -kSMALL) { r = mnD[k] / ext; bq = -1; }
+                if (ext > kSMALL) { r = mxD[i] / ext; bq = 1; }
+                else if (ext < -kSMALL) { r = mnD[i] / ext; bq = -1; }
                 double l;
                 if (ph.limiter == 1) l = (sqr(r) + 2 * r) / (sqr(r) + r + 2);
                 else l = fmin(r, 1.0);
-                if (l < lm[k]) { lm[k] = l; fs[k] = f; rs[k] = r; es[k] = ext; br[k] = bq; }
+                if (l < lm[i]) { lm[i] = l; fs[i] = f; rs[i] = r; es[i] = ext; br[i] = bq; }
             }
         }
     }
-    static_assert(NFLD % 2 == 0, "fields stored in pairs");
-    double pq = 0.0, pv = 0.0, px = 0.0;
-    int pt = -1, pf = -1;
-    V3 pG{0, 0, 0};
+    static_assert(NK == 4, "rows stored as four fields");
+    double qo[NK], tv[NK], fx[NK], Go[3 * NK];
+    int tg[NK], fo[NK];
 #pragma unroll
-    for (int k = 0; k < NFLD; ++k) {
-        const size_t ck = (size_t)c * NFLD + k;
-        int tgt = -1, fsk = -1;
-        double tv = 0.0, fx = 0.0, qk = qd[k];
+    for (int i = 0; i < NK; ++i) {
+        const int k = K0 + i;
+        tg[i] = fo[i] = -1;
+        tv[i] = fx[i] = 0.0;
+        double qk = qd[i];
         V3 G{0, 0, 0};
         // viscous: grad(U_j) is the unlimited Gauss gradient of field U_j
-        const bool vk = visc && k >= F_UX && k <= F_UZ;
-        if (vk && !rec) G = V3{zu[k - F_UX], zu[3 + k - F_UX], zu[6 + k - F_UX]} / Vc;
+        V3 z{0, 0, 0};
+        if (isU(k)) z = V3{zu[k - F_UX], zu[3 + k - F_UX], zu[6 + k - F_UX]};
+        if (isU(k) && !rec) G = z / Vc;
         if (used(ph.flux, k) && rec) {
-            V3 gbk = gb[k];
-            if (vk) gbk = gbk + V3{zu[k - F_UX], zu[3 + k - F_UX], zu[6 + k - F_UX]};
-            if (limit && (limb[k] != 0.0 || records) && fs[k] >= 0 && br[k] != 0) {
+            V3 gbk = gb[i];
+            if (isU(k)) gbk = gbk + z;
+            if (limit && (limb[i] != 0.0 || records) && fs[i] >= 0 && br[i] != 0) {
                 double dl;
                 if (ph.limiter == 1) {
-                    const double den = sqr(rs[k]) + rs[k] + 2;
-                    dl = (-sqr(rs[k]) + 4 * rs[k] + 4) / sqr(den);
-                } else dl = rs[k] <= 1.0 ? 1.0 : 0.0;
-                const double rb = limb[k] * dl;
-                const double numb = rb / es[k];
-                fx = -rb * rs[k] / es[k];
-                fsk = fs[k];
-                gbk = gbk + fx * (ld3(m.Cf + 3 * (size_t)fsk) - Cc);
-                const int id = br[k] > 0 ? imx[k] : imn[k];
+                    const double den = sqr(rs[i]) + rs[i] + 2;
+                    dl = (-sqr(rs[i]) + 4 * rs[i] + 4) / sqr(den);
+                } else dl = rs[i] <= 1.0 ? 1.0 : 0.0;
+                const double rb = limb[i] * dl;
+                const double numb = rb / es[i];
+                fx[i] = -rb * rs[i] / es[i];
+                fo[i] = fs[i];
+                gbk = gbk + fx[i] * (ld3(m.Cf + 3 * (size_t)fs[i]) - Cc);
+                const int id = br[i] > 0 ? imx[i] : imn[i];
                 if (id >= 0) {
-                    tgt = id;
-                    tv = numb;
+                    tg[i] = id;
+                    tv[i] = numb;
                     qk -= numb;
                 }
             }
             G = gbk / Vc;
         }
-        // stored a pair of fields at a time (128-bit stores; 64-bit for
-        // the int rows): the even field is held until the odd one is done
-        const double qv = used(ph.flux, k) ? qk : 0.0;
-        if (k & 1) {
-            const size_t c0 = ck - 1;
-            *reinterpret_cast<double2*>(a.qc + c0) = double2{pq, qv};
-            *reinterpret_cast<int2*>(a.tgt + c0) = int2{pt, tgt};
-            *reinterpret_cast<double2*>(a.tval + c0) = double2{pv, tv};
-            *reinterpret_cast<int2*>(a.fst + c0) = int2{pf, fsk};
-            *reinterpret_cast<double2*>(a.fext + c0) = double2{px, fx};
-            double2* gq = reinterpret_cast<double2*>(a.G + 3 * c0);
-            gq[0] = double2{pG.x, pG.y};
-            gq[1] = double2{pG.z, G.x};
-            gq[2] = double2{G.y, G.z};
-        } else {
-            pq = qv; pt = tgt; pv = tv; pf = fsk; px = fx; pG = G;
-        }
+        qo[i] = used(ph.flux, k) ? qk : 0.0;
+        Go[3 * i] = G.x; Go[3 * i + 1] = G.y; Go[3 * i + 2] = G.z;
     }
-    if (visc) {
+    const size_t ck = (size_t)c * NFLD + K0;
+    stRow(a.qc + ck, qo);
+    stRow(a.tval + ck, tv);
+    stRow(a.fext + ck, fx);
+    stRow(a.G + 3 * ck, Go);
+    *reinterpret_cast<int4*>(a.tgt + ck) = int4{tg[0], tg[1], tg[2], tg[3]};
+    *reinterpret_cast<int4*>(a.fst + ck) = int4{fo[0], fo[1], fo[2], fo[3]};
+    if (GE) {
         const V3 Ge = ges / Vc;
         a.Ge[3 * (size_t)c] = Ge.x; a.Ge[3 * (size_t)c + 1] = Ge.y; a.Ge[3 * (size_t)c + 2] = Ge.z;
     }
 }
+template <bool VISC>
+__global__ void __launch_bounds__(kAdjCellBlock) k_adj_cell(MeshView m, Phys ph, StateView s, AdjView a) {
+    const int c = xcdBlock() * (kAdjCellBlock / 2) + threadIdx.x % (kAdjCellBlock / 2);
+    if (c >= m.nC) return;
+    if (threadIdx.x < kAdjCellBlock / 2) adjCellBody<VISC, 0>(m, ph, s, a, c);
+    else adjCellBody<VISC, NKC>(m, ph, s, a, c);
+}
 
-// Face pass 2: Gauss-gradient face values (internal faces: adjoint of
-// w*(q_o - q_n) + q_n for the cell pull, Sf part), boundary values
-// (flux + Gauss + limiter max/min) chained through rho_b = p_b/(R T_b),
-// E_b, H_b, c*_b to the owner's p, T, U and to Sf (slip normal), and the
-// limiter's Cf part.
+// Boundary face f: its values' adjoint (flux + Gauss + limiter max/min),
+// chained through rho_b = p_b/(R T_b), E_b, H_b, c*_b to the owner's p, T, U
+// (a.bprim), and to Sf (Gauss sum, slip normal) and Cf (the limiter's part).
+template <bool VISC>
+__device__ __forceinline__ void adjBoundaryFace(const MeshView& m, const Phys& ph, const StateView& s,
+                                                const AdjView& a, int f, V3& bS, V3& bC) {
+    const V3 S = ld3(m.Sf + 3 * (size_t)f);
+    const int o = m.own[f];
+    const bool rec = ph.recon == 1;
+    constexpr bool visc = VISC;
+    const auto grads = [&](int k) { return (used(ph.flux, k) && rec) || (visc && k >= F_UX && k <= F_UZ); };
+    const int b = f - m.nI;
+    const double* bv = s.bfld + (size_t)b * NFLD;
+    const double* lr = a.fLR + (size_t)f * 2 * NFLD;
+    double qb[NFLD];
+#pragma unroll
+    for (int k = 0; k < NFLD; ++k) {
+        qb[k] = 0.0;
+        if (used(ph.flux, k)) qb[k] = lr[k];
+        if (grads(k)) {
+            const size_t ok = (size_t)o * NFLD + k;
+            const V3 Go = ld3(a.G + 3 * ok);
+            qb[k] += dot(S, Go);
+            if (a.tgt[ok] == m.nC + b) qb[k] += a.tval[ok];
+            bS = bS + bv[k] * Go;
+            if (a.fst[ok] == f) bC = bC + a.fext[ok] * ld3(a.gun + 3 * ok);
+        }
+    }
+    // c*_b = sqrt(kappa H_b), H_b = max(E_b, SMALL) + max(p_b/rho_b, SMALL)
+    const double g = ph.gamma;
+    const double kap = 2.0 * (g - 1.0) / (g + 1.0);
+    double Hb = qb[F_H];
+    const bool hllc = ph.flux == FLUX_HLLC;
+    if (!hllc && bv[F_CS] > 0.0) Hb += qb[F_CS] * kap / (2.0 * bv[F_CS]);
+    const double TB = s.bT[b];
+    const double pB = bv[F_P], rhoB = bv[F_RHO];
+    const V3 UB{bv[F_UX], bv[F_UY], bv[F_UZ]};
+    const double EB = ph.Cv * TB + 0.5 * magSqr(UB);
+    double Eb = qb[F_E], pb = qb[F_P], rb = qb[F_RHO];
+    V3 Ub{qb[F_UX], qb[F_UY], qb[F_UZ]};
+    if (!(EB < kSMALL)) Eb += Hb;
+    const double pr = pB / rhoB;
+    if (!(pr < kSMALL)) { pb += Hb / rhoB; rb -= Hb * pr / rhoB; }
+    double Tb = ph.Cv * Eb;
+    // HLLC: c_b = max(sqrt(gamma/psi_b), VSMALL), sqrt(gamma R T_b)
+    if (hllc && !(bv[F_CS] < kVSMALL)) Tb += qb[F_CS] * g * ph.R / (2.0 * bv[F_CS]);
+    Ub = Ub + Eb * UB;
+    if (visc) {
+        // the viscous terms' boundary U, and the boundary e of grad(e)
+        // and of laplacian(alphaEff, e): e_b = rhoE_b / rho_b - |U_b|^2 / 2
+        // with rhoE_b = rho_b (Cv T_b + |U_b|^2 / 2), i.e. Cv T_b
+        const double* vs = a.vis + (size_t)f * NVIS;
+        Ub = Ub + V3{vs[VS_UN], vs[VS_UN + 1], vs[VS_UN + 2]};
+        Tb += ph.Cv * (vs[VS_EN] + dot(S, ld3(a.Ge + 3 * (size_t)o)));
+    }
+    // rho_b = psi p_b, psi = 1/(R T_b)
+    const double psi = 1.0 / (ph.R * TB);
+    pb += rb * psi;
+    Tb -= rb * pB * psi / TB;
+    double* bp = a.bprim + (size_t)b * 5;
+    bp[0] = m.bPT[b] == BC_FIXED ? 0.0 : pb;
+    bp[1] = m.bTT[b] == BC_FIXED ? 0.0 : Tb;
+    V3 Uc_b{0, 0, 0};
+    const int ut = m.bUT[b];
+    if (ut == BC_ZG) Uc_b = Ub;
+    else if (ut == BC_SLIP) {
+        // U_b = U_c - n (n.U_c), n = Sf/|Sf|
+        const double ms = m.magSf[f];
+        const V3 nn = S / ms;
+        const V3 Uc = cellU(s.fld, o);
+        const double nUb = dot(nn, Ub), nUc = dot(nn, Uc);
+        Uc_b = Ub - nUb * nn;
+        const V3 nb = (-nUc) * Ub - nUb * Uc;
+        bS = bS + (nb - dot(nn, nb) * nn) / ms;
+    }
+    bp[2] = Uc_b.x; bp[3] = Uc_b.y; bp[4] = Uc_b.z;
+}
+
+// Face pass 2 of the geometry adjoint: Gauss-gradient face values (internal
+// faces: adjoint of w*(q_o - q_n) + q_n for the cell pull, Sf part), the
+// boundary faces, and the limiter's Cf part.
 template <bool VISC>
 __global__ void __launch_bounds__(256) k_adj_gauss(MeshView m, Phys ph, StateView s, AdjView a,
                                                    double* __restrict__ gS, double* __restrict__ gC) {
@@ -699,8 +705,6 @@ __global__ void __launch_bounds__(256) k_adj_gauss(MeshView m, Phys ph, StateVie
     if (f >= m.nF) return;
     double* qf = a.qf + (size_t)f * NFLD;
     if (f >= m.nI && m.bKind[f - m.nI] == PK_EMPTY) {
-#pragma unroll
-        for (int k = 0; k < NFLD; ++k) qf[k] = 0.0;
         double* bp = a.bprim + (size_t)(f - m.nI) * 5;
         for (int q = 0; q < 5; ++q) bp[q] = 0.0;
         return;
@@ -746,82 +750,33 @@ __global__ void __launch_bounds__(256) k_adj_gauss(MeshView m, Phys ph, StateVie
             }
         }
         stRow(qf, qv);
-    } else {
-        const int b = f - m.nI;
-        const double* bv = s.bfld + (size_t)b * NFLD;
-        const double* lr = a.fLR + (size_t)f * 2 * NFLD;
-        double qb[NFLD];
-#pragma unroll
-        for (int k = 0; k < NFLD; ++k) {
-            qf[k] = 0.0;
-            qb[k] = 0.0;
-            if (used(ph.flux, k)) qb[k] = lr[k];
-            if (grads(k)) {
-                const size_t ok = (size_t)o * NFLD + k;
-                const V3 Go = ld3(a.G + 3 * ok);
-                qb[k] += dot(S, Go);
-                if (a.tgt[ok] == m.nC + b) qb[k] += a.tval[ok];
-                bS = bS + bv[k] * Go;
-                if (a.fst[ok] == f) bC = bC + a.fext[ok] * ld3(a.gun + 3 * ok);
-            }
-        }
-        // c*_b = sqrt(kappa H_b), H_b = max(E_b, SMALL) + max(p_b/rho_b, SMALL)
-        const double g = ph.gamma;
-        const double kap = 2.0 * (g - 1.0) / (g + 1.0);
-        double Hb = qb[F_H];
-        const bool hllc = ph.flux == FLUX_HLLC;
-        if (!hllc && bv[F_CS] > 0.0) Hb += qb[F_CS] * kap / (2.0 * bv[F_CS]);
-        const double TB = s.bT[b];
-        const double pB = bv[F_P], rhoB = bv[F_RHO];
-        const V3 UB{bv[F_UX], bv[F_UY], bv[F_UZ]};
-        const double EB = ph.Cv * TB + 0.5 * magSqr(UB);
-        double Eb = qb[F_E], pb = qb[F_P], rb = qb[F_RHO];
-        V3 Ub{qb[F_UX], qb[F_UY], qb[F_UZ]};
-        if (!(EB < kSMALL)) Eb += Hb;
-        const double pr = pB / rhoB;
-        if (!(pr < kSMALL)) { pb += Hb / rhoB; rb -= Hb * pr / rhoB; }
-        double Tb = ph.Cv * Eb;
-        // HLLC: c_b = max(sqrt(gamma/psi_b), VSMALL), sqrt(gamma R T_b)
-        if (hllc && !(bv[F_CS] < kVSMALL)) Tb += qb[F_CS] * g * ph.R / (2.0 * bv[F_CS]);
-        Ub = Ub + Eb * UB;
-        if (visc) {
-            // the viscous terms' boundary U, and the boundary e of grad(e)
-            // and of laplacian(alphaEff, e): e_b = rhoE_b / rho_b - |U_b|^2 / 2
-            // with rhoE_b = rho_b (Cv T_b + |U_b|^2 / 2), i.e. Cv T_b
-            const double* vs = a.vis + (size_t)f * NVIS;
-            Ub = Ub + V3{vs[VS_UN], vs[VS_UN + 1], vs[VS_UN + 2]};
-            Tb += ph.Cv * (vs[VS_EN] + dot(S, ld3(a.Ge + 3 * (size_t)o)));
-        }
-        // rho_b = psi p_b, psi = 1/(R T_b)
-        const double psi = 1.0 / (ph.R * TB);
-        pb += rb * psi;
-        Tb -= rb * pB * psi / TB;
-        double* bp = a.bprim + (size_t)b * 5;
-        bp[0] = m.bPT[b] == BC_FIXED ? 0.0 : pb;
-        bp[1] = m.bTT[b] == BC_FIXED ? 0.0 : Tb;
-        V3 Uc_b{0, 0, 0};
-        const int ut = m.bUT[b];
-        if (ut == BC_ZG) Uc_b = Ub;
-        else if (ut == BC_SLIP) {
-            // U_b = U_c - n (n.U_c), n = Sf/|Sf|
-            const double ms = m.magSf[f];
-            const V3 nn = S / ms;
-            const V3 Uc = cellU(s.fld, o);
-            const double nUb = dot(nn, Ub), nUc = dot(nn, Uc);
-            Uc_b = Ub - nUb * nn;
-            const V3 nb = (-nUc) * Ub - nUb * Uc;
-            bS = bS + (nb - dot(nn, nb) * nn) / ms;
-        }
-        bp[2] = Uc_b.x; bp[3] = Uc_b.y; bp[4] = Uc_b.z;
-    }
+    } else adjBoundaryFace<VISC>(m, ph, s, a, f, bS, bC);
     gS[3 * (size_t)f] += bS.x; gS[3 * (size_t)f + 1] += bS.y; gS[3 * (size_t)f + 2] += bS.z;
     gC[3 * (size_t)f] += bC.x; gC[3 * (size_t)f + 1] += bC.y; gC[3 * (size_t)f + 2] += bC.z;
 }
 
+// The boundary faces alone (no geometry adjoint).
+template <bool VISC>
+__global__ void __launch_bounds__(256) k_adj_boundary(MeshView m, Phys ph, StateView s, AdjView a) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= m.nB) return;
+    if (m.bKind[b] == PK_EMPTY) {
+        double* bp = a.bprim + (size_t)b * 5;
+        for (int q = 0; q < 5; ++q) bp[q] = 0.0;
+        return;
+    }
+    V3 bS{0, 0, 0}, bC{0, 0, 0};
+    adjBoundaryFace<VISC>(m, ph, s, a, m.nI + b, bS, bC);
+}
+
 // Cell pass 2: total cell-value adjoints (direct + Gauss face values +
 // limiter targets of the neighbours + boundary primitives), then
-// c*, H, E -> rho, p, U, T and the updateFields chain back to W.
-template <bool VISC>
+// c*, H, E -> rho, p, U, T and the updateFields chain back to W.  DIRECT (no
+// geometry adjoint): the Gauss face values S . (G_o - G_n) from the neighbours'
+// gradient-adjoint rows, the bits k_adj_gauss would have stored: no face pass
+// over the internal faces, whose results are read by this one only (HLLC,
+// 61x57x50: 125 + 47 us -> 13 us for the boundary faces + 61 us).
+template <bool VISC, bool DIRECT>
 __global__ void __launch_bounds__(256) k_adj_state(MeshView m, Phys ph, StateView s, AdjView a,
                                                    double* __restrict__ gW) {
     const int c = xcdBlock() * blockDim.x + threadIdx.x;
@@ -834,8 +789,13 @@ __global__ void __launch_bounds__(256) k_adj_state(MeshView m, Phys ph, StateVie
     // viscous: direct U and e adjoints of the viscous face terms, and the
     // Gauss face values of e
     constexpr bool visc = VISC;
-    V3 Uv{0, 0, 0};
+    V3 Uv{0, 0, 0}, GeC{0, 0, 0};
     double ecB = 0.0;
+    double Gc[DIRECT ? 3 * NFLD : 2];
+    if constexpr (DIRECT) {
+        ldRow(a.G + (size_t)c * NFLD * 3, Gc);
+        if (visc) GeC = ld3(a.Ge + 3 * (size_t)c);
+    }
     const int nLo = m.nLower[c];
     const size_t rslot = (size_t)m.slicePtr[c >> 6] * 64 + (c & 63);
     for (int e = e0; e < e1; ++e) {
@@ -849,8 +809,18 @@ __global__ void __launch_bounds__(256) k_adj_state(MeshView m, Phys ph, StateVie
             const double wt = isOwn ? wf : 1.0 - wf;
             double qf[NFLD];
             int tg[NFLD];
-            ldRow(a.qf + (size_t)f * NFLD, qf);
             ldRowI(a.tgt + (size_t)j * NFLD, tg);
+            V3 S{0, 0, 0};
+            if constexpr (DIRECT) {
+                S = V3{m.sgeo[sgOff(sk, SG_SX)], m.sgeo[sgOff(sk, SG_SX + 1)], m.sgeo[sgOff(sk, SG_SX + 2)]};
+                double Gn[3 * NFLD];
+                ldRow(a.G + (size_t)j * NFLD * 3, Gn);
+#pragma unroll
+                for (int k = 0; k < NFLD; ++k) {
+                    const V3 gc{Gc[3 * k], Gc[3 * k + 1], Gc[3 * k + 2]}, gn{Gn[3 * k], Gn[3 * k + 1], Gn[3 * k + 2]};
+                    qf[k] = dot(S, isOwn ? gc - gn : gn - gc);
+                }
+            } else ldRow(a.qf + (size_t)f * NFLD, qf);
 #pragma unroll
             for (int k = 0; k < NFLD; ++k) {
                 if (!used(ph.flux, k) && !(visc && k >= F_UX && k <= F_UZ)) continue;
@@ -864,7 +834,12 @@ __global__ void __launch_bounds__(256) k_adj_state(MeshView m, Phys ph, StateVie
                 ldRow(a.vis + (size_t)f * NVIS + VS_UO, vu);
                 const int u0 = (isOwn ? VS_UO : VS_UN) - VS_UO;
                 Uv = Uv + V3{vu[u0], vu[u0 + 1], vu[u0 + 2]};
-                ecB += (isOwn ? vu[VS_EO - VS_UO] : vu[VS_EN - VS_UO]) + wt * a.qe[f];
+                double qe;
+                if constexpr (DIRECT) {
+                    const V3 Gj = ld3(a.Ge + 3 * (size_t)j);
+                    qe = dot(S, isOwn ? GeC - Gj : Gj - GeC);
+                } else qe = a.qe[f];
+                ecB += (isOwn ? vu[VS_EO - VS_UO] : vu[VS_EN - VS_UO]) + wt * qe;
             }
         } else {
             const double* bp = a.bprim + (size_t)(f - m.nI) * 5;
@@ -935,15 +910,22 @@ void launchResidualVjp(const MeshView& m, const Phys& ph, const StateView& s, co
     if (ph.flux == FLUX_ROE) k_adj_face<FLUX_ROE><<<gf, 256, 0, st>>>(m, ph, s, a, v, gS, gC, geom);
     else if (ph.flux == FLUX_HLLC) k_adj_face<FLUX_HLLC><<<gf, 256, 0, st>>>(m, ph, s, a, v, gS, gC, geom);
     else k_adj_face<FLUX_AUSM><<<gf, 256, 0, st>>>(m, ph, s, a, v, gS, gC, geom);
+    const dim3 gc2(xcdGrid((size_t)m.nC * 2, kAdjCellBlock));
+    const int gb = (m.nB + 255) / 256;
     if (ph.viscous) {
         k_adj_visc<<<gf, 256, 0, st>>>(m, ph, s, a, v);
-        k_adj_cell<true><<<gc, 256, 0, st>>>(m, ph, s, a);
-        k_adj_gauss<true><<<gf, 256, 0, st>>>(m, ph, s, a, gS, gC);
-        k_adj_state<true><<<gc, 256, 0, st>>>(m, ph, s, a, gW);
-    } else {
-        k_adj_cell<false><<<gc, 256, 0, st>>>(m, ph, s, a);
+        k_adj_cell<true><<<gc2, kAdjCellBlock, 0, st>>>(m, ph, s, a);
+    } else k_adj_cell<false><<<gc2, kAdjCellBlock, 0, st>>>(m, ph, s, a);
+    if (geom) {
+        // inviscid residuals only
         k_adj_gauss<false><<<gf, 256, 0, st>>>(m, ph, s, a, gS, gC);
-        k_adj_state<false><<<gc, 256, 0, st>>>(m, ph, s, a, gW);
+        k_adj_state<false, false><<<gc, 256, 0, st>>>(m, ph, s, a, gW);
+    } else if (ph.viscous) {
+        if (gb) k_adj_boundary<true><<<gb, 256, 0, st>>>(m, ph, s, a);
+        k_adj_state<true, true><<<gc, 256, 0, st>>>(m, ph, s, a, gW);
+    } else {
+        if (gb) k_adj_boundary<false><<<gb, 256, 0, st>>>(m, ph, s, a);
+        k_adj_state<false, true><<<gc, 256, 0, st>>>(m, ph, s, a, gW);
     }
 }
 
