@@ -160,8 +160,11 @@ void launchExpandBlocks(const MeshView& m, int fp32, const void* gen, void* out,
 void launchProjectionPasses(const MeshView& m, int vecFp32, int ch, int mgs, const void* w, const void* V, int nv,
                             double* part, hipStream_t st);
 
+// State update from Wsrc (null: the state's W) plus dW (null: none); W0 (optional)
+// keeps a copy of Wsrc.
 void launchUpdate(const MeshView& m, const Phys& ph, const StateView& s, const double* dW, int mode,
-                  const double* rho0, const double* U0, const double* T0, hipStream_t st);
+                  const double* rho0, const double* U0, const double* T0, hipStream_t st,
+                  const double* Wsrc = nullptr, double* W0 = nullptr);
 // Forward part of the residual adjoint: boundary values and gradients,
 // keeping the unlimited gradients and limiter values.
 void launchAdjointForward(const MeshView& m, const Phys& ph, const StateView& s, double* gun, double* limo,
@@ -172,8 +175,12 @@ void launchAdjointForward(const MeshView& m, const Phys& ph, const StateView& s,
 void launchResidualVjp(const MeshView& m, const Phys& ph, const StateView& s, const AdjView& a, const double* v,
                        double* gW, double* gS, double* gC, bool geom, hipStream_t st);
 // cellSums false: everything up to the face terms; the cell sums (b,
-// rPseudoDeltaT) are then formed by launchCellSumsJacobian.
-void launchResidual(const MeshView& m, const Phys& ph, const StateView& s, hipStream_t st, bool cellSums = true);
+// rPseudoDeltaT) are then formed by launchCellSumsJacobian.  bOut: b is written
+// there too, and the face records are short ones that the Jacobian cannot read
+// (launchFaceTerms makes the full ones).
+void launchResidual(const MeshView& m, const Phys& ph, const StateView& s, hipStream_t st, bool cellSums = true,
+                    double* bOut = nullptr);
+void launchFaceTerms(const MeshView& m, const Phys& ph, const StateView& s, hipStream_t st);
 void launchFaceFlux(const MeshView& m, const Phys& ph, const StateView& s, double* phi, double* phiU, double* phiE,
                     hipStream_t st);
 void launchJacobian(const MeshView& m, const Phys& ph, const StateView& s, void* blk, void* dg, int fp32,

@@ -15,9 +15,10 @@ namespace {
 
 // Primitive/derived cell fields from conserved W after an increment
 // (updateFields.H:7-78), or from (rho, U, T) at initialisation.
+// Wsrc: the state the increment applies to (null: s.W); W0: keeps a copy of it.
 __global__ void k_update(MeshView m, Phys ph, StateView s, const double* __restrict__ dW, int mode,
                          const double* __restrict__ rho0, const double* __restrict__ U0,
-                         const double* __restrict__ T0) {
+                         const double* __restrict__ T0, const double* Wsrc, double* W0) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= m.nC) return;
     if (s.halt && *s.halt) return;
@@ -33,9 +34,17 @@ __global__ void k_update(MeshView m, Phys ph, StateView s, const double* __restr
         const double psi = 1.0 / (ph.R * T);
         p = rho / psi;
     } else {
-        rho = s.W[c];
-        V3 rU = V3{s.W[2 * (size_t)nC + c], s.W[3 * (size_t)nC + c], s.W[4 * (size_t)nC + c]};
-        double rE = s.W[(size_t)nC + c];
+        const double* Wi = Wsrc ? Wsrc : s.W;
+        rho = Wi[c];
+        V3 rU = V3{Wi[2 * (size_t)nC + c], Wi[3 * (size_t)nC + c], Wi[4 * (size_t)nC + c]};
+        double rE = Wi[(size_t)nC + c];
+        if (W0) {
+            W0[c] = rho;
+            W0[(size_t)nC + c] = rE;
+            W0[2 * (size_t)nC + c] = rU.x;
+            W0[3 * (size_t)nC + c] = rU.y;
+            W0[4 * (size_t)nC + c] = rU.z;
+        }
         if (dW) {
             rho += dW[c];
             rU = V3{rU.x + dW[2 * (size_t)nC + c], rU.y + dW[3 * (size_t)nC + c], rU.z + dW[4 * (size_t)nC + c]};
@@ -458,8 +467,19 @@ __device__ __forceinline__ void faceFlux(const MeshView& m, const Phys& ph, cons
 // Cell kernels then sum these in face order (the reference's face loops).
 // o: the face's NFT-entry record (entries a face kind does not use are
 // left as they are).
+// MODE FT_ALL: that record.  A residual evaluation alone reads the flux, the
+// viscous terms and FT_FRDT: FT_VISC keeps the record's first 16 entries,
+// FT_INV (inviscid) eight, the flux and FT_FRDT in entry 5.  Writing and
+// reading 64 or 128 B per face instead of 192 B is what these are for.
+enum { FT_ALL = 0, FT_VISC = 1, FT_INV = 2 };
+template <int MODE>
+constexpr int ftSize() { return MODE == FT_ALL ? NFT : MODE == FT_VISC ? 16 : 8; }
+template <int MODE>
+constexpr int ftFrdt() { return MODE == FT_INV ? 5 : FT_FRDT; }
+template <int MODE>
 __device__ __forceinline__ void faceTermsBody(const MeshView& m, const Phys& ph, const StateView& s, int f,
                                               double* o) {
+    constexpr bool ALL = MODE == FT_ALL;
     double fr, fe;
     V3 fu;
     double rec[8];
@@ -479,7 +499,7 @@ __device__ __forceinline__ void faceTermsBody(const MeshView& m, const Phys& ph,
     o[FT_CONV + 4] = fu.z;
     const V3 S{ldnt(m.Sf + 3 * (size_t)f), ldnt(m.Sf + 3 * (size_t)f + 1), ldnt(m.Sf + 3 * (size_t)f + 2)};
     const double ms = ldnt(m.magSf + f);
-    const bool visc = ph.viscous;
+    const bool visc = MODE != FT_INV && ph.viscous;
     const double mu = ph.mu, alpha = ph.alpha;
     if (internal) {
         const double w = ldnt(m.w + f);
@@ -488,10 +508,11 @@ __device__ __forceinline__ void faceTermsBody(const MeshView& m, const Phys& ph,
         const V3 Uo{fo[F_UX], fo[F_UY], fo[F_UZ]}, Un{fn[F_UX], fn[F_UY], fn[F_UZ]};
         const V3 Uf = w * (Uo - Un) + Un;
         const double lam = cf + fabs(dot(Uf, S / ms) - um);
-        o[FT_LAM] = lam;
-        o[FT_FRDT] = m.nodc[f] * lam;
+        if (ALL) o[FT_LAM] = lam;
+        o[ftFrdt<MODE>()] = m.nodc[f] * lam;
+        if (ALL)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) o[FT_REC + k] = rec[k];
+            for (int k = 0; k < 8; ++k) o[FT_REC + k] = rec[k];
         if (visc) {
             double vo[NGV], vn[NGV];
             ldRow(s.gv + (size_t)ow * NGV, vo);
@@ -519,7 +540,7 @@ __device__ __forceinline__ void faceTermsBody(const MeshView& m, const Phys& ph,
             o[FT_LAPE] = (alf * sne) * ms;
             const double rf = w * (fo[F_RHO] - fn[F_RHO]) + fn[F_RHO];
             const double lv = (muf + alf) / rf;
-            o[FT_SV] = 0.5 * lv * ms * m.dc[f];
+            if (ALL) o[FT_SV] = 0.5 * lv * ms * m.dc[f];
         }
     } else if (m.bKind[f - m.nI] == PK_CYCLIC) {
         // coupled interpolation of c and U (setCoAndDeltaT.H:44-56,78-89,
@@ -535,10 +556,11 @@ __device__ __forceinline__ void faceTermsBody(const MeshView& m, const Phys& ph,
         const V3 Un = pl ? V3{pf[PL_UV], pf[PL_UV + 1], pf[PL_UV + 2]} : rot3(m.cycR + 9 * (size_t)kc, cellU(s.fld, nc));
         const V3 Uf = w * cellU(s.fld, ow) + (1.0 - w) * Un;
         const double lam = cf + fabs(dot(Uf, S / ms) - um);
-        o[FT_LAM] = lam;
-        o[FT_FRDT] = m.nodc[f] * lam;
+        if (ALL) o[FT_LAM] = lam;
+        o[ftFrdt<MODE>()] = m.nodc[f] * lam;
+        if (ALL)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) o[FT_REC + k] = rec[k];
+            for (int k = 0; k < 8; ++k) o[FT_REC + k] = rec[k];
         if (visc) {
             // coupled viscous terms: every interpolation w v_P + (1 - w)
             // v_far with the far value through patchNeighbourField: U
@@ -579,7 +601,7 @@ __device__ __forceinline__ void faceTermsBody(const MeshView& m, const Phys& ph,
             const double rN = pl ? pf[F_RHO] : s.fld[(size_t)nc * NFLD + F_RHO];
             const double rf = w * s.fld[(size_t)ow * NFLD + F_RHO] + (1.0 - w) * rN;
             const double lv = (muf + alf) / rf;
-            o[FT_SV] = 0.5 * lv * ms * m.dc[f];
+            if (ALL) o[FT_SV] = 0.5 * lv * ms * m.dc[f];
         }
     } else {
         const int b = f - m.nI;
@@ -587,8 +609,8 @@ __device__ __forceinline__ void faceTermsBody(const MeshView& m, const Phys& ph,
         if (!(s.halt && *s.halt)) s.bcPhi[b] = fr;  // the registered phi the derived conditions read
         const double* bf = s.bfld + (size_t)b * NFLD;
         const V3 UB{bf[F_UX], bf[F_UY], bf[F_UZ]};
-        o[FT_LAM] = soundSpeed(ph, s.bT[b]) + fabs(dot(UB, S / ms) - um);
-        o[FT_FRDT] = m.bKind[b] == PK_WALL
+        if (ALL) o[FT_LAM] = soundSpeed(ph, s.bT[b]) + fabs(dot(UB, S / ms) - um);
+        o[ftFrdt<MODE>()] = m.bKind[b] == PK_WALL
                          ? 0.5 * m.nodc[f] * (soundSpeed(ph, s.T[c]) + fabs(dot(cellU(s.fld, c), S / ms) - um))
                          : -1.0;
         if (visc) {
@@ -618,37 +640,39 @@ __device__ __forceinline__ void faceTermsBody(const MeshView& m, const Phys& ph,
     }
 }
 
-// Face records of workgroup blk: assembled in LDS (row stride NFT + 1
+// Face records of workgroup blk: assembled in LDS (row stride the record + 1
 // doubles, zero where a face kind writes nothing, as the buffer holds from
 // its allocation), then stored as one contiguous range of whole records.
 // Each thread storing its own record directly issues NFT 8-byte stores at a
 // 192-byte stride across the wave, which reach memory as partial cache
 // lines, about twice the record bytes.
+template <int MODE>
 __device__ __forceinline__ void faceTermsBlock(const MeshView& m, const Phys& ph, const StateView& s, int blk) {
     extern __shared__ double shFT[];
+    constexpr int N = ftSize<MODE>();
     const int bs = blockDim.x;
     const int f0 = blk * bs;
-    double* o = shFT + (size_t)threadIdx.x * (NFT + 1);
+    double* o = shFT + (size_t)threadIdx.x * (N + 1);
 #pragma unroll
-    for (int k = 0; k < NFT; ++k) o[k] = 0.0;
+    for (int k = 0; k < N; ++k) o[k] = 0.0;
     const int f = f0 + threadIdx.x;
-    if (f < m.nF && !(f >= m.nI && m.bKind[f - m.nI] == PK_EMPTY)) faceTermsBody(m, ph, s, f, o);
+    if (f < m.nF && !(f >= m.nI && m.bKind[f - m.nI] == PK_EMPTY)) faceTermsBody<MODE>(m, ph, s, f, o);
     __syncthreads();
     const int nRec = min(bs, m.nF - f0);
-    double* g = s.ft + (size_t)f0 * NFT;
-    for (int i = threadIdx.x; i < nRec * NFT; i += bs) {
-        const int r = i / NFT, k = i - r * NFT;
-        stnt(g + i, shFT[r * (NFT + 1) + k]);
+    double* g = s.ft + (size_t)f0 * N;
+    for (int i = threadIdx.x; i < nRec * N; i += bs) {
+        const int r = i / N, k = i - r * N;
+        stnt(g + i, shFT[r * (N + 1) + k]);
     }
 }
 
-template <int W>
+template <int W, int MODE = FT_ALL>
 __global__ void __launch_bounds__(256, W) k_face_terms(MeshView m, Phys ph, StateView s) {
-    faceTermsBlock(m, ph, s, xcdBlock());
+    faceTermsBlock<MODE>(m, ph, s, xcdBlock());
 }
 __global__ void __launch_bounds__(256) k_face_terms_hb(const HBInst* __restrict__ I, Phys ph) {
     const HBInst q = I[blockIdx.y];
-    faceTermsBlock(q.m, ph, q.s, xcdBlock());
+    faceTermsBlock<FT_ALL>(q.m, ph, q.s, xcdBlock());
 }
 
 // Residual b = R*V (residualsUpdate.H) and rPseudoDeltaT
@@ -659,12 +683,14 @@ struct CellSums {
     double ar = 0, ae = 0;
     V3 au{0, 0, 0}, aLap{0, 0, 0}, aTau{0, 0, 0};
     double aSig = 0, aLapE = 0, rdt = 0.0;
+    template <int MODE = FT_ALL>
     __device__ __forceinline__ void add(const double* t, bool plus, bool visc) {
+        constexpr int FR = ftFrdt<MODE>();
         const double fr = t[FT_CONV], fe = t[FT_CONV + 1];
         const V3 fu{t[FT_CONV + 2], t[FT_CONV + 3], t[FT_CONV + 4]};
         if (plus) { ar += fr; ae += fe; au = au + fu; }
         else { ar -= fr; ae -= fe; au = au - fu; }
-        if (t[FT_FRDT] >= 0) rdt = fmax(rdt, t[FT_FRDT]);
+        if (t[FR] >= 0) rdt = fmax(rdt, t[FR]);
         if (visc) {
             const V3 lap{t[FT_LAP], t[FT_LAP + 1], t[FT_LAP + 2]};
             const V3 dt{t[FT_TAU], t[FT_TAU + 1], t[FT_TAU + 2]};
@@ -672,8 +698,9 @@ struct CellSums {
             else { aLap = aLap - lap; aTau = aTau - dt; aSig -= t[FT_SIG]; aLapE -= t[FT_LAPE]; }
         }
     }
-    // writes b and rDT of cell c; returns rDT
-    __device__ __forceinline__ double store(const MeshView& m, const StateView& s, int c, bool visc) const {
+    // writes b (to bOut too, when given) and rDT of cell c; returns rDT
+    __device__ __forceinline__ double store(const MeshView& m, const StateView& s, int c, bool visc,
+                                            double* __restrict__ bOut = nullptr) const {
         const double Vc = m.V[c];
         const int nC = m.nC;
         double Rr = -(ar / Vc);
@@ -700,32 +727,43 @@ struct CellSums {
             s.b[3 * (size_t)nC + c] -= sc.y;
             s.b[4 * (size_t)nC + c] -= sc.z;
         }
+        if (bOut)
+#pragma unroll
+            for (int q = 0; q < 5; ++q) bOut[(size_t)q * nC + c] = s.b[(size_t)q * nC + c];
         const double r = rdt / s.pseudoCo[c];
         s.rDT[c] = r;
         return r;
     }
 };
 
-__device__ __forceinline__ void cellResidualBody(const MeshView& m, const Phys& ph, const StateView& s) {
+// Cell sums over the face records, read as 128-bit rows: every lane's record
+// has its own cache lines, so the number of loads sets the time.
+template <int MODE>
+__device__ __forceinline__ void cellResidualBody(const MeshView& m, const Phys& ph, const StateView& s,
+                                                 double* bOut) {
     const int c = xcdBlock() * blockDim.x + threadIdx.x;
     if (c >= m.nC) return;
-    const bool visc = ph.viscous;
+    constexpr int N = ftSize<MODE>(), NL = N < 16 ? N : 16;
+    const bool visc = MODE != FT_INV && ph.viscous;
     const int e0 = m.cfOff[c], e1 = m.cfOff[c + 1];
     const int nLo = m.nLower[c];
     CellSums cs;
     for (int q = e0; q < e1; ++q) {
         const int f = m.cf[q];
-        cs.add(s.ft + (size_t)f * NFT, q - e0 >= nLo, visc);  // boundary and upper faces follow the lower faces
+        double t[NL];
+        ldRow(s.ft + (size_t)f * N, t);
+        cs.add<MODE>(t, q - e0 >= nLo, visc);  // boundary and upper faces follow the lower faces
     }
-    cs.store(m, s, c, visc);
+    cs.store(m, s, c, visc, bOut);
 }
 
-__global__ void __launch_bounds__(256) k_cell_residual(MeshView m, Phys ph, StateView s) {
-    cellResidualBody(m, ph, s);
+template <int MODE>
+__global__ void __launch_bounds__(256) k_cell_residual(MeshView m, Phys ph, StateView s, double* bOut) {
+    cellResidualBody<MODE>(m, ph, s, bOut);
 }
 __global__ void __launch_bounds__(256) k_cell_residual_hb(const HBInst* __restrict__ I, Phys ph) {
     const HBInst q = I[blockIdx.y];
-    cellResidualBody(q.m, ph, q.s);
+    cellResidualBody<FT_ALL>(q.m, ph, q.s, nullptr);
 }
 
 // Face fluxes of every face (convectiveFluxScheme::calcFlux output) from
@@ -1109,13 +1147,27 @@ void launchHBReconstruct(int nC, int nO, const HBInst* inst, const double* w, do
 static inline int nblk(int n, int b) { return (n + b - 1) / b; }
 
 void launchUpdate(const MeshView& m, const Phys& ph, const StateView& s, const double* dW, int mode,
-                  const double* rho0, const double* U0, const double* T0, hipStream_t st) {
-    k_update<<<nblk(m.nC, 256), 256, 0, st>>>(m, ph, s, dW, mode, rho0, U0, T0);
+                  const double* rho0, const double* U0, const double* T0, hipStream_t st, const double* Wsrc,
+                  double* W0) {
+    k_update<<<nblk(m.nC, 256), 256, 0, st>>>(m, ph, s, dW, mode, rho0, U0, T0, Wsrc, W0);
     // boundary conditions follow every state update (updateFields.H:90-105)
     if (m.nB > 0) k_bc_update<<<nblk(m.nB, 256), 256, 0, st>>>(m, ph, s, mode == 0 ? 1 : 0);
 }
 
-void launchResidual(const MeshView& m, const Phys& ph, const StateView& s, hipStream_t st, bool cellSums) {
+// The full face records.
+void launchFaceTerms(const MeshView& m, const Phys& ph, const StateView& s, hipStream_t st) {
+    const int bf = m.bsFace;
+    const dim3 gf(xcdGrid(m.nF, bf));
+    const size_t lds = (size_t)bf * (NFT + 1) * sizeof(double);
+    if (m.occFace == 1) k_face_terms<4><<<gf, bf, lds, st>>>(m, ph, s);
+    else if (m.occFace == 2) k_face_terms<3><<<gf, bf, lds, st>>>(m, ph, s);
+    else k_face_terms<1><<<gf, bf, lds, st>>>(m, ph, s);
+}
+
+// bOut (a residual evaluation alone): short face records, b to bOut as well.
+// 104x96x96 viscous Roe: face terms 345 -> 309 us, cell sums 233 -> 144 us.
+void launchResidual(const MeshView& m, const Phys& ph, const StateView& s, hipStream_t st, bool cellSums,
+                    double* bOut) {
     if (m.nB > 0) k_boundary<<<nblk(m.nB, 256), 256, 0, st>>>(m, ph, s);
     const int bc = m.bsCell, bf = m.bsFace;
     const dim3 gc(xcdGrid(m.nC, bc)), gf(xcdGrid(m.nF, bf));
@@ -1130,11 +1182,16 @@ void launchResidual(const MeshView& m, const Phys& ph, const StateView& s, hipSt
         else if (m.occCell == 2) k_grad<8, 3><<<gc, bc, 0, st>>>(m, ph, s, nullptr, nullptr);
         else k_grad<8><<<gc, bc, 0, st>>>(m, ph, s, nullptr, nullptr);
     }
-    const size_t lds = (size_t)bf * (NFT + 1) * sizeof(double);
-    if (m.occFace == 1) k_face_terms<4><<<gf, bf, lds, st>>>(m, ph, s);
-    else if (m.occFace == 2) k_face_terms<3><<<gf, bf, lds, st>>>(m, ph, s);
-    else k_face_terms<1><<<gf, bf, lds, st>>>(m, ph, s);
-    if (cellSums) k_cell_residual<<<gc, bc, 0, st>>>(m, ph, s);
+    if (bOut && ph.viscous) {
+        k_face_terms<1, FT_VISC><<<gf, bf, (size_t)bf * (ftSize<FT_VISC>() + 1) * sizeof(double), st>>>(m, ph, s);
+        k_cell_residual<FT_VISC><<<gc, bc, 0, st>>>(m, ph, s, bOut);
+    } else if (bOut) {
+        k_face_terms<1, FT_INV><<<gf, bf, (size_t)bf * (ftSize<FT_INV>() + 1) * sizeof(double), st>>>(m, ph, s);
+        k_cell_residual<FT_INV><<<gc, bc, 0, st>>>(m, ph, s, bOut);
+    } else {
+        launchFaceTerms(m, ph, s, st);
+        if (cellSums) k_cell_residual<FT_ALL><<<gc, bc, 0, st>>>(m, ph, s, nullptr);
+    }
 }
 
 void launchResidualHB(const HBInst* inst, int nO, const MeshView& m, const Phys& ph, hipStream_t st,

@@ -208,6 +208,7 @@ struct icsf_case {
     int nPseudoCorr = 20, nPseudoCorrMin = 1;
     int blkFp32 = 0;
     bool haveResidual = false, assembled = false, haveFields = false;
+    bool shortFaces = false;  // the face records are a residual evaluation's short ones
     // Krylov work (FP64)
     double *V = nullptr, *r = nullptr, *t1 = nullptr, *t2 = nullptr, *dW = nullptr, *Z = nullptr;
     double* dres = nullptr;  // [2][5] init / previous initial residuals
@@ -596,12 +597,14 @@ int uploadBC(icsf_case* c) {
 
 // cellSums false (pseudo-step): the residual's cell sums are left to
 // jacobianStage(c, true), which forms them in the Jacobian's face walk.
-int residualStage(icsf_case* c, bool cellSums = true) {
+// bOut: b goes there as well (launchResidual).
+int residualStage(icsf_case* c, bool cellSums = true, double* bOut = nullptr) {
     RC(uploadBC(c));
     {
         Timed t(c, TK_RESIDUAL);
-        launchResidual(c->mv, c->ph, c->sv, c->st, cellSums);
+        launchResidual(c->mv, c->ph, c->sv, c->st, cellSums, bOut);
     }
+    c->shortFaces = bOut != nullptr;
     // without the cell sums b and rDT are complete only after
     // jacobianStage(c, true)
     c->haveResidual = cellSums;
@@ -611,6 +614,8 @@ int residualStage(icsf_case* c, bool cellSums = true) {
 int jacobianStage(icsf_case* c, bool cellSums = false) {
     {
         Timed t(c, TK_JACOBIAN);
+        if (c->shortFaces) launchFaceTerms(c->mv, c->ph, c->sv, c->st);
+        c->shortFaces = false;
         if (cellSums) launchCellSumsJacobian(c->mv, c->ph, c->sv, c->blk, c->dg, c->blkFp32, c->rD, c->derr, c->st);
         else launchJacobian(c->mv, c->ph, c->sv, c->blk, c->dg, c->blkFp32, c->rD, c->derr, c->st);
     }
@@ -951,12 +956,10 @@ int adjointPrepare(icsf_case* c) {
 
 // State from W (device, or the current W when NULL) through updateFields
 // with a zero increment; W is kept in adj.W0.
-int stateFromW(icsf_case* c, const double* W) {
+int stateFromW(icsf_case* c, const double* W, bool keep = true) {
     const size_t n5 = 5 * (size_t)c->mv.nC;
-    if (!c->adj.W0) RC(c->buf.alloc(c->adj.W0, n5));
-    if (W) HIPCHK(hipMemcpyAsync(c->sv.W, W, n5 * sizeof(double), hipMemcpyDeviceToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->adj.W0, c->sv.W, n5 * sizeof(double), hipMemcpyDeviceToDevice, c->st));
-    launchUpdate(c->mv, c->ph, c->sv, nullptr, 1, nullptr, nullptr, nullptr, c->st);
+    if (keep && !c->adj.W0) RC(c->buf.alloc(c->adj.W0, n5));
+    launchUpdate(c->mv, c->ph, c->sv, nullptr, 1, nullptr, nullptr, nullptr, c->st, W, keep ? c->adj.W0 : nullptr);
     c->haveFields = true;
     c->haveResidual = c->assembled = false;
     return ICSF_OK;
@@ -2270,10 +2273,7 @@ int icsf_residual_vjp_device_noalloc(icsf_case* c, const double* W, const double
     sc = ScratchCarve{base, 0};
     carve(a, gS, gC);
     RC(uploadBC(c));
-    const size_t n5 = 5 * nC;
-    if (W) HIPCHK(hipMemcpyAsync(c->sv.W, W, n5 * sizeof(double), hipMemcpyDeviceToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(a.W0, c->sv.W, n5 * sizeof(double), hipMemcpyDeviceToDevice, c->st));
-    launchUpdate(c->mv, c->ph, c->sv, nullptr, 1, nullptr, nullptr, nullptr, c->st);
+    launchUpdate(c->mv, c->ph, c->sv, nullptr, 1, nullptr, nullptr, nullptr, c->st, W, a.W0);
     c->haveFields = true;
     c->haveResidual = c->assembled = false;
     launchAdjointForward(c->mv, c->ph, c->sv, a.gun, a.lim, c->st);
@@ -2287,9 +2287,8 @@ int icsf_residual_device(icsf_case* c, const double* W, double* b) {
     if (!c || !b) return fail(ICSF_ERR_ARG, "icsf_residual_device: NULL argument");
     if (!W && !c->haveFields) return fail(ICSF_ERR_STATE, "fields not set");
     RC(uploadBC(c));
-    RC(stateFromW(c, W));
-    RC(residualStage(c));
-    HIPCHK(hipMemcpyAsync(b, c->sv.b, 5 * (size_t)c->mv.nC * sizeof(double), hipMemcpyDeviceToDevice, c->st));
+    RC(stateFromW(c, W, false));
+    RC(residualStage(c, true, b));
     HIPCHK(hipStreamSynchronize(c->st));
     return takeDeviceErrors(c->st, {c->derr});
 }
