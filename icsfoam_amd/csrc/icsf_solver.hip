@@ -140,6 +140,9 @@ struct icsf_mesh {
 
 // ------------------------------------------------------------------ case --
 enum { NTIMER = 6 };
+// pseudo-steps whose residuals are collected in pinned memory before the host
+// waits for them
+constexpr int kResBatch = 32;
 
 // One frame zone's contribution (rotating or translating): faceU & Sf/|Sf|
 // per face, the moving boundary faces and their U.
@@ -199,6 +202,8 @@ struct icsf_case {
     void *blk = nullptr, *dg = nullptr, *dinv = nullptr;
     double* rD = nullptr;
     int* derr = nullptr;
+    int* hErr = nullptr;  // pinned: the error flags as read back by caseErrors
+    double* hRes = nullptr;  // pinned: the residuals of up to kResBatch steps
     // pseudo-time loop control (pseudotimeControl): device block [NCTL],
     // stored initial residuals [5]; criteria from fvSolution pseudoTime
     // (pseudoTol / pseudoTolRel NaN when absent)
@@ -244,6 +249,8 @@ struct icsf_case {
         for (auto& e : open)
             if (e) (void)hipEventDestroy(e);
         if (st && ownStream) (void)hipStreamDestroy(st);
+        if (hErr) (void)hipHostFree(hErr);
+        if (hRes) (void)hipHostFree(hRes);
     }
 };
 
@@ -311,6 +318,36 @@ __global__ void k_ser(int nC, double* co, const double* dres, double coIncr, dou
     double v = co[c] * ratio;
     v = fmax(fmin(v, coMax), coMin);
     co[c] = v;
+}
+
+// Up to HB_MAXO instances' residuals (10 each) into pinned host memory, and
+// their error flags cleared or read back (the last one the coupled system's).
+struct ResPtrs {
+    const double* r[HB_MAXO];
+};
+__global__ void k_store_residuals(ResPtrs q, int n, double* host) {
+    const int i = threadIdx.x;
+    if (i < 10 * n) host[i] = q.r[i / 10][i % 10];
+}
+struct FlagPtrs {
+    int* p[HB_MAXO + 1];
+    int n;
+};
+__global__ void k_flags(FlagPtrs q, int* host) {
+    const int i = threadIdx.x;
+    if (i >= q.n) return;
+    if (host) host[i] = *q.p[i];
+    else *q.p[i] = 0;
+}
+
+// rho [nC], p [nC] and U [nC][3] out of the field rows
+__global__ void k_pack_fields(int nC, const double* fld, double* q) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= nC) return;
+    const double* f = fld + (size_t)c * NFLD;
+    q[c] = f[F_RHO];
+    q[(size_t)nC + c] = f[F_P];
+    for (int d = 0; d < 3; ++d) q[2 * (size_t)nC + 3 * (size_t)c + d] = f[F_UX + d];
 }
 
 __global__ void k_copy5(const double* a, double* b) {
@@ -429,24 +466,23 @@ __global__ void k_fill(int n, double v, double* x) {
 
 int nblk(size_t n, int b) { return (int)((n + b - 1) / b); }
 
-// Read the device error flags of the given flag words (after the work on
-// `st`), clear them, and turn them into a return code: a non-finite state
-// first, then a diagonal whose LU-SGS coefficient fell below VSMALL
-// (lusgs.C:119-123).
-int takeDeviceErrors(hipStream_t st, const std::vector<int*>& flags) {
-    int any = 0;
-    for (int* f : flags) {
-        if (!f) continue;
-        int e = 0;
-        HIPCHK(hipMemcpyAsync(&e, f, sizeof(int), hipMemcpyDeviceToHost, st));
-        HIPCHK(hipStreamSynchronize(st));
-        if (e) HIPCHK(hipMemset(f, 0, sizeof(int)));
-        any |= e;
-    }
+// Device error flags as a return code: a non-finite state first, then a
+// diagonal whose LU-SGS coefficient fell below VSMALL (lusgs.C:119-123).
+int flagError(int any) {
     if (any & ERR_FLAG_NONFINITE) return fail(ICSF_ERR_NONFINITE, "non-finite conserved state after the update");
     if (any & ERR_FLAG_SWEEP) return fail(ICSF_ERR_HIP, "LU-SGS sweep: a wait ended at its limit");
     if (any & ERR_FLAG_DIAG) return fail(ICSF_ERR_ZERO_DIAG, "All diagonals of coupledMatrix are zero.");
     return ICSF_OK;
+}
+
+// Waits for the case's stream and reports its error flags: the flags follow
+// the queued work into pinned memory, so that a call waits once.
+int caseErrors(icsf_case* c) {
+    HIPCHK(hipMemcpyAsync(c->hErr, c->derr, sizeof(int), hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipStreamSynchronize(c->st));
+    const int e = *c->hErr;
+    if (e) HIPCHK(hipMemset(c->derr, 0, sizeof(int)));
+    return flagError(e);
 }
 
 // ---- settings -----------------------------------------------------------
@@ -973,8 +1009,7 @@ int vjpDevice(icsf_case* c, const double* W, const double* v, double* gW, double
     launchAdjointForward(c->mv, c->ph, c->sv, c->adj.gun, c->adj.lim, c->st);
     launchResidualVjp(c->mv, c->ph, c->sv, c->adj, v, gW, gSf ? gSf : c->adjGS, gCf ? gCf : c->adjGC, geom, c->st);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(c->st));
-    return takeDeviceErrors(c->st, {c->derr});
+    return caseErrors(c);
 }
 
 }  // namespace
@@ -1002,6 +1037,8 @@ struct icsf_hb {
     float *r32 = nullptr, *r32b = nullptr, *V32 = nullptr;
     GmresScalars* g2 = nullptr;
     int* derr = nullptr;
+    int* hErr = nullptr;     // pinned, as icsf_case's
+    double* hRes = nullptr;  // pinned: [kResBatch][nO][10]
     HBInst* dInst = nullptr;  // per-instance views, blockIdx.y of the batched launches
     GmresScalars* g = nullptr;
     std::vector<GmresScalars*> gJ;
@@ -1029,6 +1066,8 @@ struct icsf_hb {
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (graph) (void)hipGraphDestroy(graph);
         for (icsf_case* c : inst) delete c;
+        if (hErr) (void)hipHostFree(hErr);
+        if (hRes) (void)hipHostFree(hRes);
         if (st) (void)hipStreamDestroy(st);
     }
 };
@@ -1188,10 +1227,17 @@ int hbJacobianStage(icsf_hb* h, bool cellSums = false) {
     return ICSF_OK;
 }
 
+// the instances' residuals into host (pinned, [nO][10]) after the queued work
+void hbQueueResiduals(icsf_hb* h, double* host) {
+    ResPtrs q{};
+    for (int J = 0; J < h->nO; ++J) q.r[J] = gmresResidualsDevice(h->gJ[J]);
+    k_store_residuals<<<1, 10 * HB_MAXO, 0, h->st>>>(q, h->nO, host);
+}
+
 void hbReadResiduals(icsf_hb* h, std::vector<double>& res) {
-    res.assign(10 * (size_t)h->nO, 0.0);
+    hbQueueResiduals(h, h->hRes);
     (void)hipStreamSynchronize(h->st);
-    for (int J = 0; J < h->nO; ++J) gmresReadResiduals(h->gJ[J], &res[10 * (size_t)J], h->st);
+    res.assign(h->hRes, h->hRes + 10 * (size_t)h->nO);
 }
 
 // gmres::solveDelta on the HB system (left LU-SGS, reference algorithm)
@@ -1745,6 +1791,8 @@ int createCase(icsf_mesh* mesh, const char* thermo, const char* schemes, const c
     RC(B.alloc(C->derr, 1));
     HIPCHK(hipMemset(C->derr, 0, sizeof(int)));
     C->sv.err = C->derr;
+    HIPCHK(hipHostMalloc((void**)&C->hErr, sizeof(int), hipHostMallocDefault));
+    HIPCHK(hipHostMalloc((void**)&C->hRes, kResBatch * 10 * sizeof(double), hipHostMallocDefault));
     RC(B.alloc(C->dctl, NCTL));
     RC(B.alloc(C->dctlInit, 5));
     {
@@ -2097,17 +2145,22 @@ int icsf_set_fields(icsf_case* c, const double* rho, const double* U, const doub
 
 int icsf_get_fields(icsf_case* c, double* rho, double* U, double* T, double* p, double* W) {
     if (!c) return fail(ICSF_ERR_ARG, "NULL case");
-    const int nC = c->mv.nC;
-    HIPCHK(hipStreamSynchronize(c->st));
-    std::vector<double> fld((size_t)NFLD * nC);
-    HIPCHK(hipMemcpy(fld.data(), c->sv.fld, fld.size() * sizeof(double), hipMemcpyDeviceToHost));
-    if (rho) for (int i = 0; i < nC; ++i) rho[i] = fld[(size_t)i * NFLD + F_RHO];
-    if (p) for (int i = 0; i < nC; ++i) p[i] = fld[(size_t)i * NFLD + F_P];
-    if (U)
-        for (int i = 0; i < nC; ++i)
-            for (int d = 0; d < 3; ++d) U[3 * i + d] = fld[(size_t)i * NFLD + F_UX + d];
-    if (T) HIPCHK(hipMemcpy(T, c->sv.T, (size_t)nC * sizeof(double), hipMemcpyDeviceToHost));
-    if (W) HIPCHK(hipMemcpy(W, c->sv.W, (size_t)5 * nC * sizeof(double), hipMemcpyDeviceToHost));
+    const size_t nC = c->mv.nC;
+    if (rho || p || U) {
+        // the asked-for entries of the field rows, gathered on the device
+        // (a work vector of the case, else a temporary one)
+        DevBuf tmp;
+        double* q = c->t1;
+        if (!q) RC(tmp.alloc(q, 5 * nC));
+        k_pack_fields<<<nblk((int)nC, 256), 256, 0, c->st>>>((int)nC, c->sv.fld, q);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipStreamSynchronize(c->st));
+        if (rho) HIPCHK(hipMemcpy(rho, q, nC * sizeof(double), hipMemcpyDeviceToHost));
+        if (p) HIPCHK(hipMemcpy(p, q + nC, nC * sizeof(double), hipMemcpyDeviceToHost));
+        if (U) HIPCHK(hipMemcpy(U, q + 2 * nC, 3 * nC * sizeof(double), hipMemcpyDeviceToHost));
+    } else HIPCHK(hipStreamSynchronize(c->st));
+    if (T) HIPCHK(hipMemcpy(T, c->sv.T, nC * sizeof(double), hipMemcpyDeviceToHost));
+    if (W) HIPCHK(hipMemcpy(W, c->sv.W, 5 * nC * sizeof(double), hipMemcpyDeviceToHost));
     return ICSF_OK;
 }
 
@@ -2182,8 +2235,7 @@ int icsf_set_state(icsf_case* c, const double* W) {
     RC(tmp.upload(dW, W, n5));
     RC(uploadBC(c));
     RC(stateFromW(c, dW));
-    HIPCHK(hipStreamSynchronize(c->st));
-    return takeDeviceErrors(c->st, {c->derr});
+    return caseErrors(c);
 }
 
 int icsf_get_boundary_values(icsf_case* c, double* p, double* U, double* T) {
@@ -2223,9 +2275,8 @@ int icsf_residual_records_device(icsf_case* c, const double* W, int* faceBranche
     HIPCHK(hipMemcpyAsync(limiterElement, a.tgt, nC * NFLD * sizeof(int), hipMemcpyDeviceToDevice, c->st));
     HIPCHK(hipMemcpyAsync(limiterFace, a.fst, nC * NFLD * sizeof(int), hipMemcpyDeviceToDevice, c->st));
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(c->st));
     (void)nF;
-    return takeDeviceErrors(c->st, {c->derr});
+    return caseErrors(c);
 }
 
 int icsf_residual_vjp_device_noalloc(icsf_case* c, const double* W, const double* v, double* gW, double* gSf,
@@ -2279,8 +2330,7 @@ int icsf_residual_vjp_device_noalloc(icsf_case* c, const double* W, const double
     launchAdjointForward(c->mv, c->ph, c->sv, a.gun, a.lim, c->st);
     launchResidualVjp(c->mv, c->ph, c->sv, a, v, gW, gSf ? gSf : gS, gCf ? gCf : gC, gSf || gCf, c->st);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(c->st));
-    return takeDeviceErrors(c->st, {c->derr});
+    return caseErrors(c);
 }
 
 int icsf_residual_device(icsf_case* c, const double* W, double* b) {
@@ -2289,15 +2339,14 @@ int icsf_residual_device(icsf_case* c, const double* W, double* b) {
     RC(uploadBC(c));
     RC(stateFromW(c, W, false));
     RC(residualStage(c, true, b));
-    HIPCHK(hipStreamSynchronize(c->st));
-    return takeDeviceErrors(c->st, {c->derr});
+    return caseErrors(c);
 }
 
 int icsf_assemble_jacobian(icsf_case* c) {
     if (!c) return fail(ICSF_ERR_ARG, "NULL case");
     if (!c->haveResidual) return fail(ICSF_ERR_STATE, "icsf_residual must run before the Jacobian assembly");
     RC(jacobianStage(c));
-    return takeDeviceErrors(c->st, {c->derr});
+    return caseErrors(c);
 }
 
 int icsf_get_jacobian(icsf_case* c, double* diag, double* upper, double* lower) {
@@ -2449,8 +2498,7 @@ int icsf_precondition(icsf_case* c, double* r) {
     HIPCHK(hipMemcpyAsync(c->t1, r, vs * 8, hipMemcpyHostToDevice, c->st));
     applyPrecond(c, 0, c->t1);
     HIPCHK(hipMemcpyAsync(r, c->t1, vs * 8, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
-    return takeDeviceErrors(c->st, {c->derr});
+    return caseErrors(c);
 }
 
 int icsf_solve_for_incr(icsf_case* c, const double* W, const double* b, double* dW, double* residuals,
@@ -2485,17 +2533,25 @@ int icsf_pseudo_steps(icsf_case* c, int nSteps, double* residuals, int* nIter) {
     if (!c->haveFields) return fail(ICSF_ERR_STATE, "fields not set");
     // flags left by earlier calls (e.g. a state handed to the VJP) do not
     // belong to these steps
-    HIPCHK(hipStreamSynchronize(c->st));
-    HIPCHK(hipMemset(c->derr, 0, sizeof(int)));
+    k_flags<<<1, 64, 0, c->st>>>(FlagPtrs{{c->derr}, 1}, nullptr);
     for (int i = 0; i < nSteps; ++i) {
         int it = 1;
         if (graphable(c)) RC(graphStep(c));
         else RC(pseudoStep(c, it));
-        if (residuals) gmresReadResiduals(c->g, residuals + 10 * (size_t)i, c->st);
+        if (residuals) {
+            // collected without a wait per step, so that the steps follow
+            // each other on the device
+            const int k = i % kResBatch;
+            k_store_residuals<<<1, 64, 0, c->st>>>(ResPtrs{{gmresResidualsDevice(c->g)}}, 1, c->hRes + 10 * k);
+            if (k == kResBatch - 1 || i == nSteps - 1) {
+                HIPCHK(hipStreamSynchronize(c->st));
+                std::copy(c->hRes, c->hRes + 10 * (k + 1), residuals + 10 * (size_t)(i - k));
+            }
+        }
         if (nIter) nIter[i] = it;
     }
     HIPCHK(hipGetLastError());
-    const int rc = takeDeviceErrors(c->st, {c->derr});
+    const int rc = caseErrors(c);
     resolveEvents(c);
     return rc;
 }
@@ -2546,7 +2602,7 @@ int icsf_pseudo_time_loop(icsf_case* c, int maxSteps, int batch, int* stepsRun, 
     if (converged) *converged = conv ? 1 : 0;
     if (rc) return rc;
     HIPCHK(hipGetLastError());
-    rc = takeDeviceErrors(c->st, {c->derr});
+    rc = caseErrors(c);
     resolveEvents(c);
     return rc;
 }
@@ -2691,6 +2747,9 @@ int icsf_hb_create(icsf_mesh* mesh, const char* thermo, const char* schemes, con
     RC(B.alloc(H->dres, 10 * (size_t)HB_MAXO));
     RC(B.alloc(H->derr, 1));
     HIPCHK(hipMemset(H->derr, 0, sizeof(int)));
+    HIPCHK(hipHostMalloc((void**)&H->hErr, (HB_MAXO + 1) * sizeof(int), hipHostMallocDefault));
+    HIPCHK(hipHostMalloc((void**)&H->hRes, (size_t)kResBatch * nInstants * 10 * sizeof(double),
+                         hipHostMallocDefault));
     RC(B.alloc(H->wk.part, kPartSize));
     {
         char* p;
@@ -2864,12 +2923,25 @@ int icsf_hb_get_fields(icsf_hb* h, int instant, double* rho, double* U, double* 
 }
 
 // error flags of the coupled diagonal and of every instance
-static std::vector<int*> hbErrorFlags(const icsf_hb* h) {
-    std::vector<int*> f{h->derr};
-    for (icsf_case* c : h->inst) f.push_back(c->derr);
-    return f;
+static FlagPtrs hbFlagPtrs(const icsf_hb* h) {
+    FlagPtrs q{};
+    for (icsf_case* c : h->inst) q.p[q.n++] = c->derr;
+    q.p[q.n++] = h->derr;
+    return q;
 }
-
+// As caseErrors, for the coupled system and every instance.
+static int hbErrors(icsf_hb* h) {
+    const FlagPtrs q = hbFlagPtrs(h);
+    k_flags<<<1, 64, 0, h->st>>>(q, h->hErr);
+    HIPCHK(hipStreamSynchronize(h->st));
+    int any = 0;
+    for (int i = 0; i < q.n; ++i) any |= h->hErr[i];
+    if (any) {
+        k_flags<<<1, 64, 0, h->st>>>(q, nullptr);
+        HIPCHK(hipStreamSynchronize(h->st));
+    }
+    return flagError(any);
+}
 static int hbReady(icsf_hb* h) {
     if (!h) return fail(ICSF_ERR_ARG, "NULL HB case");
     for (icsf_case* c : h->inst)
@@ -2892,7 +2964,7 @@ int icsf_hb_assemble_jacobian(icsf_hb* h) {
     for (icsf_case* c : h->inst)
         if (!c->haveResidual) return fail(ICSF_ERR_STATE, "icsf_hb_residual must run before the Jacobian assembly");
     RC(hbJacobianStage(h));
-    return takeDeviceErrors(h->st, hbErrorFlags(h));
+    return hbErrors(h);
 }
 
 int icsf_hb_matrix_mul(icsf_hb* h, const double* x, double* y) {
@@ -2940,20 +3012,26 @@ int icsf_hb_solve_for_incr(icsf_hb* h, const double* b, double* dW, double* resi
 int icsf_hb_pseudo_steps(icsf_hb* h, int nSteps, double* residuals) {
     RC(hbReady(h));
     if (nSteps < 0) return fail(ICSF_ERR_ARG, "icsf_hb_pseudo_steps: nSteps < 0");
-    HIPCHK(hipStreamSynchronize(h->st));
-    HIPCHK(hipMemset(h->derr, 0, sizeof(int)));
-    for (icsf_case* c : h->inst) HIPCHK(hipMemset(c->derr, 0, sizeof(int)));
+    const FlagPtrs flags = hbFlagPtrs(h);
+    k_flags<<<1, 64, 0, h->st>>>(flags, nullptr);
+    const size_t nr = (size_t)10 * h->nO;
+    // one step's residuals may be in use by the solver's own stop test
+    // (maxIter > 1, hbReadResiduals): those steps are read one by one
+    const int batch = h->maxIter == 1 && h->minIter <= 1 ? kResBatch : 1;
     for (int i = 0; i < nSteps; ++i) {
         if (hbGraphable(h)) RC(hbGraphStep(h));
         else RC(hbPseudoStep(h));
         if (residuals) {
-            std::vector<double> res;
-            hbReadResiduals(h, res);
-            std::copy(res.begin(), res.end(), residuals + (size_t)i * 10 * h->nO);
+            const int k = i % batch;
+            hbQueueResiduals(h, h->hRes + k * nr);
+            if (k == batch - 1 || i == nSteps - 1) {
+                HIPCHK(hipStreamSynchronize(h->st));
+                std::copy(h->hRes, h->hRes + (k + 1) * nr, residuals + (size_t)(i - k) * nr);
+            }
         }
     }
     HIPCHK(hipGetLastError());
-    return takeDeviceErrors(h->st, hbErrorFlags(h));
+    return hbErrors(h);
 }
 
 int icsf_hb_synchronize(icsf_hb* h) {

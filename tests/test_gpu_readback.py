@@ -1,0 +1,59 @@
+"""Residual histories longer than one batch of the pinned collection buffer
+(32 steps): the same bits as steps asked for one at a time, for a single case
+and for harmonic balance with one and with several solver cycles; and field
+read-backs of any subset."""
+import ctypes
+import dataclasses
+
+import numpy as np
+import pytest
+
+from icsfoam_amd import cases, dbnsCase
+from icsfoam_amd._lib import check, lib, ptr
+from icsfoam_amd.mesh import prepare_case
+from icsfoam_amd.solver import hbCase
+
+from helpers import bump_small
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 70])
+def test_history_batches(n):
+    print(f"[history {n}]", flush=True)
+    c = bump_small(16, 8)
+    a, b = dbnsCase.from_case(c), dbnsCase.from_case(c)
+    h = a.pseudo_steps(n)
+    one = np.concatenate([b.pseudo_steps(1) for _ in range(n)])
+    np.testing.assert_array_equal(h, one)
+
+
+@pytest.mark.parametrize("max_iter", [1, 2])
+def test_hb_history_batches(max_iter):
+    print(f"[hb history {max_iter}]", flush=True)
+    insts, D, _ = cases.case_hb(n=(6, 4, 3), n_harmonics=1)
+    insts = [dataclasses.replace(prepare_case(c, permute_seed=1), fvSolution=cases.solution_dict(
+        co=20.0, nDirections=4, maxIter=max_iter, relTol=1e-6)) for c in insts]
+    a, b = hbCase.from_cases(insts, D), hbCase.from_cases(insts, D)
+    h = a.pseudo_steps(35)
+    one = np.concatenate([b.pseudo_steps(1) for _ in range(35)])
+    np.testing.assert_array_equal(h, one)
+    F = a.fields(1)
+    np.testing.assert_array_equal(F["W"][0], F["rho"])
+
+
+def test_field_subsets():
+    c = bump_small(20, 7)
+    g = dbnsCase.from_case(c)
+    g.pseudo_steps(2)
+    full = g.fields()
+    n = g.nCells
+    np.testing.assert_array_equal(full["W"][0], full["rho"])
+    np.testing.assert_allclose(full["W"][2:].T, full["rho"][:, None] * full["U"], rtol=1e-15)
+    for mask in range(1, 32):
+        out = [np.empty(n), np.empty((n, 3)), np.empty(n), np.empty(n), np.empty((5, n))]
+        arg = [ptr(x) if mask >> i & 1 else None for i, x in enumerate(out)]
+        check(lib().icsf_get_fields(g._h, *arg))
+        for i, k in enumerate(("rho", "U", "T", "p", "W")):
+            if mask >> i & 1:
+                np.testing.assert_array_equal(out[i], full[k])
