@@ -49,8 +49,17 @@ struct Work {
     int *swDone = nullptr, *err = nullptr;
 };
 
-// 1024 workgroups' partials of the 2 KMAX projection values of one step
-constexpr size_t kPartSize = (size_t)1024 * 2 * KMAX;
+// 1024 workgroups' partials of the 2 KMAX projection values of one step, then
+// those of a norm (from kNormPart)
+constexpr size_t kNormPart = (size_t)1024 * 2 * KMAX, kPartSize = kNormPart + 1024;
+
+// A norm still in partials: nb sums of squares at part; whoever reduces them
+// stores the norm at beta and hn.
+struct NormIn {
+    const double* part = nullptr;
+    int nb = 0;
+    double *beta = nullptr, *hn = nullptr;
+};
 
 struct GmresScalars;
 
@@ -83,9 +92,9 @@ struct GmresArgs {
     // fuse the Arnoldi SpMV with the LU-SGS sweeps when the level structure
     // allows it (same algorithm; a row's terms summed in another order)
     bool fuse = false;
-    // batched systems: fused operator + preconditioner (returns false when
-    // not applicable; op and pre are then used)
-    std::function<bool(const void*, const double*, void*, void*)> opPre;
+    // batched systems: fused operator + preconditioner on x / norm (empty: op
+    // and pre are used)
+    std::function<void(const void*, const NormIn&, void*, void*)> opPre;
 };
 
 // Harmonic balance, one launch per stage for all instances
@@ -195,11 +204,16 @@ void launchSpmv(const MeshView& m, int blkFp32, int vecFp32, const void* blk, co
                 const double* scal, void* vout, void* y, hipStream_t st);
 void launchLusgs(const MeshView& m, const Levels& L, const Work& wk, int blkFp32, int vecFp32, const void* blk,
                  const double* rD, void* r, hipStream_t st);
+// Whether the fused operator applies: two-colour levels, blocks and vectors of
+// one precision.
+inline bool fusedOperator(const Levels& L, int blkFp32, int vecFp32) { return L.twoColour && blkFp32 == vecFp32; }
 // y = LU-SGS(A (x/scal)) in three passes on a two-colour level structure, t
-// a work vector (false: not applicable, nothing launched).
+// a work vector (false: not applicable, nothing launched).  norm.part: the
+// scale is that norm, reduced in the first pass; scal is then where it stores
+// it (norm.beta).
 bool launchSpmvLusgs(const MeshView& m, const Levels& L, int blkFp32, int vecFp32, const void* blk, const void* dg,
-                     const double* rD, const void* x, const double* scal, void* vout, void* t, void* y,
-                     hipStream_t st);
+                     const double* rD, const void* x, const double* scal, const NormIn& norm, void* vout, void* t,
+                     void* y, hipStream_t st);
 void launchJacobiSetup(int nC, int blkFp32, const void* dg, void* dinv, hipStream_t st);
 void launchJacobiApply(int nC, int blkFp32, int vecFp32, const void* dinv, void* r, hipStream_t st);
 
@@ -228,7 +242,8 @@ void launchSpmvHB(const MeshView& m, const HBBlocks& hb, int vecFp32, const void
 // y = LU-SGS(A_HB (x/scal)) in three passes on a two-colour level
 // structure, t a work vector (false: not applicable, nothing launched).
 bool launchSpmvLusgsHB(const MeshView& m, const Levels& L, const HBBlocks& hb, int vecFp32, const double* rD,
-                       const void* x, const double* scal, void* vout, void* t, void* y, hipStream_t st);
+                       const void* x, const double* scal, const NormIn& norm, void* vout, void* t, void* y,
+                       hipStream_t st);
 // LU-SGS of all HB instances (per-instance sweeps, shared diagonal rD).
 void launchLusgsHB(const MeshView& m, const Levels& L, const HBBlocks& hb, int vecFp32, const double* rD, void* r,
                    hipStream_t st);

@@ -19,6 +19,52 @@ namespace icsf {
 
 namespace {
 
+// ---------------------------------------------------------- reductions ----
+__device__ __forceinline__ double waveSum(double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
+    return v;
+}
+
+// Wave sums of NA values per lane (NA a power of two up to 64): every lane
+// keeps half of its values and hands the other half to its partner, so the
+// values thin out as the lanes combine: 17 exchanges for 16 values instead of
+// 96.  Lane `lane` returns the sum of value `id` (the lanes of one value all
+// hold it); the pairs added are those of waveSum, whatever NA.
+template <int HALF, int D, int NA>
+__device__ __forceinline__ void waveFold(double (&v)[NA], int lane, int& id) {
+    if constexpr (HALF >= 1) {
+        const bool hi = lane & D;
+#pragma unroll
+        for (int k = 0; k < HALF; ++k) {
+            const double give = hi ? v[k] : v[k + HALF], keep = hi ? v[k + HALF] : v[k];
+            v[k] = keep + __shfl_xor(give, D, 64);
+        }
+        if (hi) id += HALF;
+        waveFold<HALF / 2, D / 2>(v, lane, id);
+    } else if constexpr (D >= 1) {
+        v[0] += __shfl_xor(v[0], D, 64);
+        waveFold<0, D / 2>(v, lane, id);
+    }
+}
+template <int NA>
+__device__ __forceinline__ double waveSums(double (&v)[NA], int lane, int& id) {
+    id = 0;
+    waveFold<NA / 2, 32>(v, lane, id);
+    return v[0];
+}
+
+// The norm whose partials (nb of them) are at part, by one wavefront; every
+// lane returns it.
+__device__ __forceinline__ double waveNorm(const double* __restrict__ part, int nb) {
+    const int lane = threadIdx.x & 63;
+    double v = 0;
+    for (int b = lane; b < nb; b += 64) v += part[b];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return sqrt(v);
+}
+
 template <typename T>
 __device__ __forceinline__ double ld(const T* p, size_t i) { return (double)p[i]; }
 
@@ -359,8 +405,29 @@ __global__ void __launch_bounds__(256, W) k_op(MeshView m, HBBlocks hb, const TB
                                                const double* __restrict__ scal, TB* __restrict__ vout,
                                                TB* __restrict__ t_, TB* __restrict__ y_,
                                                const double* __restrict__ rD, const int* __restrict__ cells, int c0,
-                                               int n) {
+                                               int n, NormIn norm) {
     const int i0 = xcdBlock() * blockDim.x + threadIdx.x;
+    double bn = 1.0;
+    if constexpr (PH == 0) {
+        // beta from the norm's partials, by every block; the first one keeps
+        // it for phase 1 and the cycle's end
+        __shared__ double sb;
+        if (norm.part) {
+            if (threadIdx.x < 64) {
+                const double v = waveNorm(norm.part, norm.nb);
+                if (threadIdx.x == 0) {
+                    sb = v;
+                    if (blockIdx.x == 0 && blockIdx.y == 0) {
+                        *norm.beta = v;
+                        *norm.hn = v;
+                    }
+                }
+            }
+            __syncthreads();
+            bn = sb;
+        } else if (scal) bn = *scal;
+    } else if (PH == 1 && scal) bn = *scal;
+    const bool scaled = scal || (PH == 0 && norm.part);
     if (i0 >= n) return;
     const int c = cells ? ldnt(cells + i0) : c0 + i0;
     const size_t nC = m.nC;
@@ -385,7 +452,7 @@ __global__ void __launch_bounds__(256, W) k_op(MeshView m, HBBlocks hb, const TB
         return;
     }
     const TB* w = w_ + off;
-    const TB beta = scal ? (TB)(*scal) : (TB)1;
+    const TB beta = (TB)bn;
     TB x[5];
 #pragma unroll
     for (int q = 0; q < 5; ++q) x[q] = w[(size_t)q * nC + c];
@@ -416,7 +483,7 @@ __global__ void __launch_bounds__(256, W) k_op(MeshView m, HBBlocks hb, const TB
     if constexpr (PH == 0) {
         // sums of w, then scaled
         rowApply<TB, GEN, true, UN>(m, blk, w, c, acc);
-        if (scal)
+        if (scaled)
 #pragma unroll
             for (int q = 0; q < 5; ++q) {
                 acc[q] /= beta;
@@ -428,7 +495,7 @@ __global__ void __launch_bounds__(256, W) k_op(MeshView m, HBBlocks hb, const TB
             t[(size_t)q * nC + c] = x[q] - rd * acc[q];
         }
     } else {
-        if (scal)
+        if (scaled)
 #pragma unroll
             for (int q = 0; q < 5; ++q) {
                 acc[q] /= beta;
@@ -802,13 +869,6 @@ __global__ void k_jacobi_apply(int nC, const TB* __restrict__ dinv, TV* __restri
     for (int i = 0; i < 5; ++i) r[(size_t)i * nC + c] = o[i];
 }
 
-// ---------------------------------------------------------- reductions ----
-__device__ __forceinline__ double waveSum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_down(v, o, 64);
-    return v;
-}
-
 // Block-level sum of NV values per thread -> out[blockIdx.x*NV + k].
 template <int NV>
 __device__ __forceinline__ void blockReduceStore(double (&v)[NV], double* out) {
@@ -950,12 +1010,9 @@ __global__ void __launch_bounds__(256) k_project(int nC, const TV* __restrict__ 
         }
     }
     __shared__ double sh[4][NA];
-    const int lane = threadIdx.x & 63, wvi = threadIdx.x >> 6;
-#pragma unroll
-    for (int k = 0; k < NA; ++k) {
-        const double t = waveSum(v[k]);
-        if (lane == 0) sh[wvi][k] = t;
-    }
+    int id;
+    const double t = waveSums<NA>(v, threadIdx.x & 63, id);
+    sh[threadIdx.x >> 6][id] = t;  // every lane of a value stores the same
     __syncthreads();
     if (threadIdx.x < NA) {
         const int k = threadIdx.x, j = j0 + (k < CH ? k : k - CH);
@@ -1062,16 +1119,10 @@ __global__ void k_gm_init(GmresScalars* g) {
     for (int k = 0; k < 5; ++k) g->res[5 + k] = g->res[k];
 }
 
-// beta = ||r|| (slot 0, a cycle's start) or ||w_i|| (slot i + 1) from the
-// norm partials (one block).
-__global__ void __launch_bounds__(256) k_reduce_norm(const double* __restrict__ part, int nb, GmresScalars* g,
-                                                     int slot) {
-    const double s = sumPartials(part, nb, 1, 0);
-    if (threadIdx.x == 0) {
-        const double beta = sqrt(s);
-        g->beta = beta;
-        g->hn[slot] = beta;
-    }
+// beta = ||r|| (a cycle's start) or ||w_i|| from the norm's partials.
+__global__ void __launch_bounds__(64) k_reduce_norm(NormIn n) {
+    const double beta = waveNorm(n.part, n.nb);
+    if (threadIdx.x == 0) *n.beta = *n.hn = beta;
 }
 
 // Sums of the projection partials, one block per value: projections
@@ -1093,12 +1144,31 @@ __global__ void __launch_bounds__(256) k_reduce_proj(const double* __restrict__ 
 // rows is kept, so the substitution is a product without a serial chain;
 // row i of T follows from L_i, the Gram values that came with s.  Block 0
 // stores column i of H and row i of T.
+// part (few workgroups): the projection partials, nb <= 64 per value, summed
+// here by every block instead of by a launch of its own.
 template <bool WY>
-__device__ void orthCoeffs(GmresScalars* g, int i, double* h) {
+__device__ void orthCoeffs(GmresScalars* g, int i, double* h, const double* __restrict__ part, int nb) {
     __shared__ double s[KMAX], l[KMAX];
     const int t = threadIdx.x;
-    if (t <= i) s[t] = g->s[t];
-    if (WY && t < i) l[t] = g->s[KMAX + t];
+    if (part) {
+        const int lane = t & 63;
+        for (int q0 = 16 * (t >> 6); q0 < (WY ? KMAX + i : i + 1); q0 += 64) {
+            double v[16];
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const int q = q0 + k;
+                const bool has = lane < nb && (q < KMAX ? q <= i : q < KMAX + i);
+                v[k] = has ? part[(size_t)q * nb + lane] : 0.0;
+            }
+            int id;
+            const double a = waveSums<16>(v, lane, id);
+            if (q0 < KMAX) s[q0 + id] = a;
+            else l[q0 - KMAX + id] = a;
+        }
+    } else {
+        if (t <= i) s[t] = g->s[t];
+        if (WY && t < i) l[t] = g->s[KMAX + t];
+    }
     __syncthreads();
     if (WY) {
         double a = 0;
@@ -1121,48 +1191,49 @@ __device__ void orthCoeffs(GmresScalars* g, int i, double* h) {
     if (blockIdx.x == 0 && t <= i) g->H[t][i] = h[t];
 }
 
-// w -= sum_j h_j V_j (j <= i), then ||w||^2 partials
+// w -= sum_j h_j V_j (j <= i), then ||w||^2 partials.  A thread takes single
+// entries, 16 basis vectors' loads in flight, added in order j = 0..i
+// (104x96x96 FP32, 16 vectors on average: 58 us with four vectors of five
+// entries in flight -> 55 us).
 template <typename TV, bool WY>
-__global__ void __launch_bounds__(256) k_orth_update(int nC, TV* __restrict__ w, const TV* __restrict__ Vb,
-                                                     size_t vstride, GmresScalars* g, int i,
+__global__ void __launch_bounds__(1024) k_orth_update(size_t n, TV* __restrict__ w, const TV* __restrict__ Vb,
+                                                     GmresScalars* g, int i, const double* __restrict__ proj, int nb,
                                                      double* __restrict__ part) {
     __shared__ double h[KMAX];
-    orthCoeffs<WY>(g, i, h);
+    orthCoeffs<WY>(g, i, h, proj, nb);
     const int nv = i + 1;
-    double v[1] = {0};
-    for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nC; c += gridDim.x * blockDim.x) {
-        // five independent chains (one per component), basis vectors in
-        // order j = 0..nv-1 on each; four basis vectors' loads in flight
-        TV a[5];
-#pragma unroll
-        for (int q = 0; q < 5; ++q) a[q] = w[(size_t)q * nC + c];
+    double v = 0;
+    for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (size_t)gridDim.x * blockDim.x) {
+        TV a = w[e];
+        const TV* q = Vb + e;
         int j = 0;
-        for (; j + 4 <= nv; j += 4) {
-            TV x[4][5];
+        for (; j + 16 <= nv; j += 16, q += 16 * n) {
+            TV x[16];
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+            for (int u = 0; u < 16; ++u) x[u] = __builtin_nontemporal_load(q + u * n);
 #pragma unroll
-                for (int q = 0; q < 5; ++q)
-                    x[u][q] = __builtin_nontemporal_load(Vb + (size_t)(j + u) * vstride + (size_t)q * nC + c);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const TV hj = (TV)h[j + u];
-#pragma unroll
-                for (int q = 0; q < 5; ++q) a[q] -= hj * x[u][q];
-            }
+            for (int u = 0; u < 16; ++u) a -= (TV)h[j + u] * x[u];
         }
-        for (; j < nv; ++j) {
-            const TV hj = (TV)h[j];
+        if (j < nv) {
+            TV x[16];
 #pragma unroll
-            for (int q = 0; q < 5; ++q) a[q] -= hj * Vb[(size_t)j * vstride + (size_t)q * nC + c];
-        }
+            for (int u = 0; u < 16; ++u) x[u] = j + u < nv ? __builtin_nontemporal_load(q + u * n) : (TV)0;
 #pragma unroll
-        for (int q = 0; q < 5; ++q) {
-            w[(size_t)q * nC + c] = a[q];
-            v[0] += (double)a[q] * (double)a[q];
+            for (int u = 0; u < 16; ++u)
+                if (j + u < nv) a -= (TV)h[j + u] * x[u];
         }
+        w[e] = a;
+        v += (double)a * (double)a;
     }
-    blockReduceStore<1>(v, part);
+    __shared__ double sh[16];
+    v = waveSum(v);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = sh[0];
+        for (int k = 1; k < (int)(blockDim.x >> 6); ++k) t += sh[k];
+        part[blockIdx.x] = t;
+    }
 }
 
 // End of a cycle (one wavefront, lane = column): the Givens rotations of the
@@ -1170,7 +1241,8 @@ __global__ void __launch_bounds__(256) k_orth_update(int nC, TV* __restrict__ w,
 // substitution into yh.  Step k's rotation is formed by lane k and applied
 // to all later columns at once, from LDS: 30 directions take 30 short steps
 // instead of the 435 dependent column updates of one thread.
-__global__ void __launch_bounds__(64) k_gm_finish(GmresScalars* g, int n) {
+// part: the last norm's partials (null: hn[n] is there).
+__global__ void __launch_bounds__(64) k_gm_finish(GmresScalars* g, int n, const double* __restrict__ part, int nb) {
     __shared__ double Hs[KMAX + 1][KMAX];
     __shared__ double bh[KMAX + 1], rot[2];
     const int t = threadIdx.x;
@@ -1181,6 +1253,11 @@ __global__ void __launch_bounds__(64) k_gm_finish(GmresScalars* g, int n) {
     }
     if (t == 0) bh[0] = g->hn[0];
     __syncthreads();
+    if (part) {
+        const double beta = waveNorm(part, nb);
+        if (t == 0) Hs[n][n - 1] = beta;
+        __syncthreads();
+    }
     for (int k = 0; k < n; ++k) {
         if (t == k) {
             double c, s;
@@ -1297,11 +1374,13 @@ void launchSpmv(const MeshView& m, int blkFp32, int vecFp32, const void* blk, co
 // 1.643 ms, 64^3 4.43 / 4.48 ms; mixed 48^3 1.90 / 1.74 ms, 64^3 3.08 /
 // 3.12 ms.
 constexpr size_t kOpLatencyRows = 65536;
+// Cells (instances included) from which a norm is summed by a launch of its own.
+constexpr int kNormMergeCells = 200000;
 
 template <typename TB, bool GEN, bool HB, int UN, int W>
 static void opPhases(const MeshView& m, const Levels& L, const HBBlocks& hb, const void* blk, const void* dg,
-                     const double* rD, const void* x, const double* scal, void* vout, void* t, void* y, int bs,
-                     hipStream_t st) {
+                     const double* rD, const void* x, const double* scal, const NormIn& norm, void* vout, void* t,
+                     void* y, int bs, hipStream_t st) {
     const int n0 = L.fwdPtrHost[1], n1 = L.fwdPtrHost[2] - n0;
     const int s0 = L.bwdPtrHost[1], nbw = L.bwdPtrHost[2] - s0;
     const int nO = HB ? hb.nO : 1;
@@ -1310,35 +1389,35 @@ static void opPhases(const MeshView& m, const Levels& L, const HBBlocks& hb, con
     const int* l2 = L.colourMajor ? nullptr : L.bwdCells + s0;
     const TB *B = (const TB*)blk, *G = (const TB*)dg, *X = (const TB*)x;
     TB *V = (TB*)vout, *T = (TB*)t, *Y = (TB*)y;
-    k_op<TB, GEN, 0, HB, UN, W><<<dim3(xcdGrid(n0, bs), nO), bs, 0, st>>>(m, hb, B, G, X, scal, V, T, Y, rD, l0, 0, n0);
-    k_op<TB, GEN, 1, HB, UN, W><<<dim3(xcdGrid(n1, bs), nO), bs, 0, st>>>(m, hb, B, G, X, scal, V, T, Y, rD, l1, n0, n1);
-    k_op<TB, GEN, 2, HB, UN, W><<<dim3(xcdGrid(nbw, bs), nO), bs, 0, st>>>(m, hb, B, G, X, scal, V, T, Y, rD, l2, 0, nbw);
+    k_op<TB, GEN, 0, HB, UN, W><<<dim3(xcdGrid(n0, bs), nO), bs, 0, st>>>(m, hb, B, G, X, scal, V, T, Y, rD, l0, 0, n0, norm);
+    k_op<TB, GEN, 1, HB, UN, W><<<dim3(xcdGrid(n1, bs), nO), bs, 0, st>>>(m, hb, B, G, X, scal, V, T, Y, rD, l1, n0, n1, norm);
+    k_op<TB, GEN, 2, HB, UN, W><<<dim3(xcdGrid(nbw, bs), nO), bs, 0, st>>>(m, hb, B, G, X, scal, V, T, Y, rD, l2, 0, nbw, norm);
 }
 
 template <typename TB, bool HB>
 static void opLaunch(const MeshView& m, const Levels& L, const HBBlocks& hb, const void* blk, const void* dg,
-                     const double* rD, const void* x, const double* scal, void* vout, void* t, void* y, int bs,
-                     hipStream_t st) {
+                     const double* rD, const void* x, const double* scal, const NormIn& norm, void* vout, void* t,
+                     void* y, int bs, hipStream_t st) {
     const bool few = (size_t)L.fwdPtrHost[1] * (HB ? hb.nO : 1) <= kOpLatencyRows;
-    if (!m.blkGen) opPhases<TB, false, HB, 1, 1>(m, L, hb, blk, dg, rD, x, scal, vout, t, y, bs, st);
-    else if (few) opPhases<TB, true, HB, sizeof(TB) == 4 ? 6 : 2, 1>(m, L, hb, blk, dg, rD, x, scal, vout, t, y, bs, st);
+    if (!m.blkGen) opPhases<TB, false, HB, 1, 1>(m, L, hb, blk, dg, rD, x, scal, norm, vout, t, y, bs, st);
+    else if (few) opPhases<TB, true, HB, sizeof(TB) == 4 ? 6 : 2, 1>(m, L, hb, blk, dg, rD, x, scal, norm, vout, t, y, bs, st);
     else {
         // register budgets: FP32 fits 8 waves per SIMD (64 VGPRs), FP64 4
         if constexpr (!HB)
             if (m.occOp)
-                return opPhases<TB, true, HB, 1, sizeof(TB) == 4 ? 8 : 4>(m, L, hb, blk, dg, rD, x, scal, vout, t, y,
-                                                                         bs, st);
-        opPhases<TB, true, HB, 1, 1>(m, L, hb, blk, dg, rD, x, scal, vout, t, y, bs, st);
+                return opPhases<TB, true, HB, 1, sizeof(TB) == 4 ? 8 : 4>(m, L, hb, blk, dg, rD, x, scal, norm, vout,
+                                                                         t, y, bs, st);
+        opPhases<TB, true, HB, 1, 1>(m, L, hb, blk, dg, rD, x, scal, norm, vout, t, y, bs, st);
     }
 }
 
 bool launchSpmvLusgs(const MeshView& m, const Levels& L, int blkFp32, int vecFp32, const void* blk, const void* dg,
-                     const double* rD, const void* x, const double* scal, void* vout, void* t, void* y,
-                     hipStream_t st) {
-    if (!L.twoColour || blkFp32 != vecFp32) return false;
+                     const double* rD, const void* x, const double* scal, const NormIn& norm, void* vout, void* t,
+                     void* y, hipStream_t st) {
+    if (!fusedOperator(L, blkFp32, vecFp32)) return false;
     const HBBlocks none{};
-    if (vecFp32) opLaunch<float, false>(m, L, none, blk, dg, rD, x, scal, vout, t, y, m.bsOp, st);
-    else opLaunch<double, false>(m, L, none, blk, dg, rD, x, scal, vout, t, y, m.bsOp, st);
+    if (vecFp32) opLaunch<float, false>(m, L, none, blk, dg, rD, x, scal, norm, vout, t, y, m.bsOp, st);
+    else opLaunch<double, false>(m, L, none, blk, dg, rD, x, scal, norm, vout, t, y, m.bsOp, st);
     return true;
 }
 
@@ -1408,29 +1487,43 @@ void launchJacobiApply(int nC, int blkFp32, int vecFp32, const void* dinv, void*
     else k_jacobi_apply<double, double><<<nb(nC, 256), 256, 0, st>>>(nC, (const double*)dinv, (double*)r);
 }
 
+// Workgroup size and workgroups of the update of 5 nC entries: at most 256
+// where every workgroup of the operator's first phase sums their partials
+// (53x42x39 FP64: 16 + 11 us, with up to 1024 of 256 threads 16 + 15), else up
+// to 1024 small ones (104x96x96 FP32: 55 us against 60, 64^3 FP64 31 against 36).
+static int updateThreads(int nC) { return nC < kNormMergeCells && (size_t)5 * nC > 65536 ? 1024 : 256; }
+static int updateBlocks(int nC) {
+    const int n = nb((size_t)5 * nC, updateThreads(nC)), most = nC < kNormMergeCells ? 256 : 1024;
+    return n < most ? n : most;
+}
+
 // Orthogonalisation of w against v_0..v_i (V): projections, their reduction,
-// the update with ||w||, and its reduction (beta).  Four launches for both
-// Gram-Schmidt forms; modified Gram-Schmidt step by step took 2 (i + 2)
-// launches and 4 (i + 1) vector passes where this takes 2 i + 6 (200x50x1
-// cells, GMRES(30): 990 of the cycle's 1110 launches).  Pseudo-steps with
-// modified Gram-Schmidt, FP64: 200x50x1 3.83 -> 1.34 ms, 53x42x39 viscous
-// 5.69 -> 2.86 ms; classical, 64^3: 5.89 -> 5.39 ms (one projection launch
-// for all chunks, the Givens chain once per cycle).
+// the update with ||w||'s partials.  Three launches for both Gram-Schmidt
+// forms, two with at most 64 workgroups (16 384 cells), whose update sums the
+// projection partials itself; modified Gram-Schmidt step by step took
+// 2 (i + 2) launches and 4 (i + 1) vector passes where this takes 2 i + 6
+// (200x50x1 cells, GMRES(30): 990 of the cycle's 1110 launches).  The norm's
+// partials are summed by whoever needs it next: the operator's first phase,
+// the cycle's end, or k_reduce_norm.  Pseudo-steps with modified
+// Gram-Schmidt, FP64: 200x50x1 3.83 -> 1.34 ms, 53x42x39 viscous 5.69 -> 2.86
+// ms; classical, 64^3: 5.89 -> 5.39 ms (one projection launch for all chunks,
+// the Givens chain once per cycle).
+template <typename TV, bool WY>
+static void orthStepT(const MeshView& m, int nC, TV* w, const TV* V, int i, GmresScalars* g, double* part,
+                      hipStream_t st) {
+    const int nbk = reduceBlocks(nC);
+    const size_t vs = (size_t)5 * nC;
+    const bool few = nbk <= 64;
+    launchProject<TV, WY>(m.mdCh, nbk, nC, w, V, vs, i + 1, part, st);
+    if (!few) k_reduce_proj<<<WY ? 2 * i + 1 : i + 1, 256, 0, st>>>(part, nbk, g, i + 1);
+    k_orth_update<TV, WY><<<updateBlocks(nC), updateThreads(nC), 0, st>>>(vs, w, V, g, i, few ? part : nullptr, nbk,
+                                                           part + kNormPart);
+}
 template <typename TV>
 static void orthStep(const MeshView& m, int orth, int nC, TV* w, const TV* V, int i, GmresScalars* g, double* part,
                      hipStream_t st) {
-    const int nbk = reduceBlocks(nC);
-    const size_t vs = (size_t)5 * nC;
-    if (orth == 0) {
-        launchProject<TV, true>(m.mdCh, nbk, nC, w, V, vs, i + 1, part, st);
-        k_reduce_proj<<<2 * i + 1, 256, 0, st>>>(part, nbk, g, i + 1);
-        k_orth_update<TV, true><<<nbk, 256, 0, st>>>(nC, w, V, vs, g, i, part);
-    } else {
-        launchProject<TV, false>(m.mdCh, nbk, nC, w, V, vs, i + 1, part, st);
-        k_reduce_proj<<<i + 1, 256, 0, st>>>(part, nbk, g, i + 1);
-        k_orth_update<TV, false><<<nbk, 256, 0, st>>>(nC, w, V, vs, g, i, part);
-    }
-    k_reduce_norm<<<1, 256, 0, st>>>(part, nbk, g, i + 1);
+    if (orth == 0) orthStepT<TV, true>(m, nC, w, V, i, g, part, st);
+    else orthStepT<TV, false>(m, nC, w, V, i, g, part, st);
 }
 
 // --------------------------------------------------------- GMRES driver --
@@ -1454,27 +1547,35 @@ void gmresCycleT(const GmresArgs& a, hipStream_t st) {
         else if (a.precond == 1) launchJacobiApply(nC, a.blkFp32, sizeof(TV) == 4, a.dinv, v, st);
         mark(TK_PRECOND, 0);
     };
-    // r <- P^-1 r; beta = ||r||
+    // r <- P^-1 r; ||r||
     precond(r);
-    k_norm2<TV><<<nbk, 256, 0, st>>>(nC, r, a.wk->part);
-    k_reduce_norm<<<1, 256, 0, st>>>(a.wk->part, nbk, g, 0);
+    double* pn = a.wk->part + kNormPart;
+    k_norm2<TV><<<nbk, 256, 0, st>>>(nC, r, pn);
+    // fused SpMV + LU-SGS on two-colour level structures (the colour-1
+    // blocks are read once for both; the SPMV timing class then covers the
+    // sweeps too), which sums the norm's partials as well; otherwise the
+    // norm, the SpMV, then the preconditioner
+    const bool fused = a.opPre || (!a.op && !a.pre && a.precond == 0 && a.fuse &&
+                                   fusedOperator(*a.lev, a.blkFp32, sizeof(TV) == 4));
     for (int i = 0; i < a.nDirs; ++i) {
         TV* vi = V + (size_t)i * vs;
-        // v_i = r / beta ; w = A v_i (into the other buffer: the SpMV gathers
+        // v_i = r / ||r|| ; w = A v_i (into the other buffer: the SpMV gathers
         // neighbour entries of its input, so it never runs in place)
-        // fused SpMV + LU-SGS on two-colour level structures (the colour-1
-        // blocks are read once for both; the SPMV timing class then covers
-        // the sweeps too); otherwise SpMV, then the preconditioner
+        const NormIn all{pn, i == 0 ? nbk : updateBlocks(nC), &g->beta, &g->hn[i]};
+        // many partials are summed once instead of by every block of the
+        // operator's first phase (104x96x96, 1024 partials: 43 us against
+        // 35 + 5; 53x42x39, 340: 11.9 against 11.1 + 4.7)
+        const bool own = !fused || nC >= kNormMergeCells;
+        if (own) k_reduce_norm<<<1, 64, 0, st>>>(all);
+        NormIn norm = all;
+        if (own) norm.part = nullptr;
         mark(TK_SPMV, 1);
-        bool fused = false;
-        if (a.opPre) fused = a.opPre(r, &g->beta, vi, r2);
-        else if (!a.op && !a.pre && a.precond == 0 && a.fuse)
-            fused = launchSpmvLusgs(m, *a.lev, a.blkFp32, sizeof(TV) == 4, a.blk, a.dg, a.rD, r, &g->beta, vi,
-                                    a.t, r2, st);
-        if (!fused) {
-            if (a.op) a.op(r, &g->beta, vi, r2);
-            else launchSpmv(m, a.blkFp32, sizeof(TV) == 4, a.blk, a.dg, r, &g->beta, vi, r2, st);
-        }
+        if (a.opPre) a.opPre(r, norm, vi, r2);
+        else if (fused)
+            launchSpmvLusgs(m, *a.lev, a.blkFp32, sizeof(TV) == 4, a.blk, a.dg, a.rD, r, &g->beta, norm, vi, a.t, r2,
+                            st);
+        else if (a.op) a.op(r, &g->beta, vi, r2);
+        else launchSpmv(m, a.blkFp32, sizeof(TV) == 4, a.blk, a.dg, r, &g->beta, vi, r2, st);
         mark(TK_SPMV, 0);
         {
             TV* t = r;
@@ -1486,7 +1587,7 @@ void gmresCycleT(const GmresArgs& a, hipStream_t st) {
         orthStep<TV>(m, a.orth, nC, r, V, i, g, a.wk->part, st);
         mark(TK_ORTH, 0);
     }
-    k_gm_finish<<<1, 64, 0, st>>>(g, a.nDirs);
+    k_gm_finish<<<1, 64, 0, st>>>(g, a.nDirs, pn, updateBlocks(nC));
 }
 
 }  // namespace icsf
@@ -1635,10 +1736,11 @@ void launchLusgsHB(const MeshView& m, const Levels& L, const HBBlocks& hb, int v
 }
 
 bool launchSpmvLusgsHB(const MeshView& m, const Levels& L, const HBBlocks& hb, int vecFp32, const double* rD,
-                       const void* x, const double* scal, void* vout, void* t, void* y, hipStream_t st) {
-    if (!L.twoColour || hb.fp32 != vecFp32) return false;
-    if (vecFp32) opLaunch<float, true>(m, L, hb, nullptr, nullptr, rD, x, scal, vout, t, y, 256, st);
-    else opLaunch<double, true>(m, L, hb, nullptr, nullptr, rD, x, scal, vout, t, y, 256, st);
+                       const void* x, const double* scal, const NormIn& norm, void* vout, void* t, void* y,
+                       hipStream_t st) {
+    if (!fusedOperator(L, hb.fp32, vecFp32)) return false;
+    if (vecFp32) opLaunch<float, true>(m, L, hb, nullptr, nullptr, rD, x, scal, norm, vout, t, y, 256, st);
+    else opLaunch<double, true>(m, L, hb, nullptr, nullptr, rD, x, scal, norm, vout, t, y, 256, st);
     return true;
 }
 
@@ -1697,11 +1799,12 @@ void fgmresCycle(const FgmresArgs& a, hipStream_t st) {
     double* V = (double*)a.V;
     double* Z = (double*)a.Z;
     GmresScalars* g = a.g;
-    k_norm2<double><<<nbk, 256, 0, st>>>(nC, r, a.wk->part);
-    k_reduce_norm<<<1, 256, 0, st>>>(a.wk->part, nbk, g, 0);
+    double* pn = a.wk->part + kNormPart;
+    k_norm2<double><<<nbk, 256, 0, st>>>(nC, r, pn);
     for (int i = 0; i < a.nDirs; ++i) {
         double* vi = V + (size_t)i * vs;
         double* zi = Z + (size_t)i * vs;
+        k_reduce_norm<<<1, 64, 0, st>>>(NormIn{pn, i == 0 ? nbk : updateBlocks(nC), &g->beta, &g->hn[i]});
         k_scale_by<double><<<nb(vs, 256), 256, 0, st>>>(vs, r, &g->beta, vi);
         a.precond(vi, zi);
         // the outer product is timed with the other work, so that the
@@ -1714,7 +1817,8 @@ void fgmresCycle(const FgmresArgs& a, hipStream_t st) {
         orthStep<double>(m, a.orth, nC, r, V, i, g, a.wk->part, st);
         if (a.mark) a.mark(TK_ORTH, 0);
     }
-    k_gm_finish<<<1, 64, 0, st>>>(g, a.nDirs);
+    k_reduce_norm<<<1, 64, 0, st>>>(NormIn{pn, updateBlocks(nC), &g->beta, &g->hn[a.nDirs]});
+    k_gm_finish<<<1, 64, 0, st>>>(g, a.nDirs, nullptr, 0);
 }
 
 // z = sum_i y_i V_i from zero (inner solve result), FP32 or FP64 vectors.

@@ -797,7 +797,7 @@ int autotune(icsf_case* c) {
         int occDummy = 0;
         pick2(m.bsOp, m.blkGen ? m.occOp : occDummy, [&] {
             if (!(c->fuse && launchSpmvLusgs(m, c->mesh->lev, c->blkFp32, v32, c->blk, c->dg, c->rD, x, nullptr,
-                                             nullptr, c->dW, y, c->st))) {
+                                             NormIn{}, nullptr, c->dW, y, c->st))) {
                 launchSpmv(m, c->blkFp32, v32, c->blk, c->dg, x, nullptr, nullptr, y, c->st);
                 launchLusgs(m, c->mesh->lev, c->wk, c->blkFp32, v32, c->blk, c->rD, y, c->st);
             }
@@ -1258,9 +1258,9 @@ int hbSolve(icsf_hb* h, const double* b, int& nIter) {
             launchSpmvHB(m, h->hbb, 0, x, scal, vout, y, h->st);
         };
         a.pre = [h](void* v) { hbLusgs(h, v); };
-        if (h->fuse)
-            a.opPre = [h, &m](const void* x, const double* scal, void* vout, void* y) {
-                return launchSpmvLusgsHB(m, h->mesh->lev, h->hbb, 0, h->rD, x, scal, vout, h->t1, y, h->st);
+        if (h->fuse && fusedOperator(h->mesh->lev, h->hbb.fp32, 0))
+            a.opPre = [h, &m](const void* x, const NormIn& n, void* vout, void* y) {
+                launchSpmvLusgsHB(m, h->mesh->lev, h->hbb, 0, h->rD, x, n.beta, n, vout, h->t1, y, h->st);
             };
         gmresCycle(a, 0, h->st);
         launchUpdateSolution((size_t)m.nC * h->nO, h->dW, h->V, vA, h->nDirs, h->g, h->st);
@@ -1315,9 +1315,9 @@ int hbSolveMixed(icsf_hb* h, const double* b, int& nIter) {
             launchSpmvHB(m, h->hbb, 1, x, scal, vout, y, h->st);
         };
         a.pre = [h](void* v) { hbLusgs(h, v, 1); };
-        if (h->fuse)
-            a.opPre = [h, &m](const void* x, const double* scal, void* vout, void* y) {
-                return launchSpmvLusgsHB(m, h->mesh->lev, h->hbb, 1, h->rD, x, scal, vout, h->t1, y, h->st);
+        if (h->fuse && fusedOperator(h->mesh->lev, h->hbb.fp32, 1))
+            a.opPre = [h, &m](const void* x, const NormIn& n, void* vout, void* y) {
+                launchSpmvLusgsHB(m, h->mesh->lev, h->hbb, 1, h->rD, x, n.beta, n, vout, h->t1, y, h->st);
             };
         gmresCycle(a, 1, h->st);
         launchCombine(nVec, 1, h->V32, h->innerDirs, h->g2, h->r32, h->st);
