@@ -174,6 +174,10 @@ void launchProjectionPasses(const MeshView& m, int vecFp32, int ch, int mgs, con
 void launchUpdate(const MeshView& m, const Phys& ph, const StateView& s, const double* dW, int mode,
                   const double* rho0, const double* U0, const double* T0, hipStream_t st,
                   const double* Wsrc = nullptr, double* W0 = nullptr);
+// the same for instances J0 .. J0 + n - 1 of a harmonic-balance system, each
+// with its own view, dW [nO][5][nC]
+void launchUpdateHB(const HBInst* inst, int J0, int n, const MeshView& m, const Phys& ph, const double* dW,
+                    hipStream_t st);
 // Forward part of the residual adjoint: boundary values and gradients,
 // keeping the unlimited gradients and limiter values.
 void launchAdjointForward(const MeshView& m, const Phys& ph, const StateView& s, double* gun, double* limo,
@@ -247,10 +251,20 @@ bool launchSpmvLusgsHB(const MeshView& m, const Levels& L, const HBBlocks& hb, i
 // LU-SGS of all HB instances (per-instance sweeps, shared diagonal rD).
 void launchLusgsHB(const MeshView& m, const Levels& L, const HBBlocks& hb, int vecFp32, const double* rD, void* r,
                    hipStream_t st);
-void sliceSubAverage(const MeshView& m, Work& wk, GmresScalars* g, const double* W, double* out, hipStream_t st);
-void sliceNormFactors(const MeshView& m, Work& wk, GmresScalars* g, const double* t, const double* b,
-                      hipStream_t st);
-void sliceFinalResidual(const MeshView& m, Work& wk, GmresScalars* g, const double* b, double* r, hipStream_t st);
+// The pieces of gmresPrepare / gmresUpdateAndResidual for nO instances' vectors
+// [nO][5][nC], one launch over all; g: the solver's scalars (scratch sums),
+// gp: each instance's residuals.
+struct GmresPtrs {
+    GmresScalars* g[HB_MAXO];
+};
+void hbSubAverage(const MeshView& m, int nO, Work& wk, GmresScalars* g, const double* W, double* out,
+                  hipStream_t st);
+void hbNormFactors(const MeshView& m, int nO, Work& wk, const GmresPtrs& gp, const double* t, const double* b,
+                   hipStream_t st);
+void hbFinalResidual(const MeshView& m, int nO, Work& wk, const GmresPtrs& gp, const double* b, double* r,
+                     hipStream_t st);
+// a solve's start over n entries: r = b, dW = 0
+void launchStart(size_t n, const double* b, double* r, double* dW, hipStream_t st);
 // dW += sum_i y_i V_i over 5*nVec entries
 void launchUpdateSolution(size_t nVec, double* dW, const double* V, size_t vstride, int nv, const GmresScalars* g,
                           hipStream_t st);

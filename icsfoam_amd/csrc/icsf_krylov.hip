@@ -902,18 +902,32 @@ __device__ __forceinline__ double sumPartials(const double* __restrict__ part, i
     return s;
 }
 
-// Final reduction of [nb][nv] partials: value k = blockIdx.x (grid nv,
-// 256 threads); out[k].
+// Sum of value k over nb partial rows of `stride` values by one wavefront, in
+// a fixed order (lane t adds rows t, t+64, ...; then the lanes).
+__device__ __forceinline__ double waveSumPartials(const double* __restrict__ part, int nb, int stride, int k) {
+    double v = 0;
+    for (int b = threadIdx.x & 63; b < nb; b += 64) v += part[(size_t)b * stride + k];
+    return waveSum(v);
+}
+
+// Final reduction of an instance's [nb][nv] partials (instance blockIdx.y):
+// value k = blockIdx.x (grid nv, 256 threads); out[8 instance + k].
 __global__ void __launch_bounds__(256) k_reduce_final(const double* __restrict__ part, int nb, int nv,
                                                       double* __restrict__ out) {
     const int k = blockIdx.x;
-    const double s = sumPartials(part, nb, nv, k);
-    if (threadIdx.x == 0) out[k] = s;
+    const double s = sumPartials(part + (size_t)blockIdx.y * nb * 8, nb, nv, k);
+    if (threadIdx.x == 0) out[8 * blockIdx.y + k] = s;
 }
+
+// The reductions of a solve's start and end run over blockIdx.y = instance of
+// a harmonic-balance system (vectors [nO][5][nC]; one otherwise), partials
+// [instance][block][value] with 8 rows' room per block.
 
 // sums of the 5 components of x (for the average) -> partials
 template <typename TV>
 __global__ void __launch_bounds__(256) k_sum5(int nC, const TV* __restrict__ x, double* __restrict__ part) {
+    x += (size_t)blockIdx.y * 5 * nC;
+    part += (size_t)blockIdx.y * gridDim.x * 8;
     double v[5] = {0, 0, 0, 0, 0};
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nC; c += gridDim.x * blockDim.x)
 #pragma unroll
@@ -926,6 +940,9 @@ __global__ void __launch_bounds__(256) k_sum5(int nC, const TV* __restrict__ x, 
 template <typename TV>
 __global__ void __launch_bounds__(256) k_normfactor(int nC, const TV* __restrict__ t, const TV* __restrict__ b,
                                                     double* __restrict__ part) {
+    t += (size_t)blockIdx.y * 5 * nC;
+    b += (size_t)blockIdx.y * 5 * nC;
+    part += (size_t)blockIdx.y * gridDim.x * 8;
     double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nC; c += gridDim.x * blockDim.x) {
         double tv[5], bv[5];
@@ -947,6 +964,9 @@ __global__ void __launch_bounds__(256) k_normfactor(int nC, const TV* __restrict
 template <typename TV>
 __global__ void __launch_bounds__(256) k_resid_l1(int nC, const TV* __restrict__ b, TV* __restrict__ Ax,
                                                   double* __restrict__ part) {
+    b += (size_t)blockIdx.y * 5 * nC;
+    Ax += (size_t)blockIdx.y * 5 * nC;
+    part += (size_t)blockIdx.y * gridDim.x * 8;
     double v[5] = {0, 0, 0, 0, 0};
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nC; c += gridDim.x * blockDim.x)
 #pragma unroll
@@ -1033,13 +1053,34 @@ void launchProject(int ch, int nbk, int nC, const TV* w, const TV* V, size_t vs,
     else k_project<TV, 16, WY><<<g, 256, 0, st>>>(nC, w, V, vs, nv, part);
 }
 
-// x = y - avg (component-wise); dW = 0 afterwards is done by memset.
+// x = y - avg (component-wise), instance blockIdx.y.  The sums are those of
+// k_reduce_final, or (part, nb partial rows) are formed here by every block.
 template <typename TV>
-__global__ void k_sub_avg(int nC, const TV* __restrict__ W, const double* __restrict__ sums, TV* __restrict__ out) {
+__global__ void __launch_bounds__(256) k_sub_avg(int nC, const TV* __restrict__ W, const double* __restrict__ sums,
+                                                 const double* __restrict__ part, int nb, TV* __restrict__ out) {
+    __shared__ double sh[5];
+    if (part) {
+        for (int k = threadIdx.x >> 6; k < 5; k += 4) {
+            const double a = waveSumPartials(part + (size_t)blockIdx.y * nb * 8, nb, 5, k);
+            if ((threadIdx.x & 63) == 0) sh[k] = a;
+        }
+    } else if (threadIdx.x < 5) sh[threadIdx.x] = sums[8 * blockIdx.y + threadIdx.x];
+    __syncthreads();
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nC) return;
+    W += (size_t)blockIdx.y * 5 * nC;
+    out += (size_t)blockIdx.y * 5 * nC;
 #pragma unroll
-    for (int k = 0; k < 5; ++k) out[(size_t)k * nC + c] = W[(size_t)k * nC + c] - (TV)(sums[k] / nC);
+    for (int k = 0; k < 5; ++k) out[(size_t)k * nC + c] = W[(size_t)k * nC + c] - (TV)(sh[k] / nC);
+}
+
+// a GMRES solve's start: r = b, dW = 0
+__global__ void __launch_bounds__(256) k_start(size_t n, const double* __restrict__ b, double* __restrict__ r,
+                                               double* __restrict__ dW) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    r[i] = b[i];
+    dW[i] = 0.0;
 }
 
 template <typename TV>
@@ -1088,7 +1129,7 @@ struct GmresScalars {
     double beta;
     double sNF[2], vNF;
     double res[10];   // sInit[2] vInit[3] sFinal[2] vFinal[3]
-    double red[64];   // scratch reduction results
+    double red[8 * HB_MAXO];  // component sums of the state, 8 per instance
 };
 
 namespace {
@@ -1106,17 +1147,23 @@ __device__ void givensRot(double h, double beta, double& c, double& s) {
     }
 }
 
-// Norm factors and initial residuals from the k_normfactor reduction.
-__global__ void k_gm_init(GmresScalars* g) {
+// Norm factors and initial residuals from the k_normfactor partials, one
+// block per instance, one wavefront per value (512 threads).
+__global__ void __launch_bounds__(512) k_gm_init(GmresPtrs gp, const double* __restrict__ part, int nb) {
+    GmresScalars* g = gp.g[blockIdx.x];
+    __shared__ double r[8];
+    const int k = threadIdx.x >> 6;
+    const double a = waveSumPartials(part + (size_t)blockIdx.x * nb * 8, nb, 8, k);
+    if ((threadIdx.x & 63) == 0) r[k] = a;
+    __syncthreads();
     if (threadIdx.x != 0) return;
-    const double* r = g->red;
     g->sNF[0] = r[0] + kVSMALL;
     g->sNF[1] = r[1] + kVSMALL;
     g->vNF = r[2] + kVSMALL;
     g->res[0] = r[3] / g->sNF[0];
     g->res[1] = r[4] / g->sNF[1];
     for (int d = 0; d < 3; ++d) g->res[2 + d] = r[5 + d] / g->vNF;
-    for (int k = 0; k < 5; ++k) g->res[5 + k] = g->res[k];
+    for (int q = 0; q < 5; ++q) g->res[5 + q] = g->res[q];
 }
 
 // beta = ||r|| (a cycle's start) or ||w_i|| from the norm's partials.
@@ -1291,9 +1338,15 @@ __global__ void __launch_bounds__(64) k_gm_finish(GmresScalars* g, int n, const 
     }
 }
 
-__global__ void k_gm_final(GmresScalars* g, int emptyDir) {
+__global__ void __launch_bounds__(320) k_gm_final(GmresPtrs gp, const double* __restrict__ part, int nb,
+                                                  int emptyDir) {
+    GmresScalars* g = gp.g[blockIdx.x];
+    __shared__ double r[5];
+    const int k = threadIdx.x >> 6;
+    const double a = waveSumPartials(part + (size_t)blockIdx.x * nb * 8, nb, 5, k);
+    if ((threadIdx.x & 63) == 0) r[k] = a;
+    __syncthreads();
     if (threadIdx.x != 0) return;
-    const double* r = g->red;
     g->res[5] = r[0] / g->sNF[0];
     g->res[6] = r[1] / g->sNF[1];
     for (int d = 0; d < 3; ++d) g->res[7 + d] = (d == emptyDir) ? 0.0 : r[2 + d] / g->vNF;
@@ -1609,18 +1662,40 @@ void gmresCycle(const GmresArgs& a, int vecFp32, hipStream_t st) {
     else gmresCycleT<double>(a, st);
 }
 
+// Up to this many workgroups of partial sums (32 768 cells) the average is
+// formed by k_sub_avg's blocks instead of by a launch of its own.
+constexpr int kSubAvgMerge = 128;
+
+template <typename TV>
+static void subAverage(int nC, int nO, Work& wk, GmresScalars* g, const TV* W, TV* out, hipStream_t st) {
+    const int nbk = reduceBlocks(nC);
+    const bool merge = nbk <= kSubAvgMerge;
+    k_sum5<TV><<<dim3(nbk, nO), 256, 0, st>>>(nC, W, wk.part);
+    if (!merge) k_reduce_final<<<dim3(5, nO), 256, 0, st>>>(wk.part, nbk, 5, g->red);
+    k_sub_avg<TV><<<dim3(nb(nC, 256), nO), 256, 0, st>>>(nC, W, g->red, merge ? wk.part : nullptr, nbk, out);
+}
+
+template <typename TV>
+static void normFactors(int nC, int nO, Work& wk, const GmresPtrs& gp, const TV* t, const TV* b, hipStream_t st) {
+    const int nbk = reduceBlocks(nC);
+    k_normfactor<TV><<<dim3(nbk, nO), 256, 0, st>>>(nC, t, b, wk.part);
+    k_gm_init<<<nO, 512, 0, st>>>(gp, wk.part, nbk);
+}
+
+template <typename TV>
+static void finalResidual(int nC, int nO, int emptyDir, Work& wk, const GmresPtrs& gp, const TV* b, TV* r,
+                          hipStream_t st) {
+    const int nbk = reduceBlocks(nC);
+    k_resid_l1<TV><<<dim3(nbk, nO), 256, 0, st>>>(nC, b, r, wk.part);
+    k_gm_final<<<nO, 320, 0, st>>>(gp, wk.part, nbk, emptyDir);
+}
+
 template <typename TV>
 static void prepareT(const MeshView& m, Work& wk, GmresScalars* g, const void* W, const void* b, void* tmp1,
                      void* tmp2, int blkFp32, const void* blk, const void* dg, hipStream_t st) {
-    const int nC = m.nC;
-    const int nbk = reduceBlocks(nC);
-    k_sum5<TV><<<nbk, 256, 0, st>>>(nC, (const TV*)W, wk.part);
-    k_reduce_final<<<5, 256, 0, st>>>(wk.part, nbk, 5, g->red);
-    k_sub_avg<TV><<<nb(nC, 256), 256, 0, st>>>(nC, (const TV*)W, g->red, (TV*)tmp1);
+    subAverage<TV>(m.nC, 1, wk, g, (const TV*)W, (TV*)tmp1, st);
     launchSpmv(m, blkFp32, sizeof(TV) == 4, blk, dg, tmp1, nullptr, nullptr, tmp2, st);
-    k_normfactor<TV><<<nbk, 256, 0, st>>>(nC, (const TV*)tmp2, (const TV*)b, wk.part);
-    k_reduce_final<<<8, 256, 0, st>>>(wk.part, nbk, 8, g->red);
-    k_gm_init<<<1, 64, 0, st>>>(g);
+    normFactors<TV>(m.nC, 1, wk, GmresPtrs{{g}}, (const TV*)tmp2, (const TV*)b, st);
 }
 
 void gmresPrepare(const MeshView& m, Work& wk, GmresScalars* g, int vecFp32, const void* W, const void* b,
@@ -1633,13 +1708,10 @@ template <typename TV>
 static void updResT(const MeshView& m, Work& wk, GmresScalars* g, int blkFp32, const void* blk, const void* dg,
                     int nDirs, const void* V, void* dW, const void* b, void* r, hipStream_t st) {
     const int nC = m.nC;
-    const int nbk = reduceBlocks(nC);
     const size_t vs = (size_t)5 * nC;
     k_update_sol<TV, TV><<<nb(vs, 256), 256, 0, st>>>(nC, (TV*)dW, (const TV*)V, vs, nDirs, g->yh);
     launchSpmv(m, blkFp32, sizeof(TV) == 4, blk, dg, dW, nullptr, nullptr, r, st);
-    k_resid_l1<TV><<<nbk, 256, 0, st>>>(nC, (const TV*)b, (TV*)r, wk.part);
-    k_reduce_final<<<5, 256, 0, st>>>(wk.part, nbk, 5, g->red);
-    k_gm_final<<<1, 64, 0, st>>>(g, m.emptyDir);
+    finalResidual<TV>(nC, 1, m.emptyDir, wk, GmresPtrs{{g}}, (const TV*)b, (TV*)r, st);
 }
 
 void gmresUpdateAndResidual(const MeshView& m, Work& wk, GmresScalars* g, int vecFp32, int blkFp32,
@@ -1744,29 +1816,23 @@ bool launchSpmvLusgsHB(const MeshView& m, const Levels& L, const HBBlocks& hb, i
     return true;
 }
 
-void sliceSubAverage(const MeshView& m, Work& wk, GmresScalars* g, const double* W, double* out, hipStream_t st) {
-    const int nC = m.nC;
-    const int nbk = reduceBlocks(nC);
-    k_sum5<double><<<nbk, 256, 0, st>>>(nC, W, wk.part);
-    k_reduce_final<<<5, 256, 0, st>>>(wk.part, nbk, 5, g->red);
-    k_sub_avg<double><<<nb(nC, 256), 256, 0, st>>>(nC, W, g->red, out);
+void hbSubAverage(const MeshView& m, int nO, Work& wk, GmresScalars* g, const double* W, double* out,
+                  hipStream_t st) {
+    subAverage<double>(m.nC, nO, wk, g, W, out, st);
 }
 
-void sliceNormFactors(const MeshView& m, Work& wk, GmresScalars* g, const double* t, const double* b,
-                      hipStream_t st) {
-    const int nC = m.nC;
-    const int nbk = reduceBlocks(nC);
-    k_normfactor<double><<<nbk, 256, 0, st>>>(nC, t, b, wk.part);
-    k_reduce_final<<<8, 256, 0, st>>>(wk.part, nbk, 8, g->red);
-    k_gm_init<<<1, 64, 0, st>>>(g);
+void hbNormFactors(const MeshView& m, int nO, Work& wk, const GmresPtrs& gp, const double* t, const double* b,
+                   hipStream_t st) {
+    normFactors<double>(m.nC, nO, wk, gp, t, b, st);
 }
 
-void sliceFinalResidual(const MeshView& m, Work& wk, GmresScalars* g, const double* b, double* r, hipStream_t st) {
-    const int nC = m.nC;
-    const int nbk = reduceBlocks(nC);
-    k_resid_l1<double><<<nbk, 256, 0, st>>>(nC, b, r, wk.part);
-    k_reduce_final<<<5, 256, 0, st>>>(wk.part, nbk, 5, g->red);
-    k_gm_final<<<1, 64, 0, st>>>(g, m.emptyDir);
+void hbFinalResidual(const MeshView& m, int nO, Work& wk, const GmresPtrs& gp, const double* b, double* r,
+                     hipStream_t st) {
+    finalResidual<double>(m.nC, nO, m.emptyDir, wk, gp, b, r, st);
+}
+
+void launchStart(size_t n, const double* b, double* r, double* dW, hipStream_t st) {
+    k_start<<<nb(n, 256), 256, 0, st>>>(n, b, r, dW);
 }
 
 void launchUpdateSolution(size_t nVec, double* dW, const double* V, size_t vstride, int nv, const GmresScalars* g,

@@ -16,9 +16,10 @@ namespace {
 // Primitive/derived cell fields from conserved W after an increment
 // (updateFields.H:7-78), or from (rho, U, T) at initialisation.
 // Wsrc: the state the increment applies to (null: s.W); W0: keeps a copy of it.
-__global__ void k_update(MeshView m, Phys ph, StateView s, const double* __restrict__ dW, int mode,
-                         const double* __restrict__ rho0, const double* __restrict__ U0,
-                         const double* __restrict__ T0, const double* Wsrc, double* W0) {
+__device__ __forceinline__ void updateBody(const MeshView& m, const Phys& ph, const StateView& s,
+                                           const double* __restrict__ dW, int mode,
+                                           const double* __restrict__ rho0, const double* __restrict__ U0,
+                                           const double* __restrict__ T0, const double* Wsrc, double* W0) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= m.nC) return;
     if (s.halt && *s.halt) return;
@@ -91,6 +92,19 @@ __global__ void k_update(MeshView m, Phys ph, StateView s, const double* __restr
     if (s.e) s.e[c] = e;
 }
 
+__global__ void k_update(MeshView m, Phys ph, StateView s, const double* __restrict__ dW, int mode,
+                         const double* __restrict__ rho0, const double* __restrict__ U0,
+                         const double* __restrict__ T0, const double* Wsrc, double* W0) {
+    updateBody(m, ph, s, dW, mode, rho0, U0, T0, Wsrc, W0);
+}
+
+// harmonic-balance instance J0 + blockIdx.y
+__global__ void k_update_hb(const HBInst* inst, int J0, Phys ph, const double* __restrict__ dW) {
+    const int J = J0 + blockIdx.y;
+    const HBInst& I = inst[J];
+    updateBody(I.m, ph, I.s, dW + (size_t)J * 5 * I.m.nC, 1, nullptr, nullptr, nullptr, nullptr, nullptr);
+}
+
 // Boundary values of p, U and T after a state update, on every non-empty,
 // non-coupled boundary face, in the order updateFields.H:90-105 corrects
 // them (p, then U, then T), into StateView::bcV.  fixedValue, zeroGradient
@@ -109,7 +123,7 @@ __global__ void k_update(MeshView m, Phys ph, StateView s, const double* __restr
 // init: the createFields state (createFields.H:51-145): the derived
 // conditions take their initial values from bcInit, valueFraction starts
 // at zero, and phi = Sf & (rho_b U_b).
-__global__ void k_bc_update(MeshView m, Phys ph, StateView s, int init) {
+__device__ __forceinline__ void bcUpdateBody(const MeshView& m, const Phys& ph, const StateView& s, int init) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= m.nB) return;
     if (s.halt && *s.halt) return;
@@ -174,6 +188,13 @@ __global__ void k_bc_update(MeshView m, Phys ph, StateView s, int init) {
         const V3 rUB{rhoB * UB.x, rhoB * UB.y, rhoB * UB.z};
         s.bcPhi[b] = dot(ld3(m.Sf + 3 * (size_t)f), rUB);
     }
+}
+
+__global__ void k_bc_update(MeshView m, Phys ph, StateView s, int init) { bcUpdateBody(m, ph, s, init); }
+
+__global__ void k_bc_update_hb(const HBInst* inst, int J0, Phys ph) {
+    const HBInst& I = inst[J0 + blockIdx.y];
+    bcUpdateBody(I.m, ph, I.s, 0);
 }
 
 // Boundary values of p, U, T and the derived reconstruction fields on
@@ -1152,6 +1173,12 @@ void launchUpdate(const MeshView& m, const Phys& ph, const StateView& s, const d
     k_update<<<nblk(m.nC, 256), 256, 0, st>>>(m, ph, s, dW, mode, rho0, U0, T0, Wsrc, W0);
     // boundary conditions follow every state update (updateFields.H:90-105)
     if (m.nB > 0) k_bc_update<<<nblk(m.nB, 256), 256, 0, st>>>(m, ph, s, mode == 0 ? 1 : 0);
+}
+
+void launchUpdateHB(const HBInst* inst, int J0, int n, const MeshView& m, const Phys& ph, const double* dW,
+                    hipStream_t st) {
+    k_update_hb<<<dim3(nblk(m.nC, 256), n), 256, 0, st>>>(inst, J0, ph, dW);
+    if (m.nB > 0) k_bc_update_hb<<<dim3(nblk(m.nB, 256), n), 256, 0, st>>>(inst, J0, ph);
 }
 
 // The full face records.

@@ -350,9 +350,6 @@ __global__ void k_pack_fields(int nC, const double* fld, double* q) {
     for (int d = 0; d < 3; ++d) q[2 * (size_t)nC + 3 * (size_t)c + d] = f[F_UX + d];
 }
 
-__global__ void k_copy5(const double* a, double* b) {
-    if (threadIdx.x < 5) b[threadIdx.x] = a[threadIdx.x];
-}
 // the same inside a pseudo-step (nothing once the loop has ended)
 __global__ void k_copy5_step(const double* a, double* b, const int* halt) {
     if (threadIdx.x < 5 && !*halt) b[threadIdx.x] = a[threadIdx.x];
@@ -401,9 +398,14 @@ __global__ void k_pseudo_ctl(int* ctl, double* init, const double* dres, double 
 
 // boundLocalTimeStep.H:174-271 evaluated before the state update (as in
 // outerLoop.H:99), so the state compared is the pre-solve state.
-__global__ void k_bound_flag(int nC, double lb, const double* W, double* bad) {
+// I: harmonic-balance instance blockIdx.y's state, bad [nO][5 nC].
+__global__ void k_bound_flag(int nC, double lb, const double* W, double* bad, const HBInst* I = nullptr) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nC) return;
+    if (I) {
+        W = I[blockIdx.y].s.W;
+        bad += (size_t)blockIdx.y * 5 * nC;
+    }
     const double rho = W[c], rE = W[(size_t)nC + c];
     const double ux = W[2 * (size_t)nC + c] / rho, uy = W[3 * (size_t)nC + c] / rho, uz = W[4 * (size_t)nC + c] / rho;
     const double rhoMin = lb * rho;
@@ -413,7 +415,8 @@ __global__ void k_bound_flag(int nC, double lb, const double* W, double* bad) {
     bad[c] = (rho < rhoMin ? 1.0 : 0.0) + ((eT < eMin || eT < 1.0e-15) ? 2.0 : 0.0);
 }
 
-// The harmonic-balance instance J's phase-lagged far test: rho_ is lagged
+// Harmonic-balance instances J + blockIdx.y (I), and their phase-lagged far
+// test where there are phase-lagged patches (side): rho_ is lagged
 // over the instances as they stand (those before J already updated,
 // outerLoop.H:221-229), rhoMin, eTemp and eMin are not (their far cell's
 // bits).
@@ -433,6 +436,11 @@ struct BoundLag {
 __global__ void k_bound_apply(MeshView m, const double* bad, double* co, const int* halt, BoundLag bl = {}) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= m.nC || (halt && *halt)) return;
+    bl.J += blockIdx.y;
+    if (bl.I) {
+        bad += (size_t)bl.J * 5 * m.nC;
+        co = bl.I[bl.J].s.pseudoCo;
+    }
     double f = 1.0;
     const bool badC = bad[c] != 0.0;
     const int len = m.rowLen[c];
@@ -675,8 +683,7 @@ int gmresSolve(icsf_case* c, const double* W, const double* b, int& nIter) {
     {
         Timed t(c, 5);
         gmresPrepare(m, c->wk, c->g, 0, W, b, c->t1, c->t2, c->blkFp32, c->blk, c->dg, c->st);
-        launchZero(vs, 0, c->dW, c->st);
-        launchCopy(vs, 0, b, c->r, c->st);
+        launchStart(vs, b, c->r, c->dW, c->st);
     }
     nIter = 0;
     for (;;) {
@@ -897,8 +904,7 @@ int fgmresSolve(icsf_case* c, const double* W, const double* b, int& nIter) {
     {
         Timed t(c, 5);
         gmresPrepare(m, c->wk, c->g, 0, W, b, c->t1, c->t2, c->blkFp32, c->blk, c->dg, c->st);
-        launchZero(vs, 0, c->dW, c->st);
-        launchCopy(vs, 0, b, c->r, c->st);
+        launchStart(vs, b, c->r, c->dW, c->st);
     }
     // z = M^-1 v
     auto precond = [c, vs](const double* v, double* z) {
@@ -1161,10 +1167,12 @@ __global__ void k_phase_lag_hb(const HBInst* __restrict__ I, int nO, int nCyc, c
 }
 
 // SER over all instances (outerLoop.H:30-66): dres = [init nO*5][prev nO*5]
-__global__ void k_hb_ser(int nC, int nO, double* co, const double* dres, double coIncr, double coDecr, double coMin,
-                         double coMax) {
+// (instance blockIdx.y's Courant numbers)
+__global__ void k_hb_ser(int nC, int nO, const HBInst* I, const double* dres, double coIncr, double coDecr,
+                         double coMin, double coMax) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nC) return;
+    double* co = I[blockIdx.y].s.pseudoCo;
     double nI = 0, nP = 0;
     for (int J = 0; J < nO; ++J) {
         const double* a = dres + 5 * J;
@@ -1177,6 +1185,12 @@ __global__ void k_hb_ser(int nC, int nO, double* co, const double* dres, double 
     double v = co[c] * ratio;
     v = fmax(fmin(v, coMax), coMin);
     co[c] = v;
+}
+
+// the instances' initial residuals, [nO][5]
+__global__ void k_hb_init_residuals(ResPtrs q, int nO, double* dres) {
+    const int i = threadIdx.x;
+    if (i < 5 * nO) dres[i] = q.r[i / 5][i % 5];
 }
 
 __global__ void k_copyn(int n, const double* a, double* b) {
@@ -1227,6 +1241,12 @@ int hbJacobianStage(icsf_hb* h, bool cellSums = false) {
     return ICSF_OK;
 }
 
+GmresPtrs hbScalars(icsf_hb* h) {
+    GmresPtrs gp{};
+    for (int J = 0; J < h->nO; ++J) gp.g[J] = h->gJ[J];
+    return gp;
+}
+
 // the instances' residuals into host (pinned, [nO][10]) after the queued work
 void hbQueueResiduals(icsf_hb* h, double* host) {
     ResPtrs q{};
@@ -1244,11 +1264,11 @@ void hbReadResiduals(icsf_hb* h, std::vector<double>& res) {
 int hbSolve(icsf_hb* h, const double* b, int& nIter) {
     const MeshView& m = h->inst[0]->mv;
     const size_t vs = (size_t)5 * m.nC, vA = vs * h->nO;
-    for (int J = 0; J < h->nO; ++J) sliceSubAverage(m, h->wk, h->gJ[J], h->Wall + J * vs, h->t1 + J * vs, h->st);
+    const GmresPtrs gp = hbScalars(h);
+    hbSubAverage(m, h->nO, h->wk, h->g, h->Wall, h->t1, h->st);
     launchSpmvHB(m, h->hbb, 0, h->t1, nullptr, nullptr, h->t2, h->st);
-    for (int J = 0; J < h->nO; ++J) sliceNormFactors(m, h->wk, h->gJ[J], h->t2 + J * vs, b + J * vs, h->st);
-    launchZero(vA, 0, h->dW, h->st);
-    launchCopy(vA, 0, b, h->r, h->st);
+    hbNormFactors(m, h->nO, h->wk, gp, h->t2, b, h->st);
+    launchStart(vA, b, h->r, h->dW, h->st);
     nIter = 0;
     for (;;) {
         GmresArgs a{&m, &h->mesh->lev, &h->wk, h->g, h->nDirs, 0, h->orth, 0, nullptr, nullptr, h->rD, nullptr,
@@ -1265,7 +1285,7 @@ int hbSolve(icsf_hb* h, const double* b, int& nIter) {
         gmresCycle(a, 0, h->st);
         launchUpdateSolution((size_t)m.nC * h->nO, h->dW, h->V, vA, h->nDirs, h->g, h->st);
         launchSpmvHB(m, h->hbb, 0, h->dW, nullptr, nullptr, h->r, h->st);
-        for (int J = 0; J < h->nO; ++J) sliceFinalResidual(m, h->wk, h->gJ[J], b + J * vs, h->r + J * vs, h->st);
+        hbFinalResidual(m, h->nO, h->wk, gp, b, h->r, h->st);
         ++nIter;
         if (nIter < h->minIter) continue;
         if (nIter >= h->maxIter) break;
@@ -1296,11 +1316,11 @@ int hbSolveMixed(icsf_hb* h, const double* b, int& nIter) {
     const MeshView& m = h->inst[0]->mv;
     const size_t vs = (size_t)5 * m.nC, vA = vs * h->nO;
     const int nVec = m.nC * h->nO;
-    for (int J = 0; J < h->nO; ++J) sliceSubAverage(m, h->wk, h->gJ[J], h->Wall + J * vs, h->t1 + J * vs, h->st);
+    const GmresPtrs gp = hbScalars(h);
+    hbSubAverage(m, h->nO, h->wk, h->g, h->Wall, h->t1, h->st);
     launchSpmvHB(m, h->hbb, 0, h->t1, nullptr, nullptr, h->t2, h->st);
-    for (int J = 0; J < h->nO; ++J) sliceNormFactors(m, h->wk, h->gJ[J], h->t2 + J * vs, b + J * vs, h->st);
-    launchZero(vA, 0, h->dW, h->st);
-    launchCopy(vA, 0, b, h->r, h->st);
+    hbNormFactors(m, h->nO, h->wk, gp, h->t2, b, h->st);
+    launchStart(vA, b, h->r, h->dW, h->st);
     auto precond = [h, &m, vA, nVec](const double* v, double* z) {
         launchConvert(vA, 0, v, h->r32, h->st);
         if (h->innerDirs == 0) {
@@ -1331,7 +1351,7 @@ int hbSolveMixed(icsf_hb* h, const double* b, int& nIter) {
         fgmresCycle(a, h->st);
         launchUpdateSolution((size_t)nVec, h->dW, h->Z, vA, h->nDirs, h->g, h->st);
         launchSpmvHB(m, h->hbb, 0, h->dW, nullptr, nullptr, h->r, h->st);
-        for (int J = 0; J < h->nO; ++J) sliceFinalResidual(m, h->wk, h->gJ[J], b + J * vs, h->r + J * vs, h->st);
+        hbFinalResidual(m, h->nO, h->wk, gp, b, h->r, h->st);
         ++nIter;
         if (nIter < h->minIter) continue;
         if (nIter >= h->maxIter) break;
@@ -1360,9 +1380,8 @@ int hbPseudoStep(icsf_hb* h) {
     h->corr++;
     if (h->haveInit) {
         if (h->corr != 1 && h->havePrev)
-            for (int J = 0; J < h->nO; ++J)
-                k_hb_ser<<<nblk(m.nC, 256), 256, 0, h->st>>>(m.nC, h->nO, h->inst[J]->sv.pseudoCo, h->dres,
-                                                             c0->coIncr, c0->coDecr, c0->coMin, c0->coMax);
+            k_hb_ser<<<dim3(nblk(m.nC, 256), h->nO), 256, 0, h->st>>>(m.nC, h->nO, h->dInst, h->dres, c0->coIncr,
+                                                                      c0->coDecr, c0->coMin, c0->coMax);
         k_copyn<<<1, 5 * HB_MAXO, 0, h->st>>>(5 * h->nO, h->dres, h->dres + 5 * h->nO);
         h->havePrev = true;
     }
@@ -1372,22 +1391,33 @@ int hbPseudoStep(icsf_hb* h) {
     int nIter = 0;
     if (h->solver == 1) RC(hbSolveMixed(h, h->ball, nIter));
     else RC(hbSolve(h, h->ball, nIter));
-    for (int J = 0; J < h->nO; ++J) k_copy5<<<1, 64, 0, h->st>>>(gmresResidualsDevice(h->gJ[J]), h->dres + 5 * J);
-    h->haveInit = true;
-    for (int J = 0; J < h->nO; ++J) {
-        icsf_case* c = h->inst[J];
-        if (c->localTS && c->bounding) {
-            BoundLag bl;
-            if (h->dplFar) bl = BoundLag{h->dInst, h->nO, J, h->dplSide, h->dplD, c->lowerBound};
-            k_bound_flag<<<nblk(m.nC, 256), 256, 0, h->st>>>(m.nC, c->lowerBound, c->sv.W, c->fac);
-            k_bound_apply<<<nblk(m.nC, 256), 256, 0, h->st>>>(c->mv, c->fac, c->sv.pseudoCo, nullptr, bl);
-        }
-        // the instance's own view: its boundary conditions and values (the
-        // instants' inflow total pressures differ)
-        launchUpdate(c->mv, c->ph, c->sv, h->dW + J * vs, 1, nullptr, nullptr, nullptr, h->st);
-        // the residual and the matrix belong to the state before the update
-        c->haveResidual = c->assembled = false;
+    {
+        ResPtrs q{};
+        for (int J = 0; J < h->nO; ++J) q.r[J] = gmresResidualsDevice(h->gJ[J]);
+        k_hb_init_residuals<<<1, 5 * HB_MAXO, 0, h->st>>>(q, h->nO, h->dres);
     }
+    h->haveInit = true;
+    // all instances in one launch each, as the solve's start and end (small
+    // launches of 4.5 us, 105 of them with 7 instants one by one: 32x32x24 cells,
+    // a pseudo-step 3.05 -> 2.79 ms); but with phase-lagged patches the bound of
+    // an instance reads the updated states of those before it
+    const bool bound = c0->localTS && c0->bounding;
+    const dim3 gc(nblk(m.nC, 256), h->nO);
+    if (bound)
+        k_bound_flag<<<gc, 256, 0, h->st>>>(m.nC, c0->lowerBound, nullptr, h->t1, h->dInst);
+    const int n = bound && h->dplFar ? 1 : h->nO;
+    for (int J = 0; J < h->nO; J += n) {
+        if (bound) {
+            BoundLag bl{h->dInst, h->nO, J};
+            if (h->dplFar) bl = BoundLag{h->dInst, h->nO, J, h->dplSide, h->dplD, c0->lowerBound};
+            k_bound_apply<<<dim3(gc.x, n), 256, 0, h->st>>>(m, h->t1, nullptr, nullptr, bl);
+        }
+        // each instance's own view: its boundary conditions and values (the
+        // instants' inflow total pressures differ)
+        launchUpdateHB(h->dInst, J, n, m, c0->ph, h->dW, h->st);
+    }
+    // the residual and the matrix belong to the state before the update
+    for (icsf_case* c : h->inst) c->haveResidual = c->assembled = false;
     h->assembled = false;
     return ICSF_OK;
 }
