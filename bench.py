@@ -86,14 +86,14 @@ NGEN = 10  # generator values per off-diagonal block (jacobianStorage generators
 
 def algorithmic_bytes_fused(nC, nI, p, q, gen=True):
     """Per-group algorithmic bytes of the fused Arnoldi operator (one group
-    per Arnoldi step: SpMV of the colour-0 rows; SpMV + forward sweep +
-    first backward level of the colour-1 rows; backward sweep of the
-    colour-0 rows).  Off-diagonal blocks (10 generators each with generator
+    per Arnoldi step: SpMV of the colour-0 rows, leaving t0 = x0 - rD0 z0;
+    SpMV + forward sweep + first backward level of the colour-1 rows, one
+    gather of t0; backward sweep of the colour-0 rows).  Off-diagonal blocks (10 generators each with generator
     storage, else 25 entries): every block of a colour-0 row twice, of a
     colour-1 row once; diagonal blocks once; column indices per block read;
-    vectors: x twice, y0 once more by the colour-1 rows, y once by the last
-    pass, writes of y, the basis vector and the final colour-0 rows; rD
-    twice for colour 0 (n0 = n1 = nC/2 on these meshes)."""
+    vectors: x read by phase 0, x1 and t0 by phase 1, y by phase 2, writes
+    of y, t0, the basis vector and the final colour-0 rows; rD twice for
+    colour 0 (n0 = n1 = nC/2 on these meshes)."""
     per = NGEN if gen else 25
     return (3 * nI * per + nC * 25) * p + 3 * nI * 4 + 30 * q * nC + 12 * nC
 
@@ -712,8 +712,7 @@ def main():
                        for f, r in (("fp64", r64), ("mixed", rmx))}},
         "roofline": {"bound": "hbm",
                      "kernel": ("fused Arnoldi operator, FP64 form, off-diagonal blocks as generators: "
-                                "k_spmv_cells<double,double,false,true> + k_spmv_cells<double,double,true,true> "
-                                "+ k_lusgs_bwd<double,double,true> (one group per Arnoldi step, timed as a "
+                                "k_op<double> phases 0, 1 and 2 (one group per Arnoldi step, timed as a "
                                 "group)") if fused else
                                "k_spmv<double,double> (block SpMV, FP64 form)",
                      "achieved": round(ach / 1e9, 1), "peak": HBM_PEAK / 1e9, "unit": "GB/s",

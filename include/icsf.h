@@ -299,7 +299,7 @@ int icsf_get_interface_blocks(icsf_case* c, double* blocks);
 /* Launch parameters in use (no counterpart in the reference): params[0..9]
  * = workgroup size of the Arnoldi-operator row kernels (SpMV, LU-SGS),
  * of the face-terms kernel, of the gradient and cell-residual kernels, of
- * the Jacobian rows; basis vectors per CGS projection pass; 1 if the
+ * the Jacobian rows; basis vectors per projection workgroup; 1 if the
  * autotuner has run; then the register budget (0 the compiler's choice,
  * 1 at most 128 VGPRs for 4 waves per SIMD, 2 at most 168 for 3) of the
  * operator, face-terms,
