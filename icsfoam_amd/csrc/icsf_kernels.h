@@ -40,6 +40,9 @@ constexpr int kSweepLevelCells = 8192;
 // application and 2.43 ms in one, 17 + 17 levels are well ahead (above).
 constexpr int kSweepMinLevels = 24;
 
+// Incomplete polls after which one wait of the dataflow sweep gives up.
+constexpr int kSweepPolls = 1 << 21;
+
 // Scratch for two-stage reductions, and of the dataflow sweep: the forward
 // and the final values [5][nC], the levels' finished chunks and the next chunk
 // to draw, the case's error flags (swF null: none).
@@ -47,6 +50,7 @@ struct Work {
     double* part = nullptr;  // [kPartSize]
     void *swF = nullptr, *swO = nullptr;
     int *swDone = nullptr, *err = nullptr;
+    int swLimit = kSweepPolls;
 };
 
 // 1024 workgroups' partials of the 2 KMAX projection values of one step, then

@@ -634,10 +634,12 @@ __global__ void __launch_bounds__(256) k_lusgs_hb(MeshView m, HBBlocks hb, const
 // A row reads only rows of earlier levels, i.e. of lower chunks.  A chunk is
 // drawn by a running wavefront, which finishes the chunks it drew in order,
 // so the lowest unfinished chunk always runs, however few of the wavefronts
-// the GPU has room for.  Every wait gives up after kSweepSpins loads (seconds; the longest
-// sweep takes milliseconds) and sets ERR_FLAG_SWEEP, as does every later one.
+// the GPU has room for.  Each wait counts the polls that found it incomplete
+// and gives up past `limit` of them (kSweepPolls: seconds, while a wait is
+// for at most the grid's chunks ahead of it, milliseconds, however many
+// levels the sweep has); the wavefront then sets ERR_FLAG_SWEEP and ends, and
+// so does every wavefront that waits for its chunk.
 // Same operations and order per row as lusgsFwdRow / lusgsBwdRow.
-constexpr int kSweepSpins = 1 << 21;
 
 __device__ __forceinline__ unsigned long long sweepSentinel(double) { return 0x7FF4DEADBEEF5A5Aull; }
 __device__ __forceinline__ unsigned sweepSentinel(float) { return 0x7FA5A5A5u; }
@@ -669,17 +671,16 @@ __global__ void __launch_bounds__(64) k_sweep(MeshView m, const TB* __restrict__
                                                TV* r, TV* f, TV* o, const int* __restrict__ chunkCells,
                                                const int* __restrict__ chunkLevel,
                                                const int* __restrict__ levelChunks, int nFwd, int nChunks,
-                                               int nFwdLevels, int* done, int* next, int* err) {
+                                               int nFwdLevels, int limit, int* done, int* next, int* err) {
     constexpr int UN = 3;  // slots whose blocks and values are in flight together
     typedef TV A;
     const size_t nC = m.nC;
     const int lane = threadIdx.x & 63;
     const auto sent = sweepSentinel((TV)0);
-    int spins = 0;
     // the values at q (5 of them nC apart) of every lane with on set
     auto wait5 = [&](const TV* q, bool on, A (&v)[5]) {
         bool ready = !on;
-        for (;;) {
+        for (int polls = 0;;) {
             if (!ready) {
                 ready = true;
 #pragma unroll
@@ -690,7 +691,7 @@ __global__ void __launch_bounds__(64) k_sweep(MeshView m, const TB* __restrict__
                 }
             }
             if (__all(ready)) return true;
-            if (++spins > kSweepSpins) return false;
+            if (++polls > limit) return false;
         }
     };
     auto draw = [&]() {
@@ -717,9 +718,10 @@ __global__ void __launch_bounds__(64) k_sweep(MeshView m, const TB* __restrict__
             begun = true;
             if (lev >= 2) {
                 const int want = levelChunks[lg - 2];
+                int polls = 0;
                 while (__builtin_amdgcn_readfirstlane(
                            __hip_atomic_load(done + lg - 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) < want) {
-                    if (++spins > kSweepSpins) { ok = false; return; }
+                    if (++polls > limit) { ok = false; return; }
                     __builtin_amdgcn_s_sleep(8);
                 }
             }
@@ -761,7 +763,7 @@ __global__ void __launch_bounds__(64) k_sweep(MeshView m, const TB* __restrict__
             unsigned miss = 0;
 #pragma unroll
             for (int u = 0; u < UN; ++u) miss |= ok && k + u < n ? 1u << u : 0u;
-            while (__any(miss)) {
+            for (int polls = 0; __any(miss);) {
 #pragma unroll
                 for (int u = 0; u < UN; ++u)
                     if (miss & (1u << u)) {
@@ -774,7 +776,7 @@ __global__ void __launch_bounds__(64) k_sweep(MeshView m, const TB* __restrict__
                         }
                         if (got) miss &= ~(1u << u);
                     }
-                if (++spins > kSweepSpins) { ok = false; break; }
+                if (__any(miss) && ++polls > limit) { ok = false; break; }
             }
 #pragma unroll
             for (int u = 0; u < UN; ++u) {
@@ -1506,8 +1508,8 @@ static void sweepG(const MeshView& m, const Levels& L, const Work& wk, const voi
     k_sweep_init<TV><<<nb(n, 256), 256, 0, st>>>(n, nLev, (TV*)wk.swF, (TV*)wk.swO, wk.swDone);
     const int nWg = nCh < kSweepWaves ? nCh : kSweepWaves;
     k_sweep<TB, TV, GEN><<<nWg, 64, 0, st>>>(m, (const TB*)blk, rD, (TV*)r, (TV*)wk.swF, (TV*)wk.swO, L.chunkCells,
-                                             L.chunkLevel, L.levelChunks, L.nFwdChunks, nCh, L.nFwd, wk.swDone,
-                                             wk.swDone + nLev, wk.err);
+                                             L.chunkLevel, L.levelChunks, L.nFwdChunks, nCh, L.nFwd, wk.swLimit,
+                                             wk.swDone, wk.swDone + nLev, wk.err);
 }
 
 template <typename TB, typename TV>

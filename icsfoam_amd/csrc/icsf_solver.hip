@@ -2425,6 +2425,15 @@ int icsf_get_tuning(icsf_case* c, int* params) {
     return ICSF_OK;
 }
 
+// a captured step holds the launch parameters it was captured with
+static int dropGraph(icsf_case* c) {
+    if (!c->gexec) return ICSF_OK;
+    HIPCHK(hipStreamSynchronize(c->st));
+    (void)hipGraphExecDestroy(c->gexec);
+    c->gexec = nullptr;
+    return ICSF_OK;
+}
+
 int icsf_set_tuning(icsf_case* c, const int* params) {
     if (!c || !params) return fail(ICSF_ERR_ARG, "icsf_set_tuning: NULL argument");
     const auto wg = [](int b) { return b == 64 || b == 128 || b == 256; };
@@ -2439,13 +2448,16 @@ int icsf_set_tuning(icsf_case* c, const int* params) {
     m.bsOp = params[0]; m.bsFace = params[1]; m.bsCell = params[2]; m.bsJac = params[3]; m.mdCh = params[4];
     m.occOp = params[6]; m.occFace = params[7]; m.occCell = params[8]; m.occJac = params[9];
     c->tuned = true;
-    // a captured step holds the old launch parameters
-    if (c->gexec) {
-        HIPCHK(hipStreamSynchronize(c->st));
-        (void)hipGraphExecDestroy(c->gexec);
-        c->gexec = nullptr;
-    }
-    return ICSF_OK;
+    return dropGraph(c);
+}
+
+// The limit of the dataflow sweep's waits (Work::swLimit; negative:
+// the default).  Not part of the interface: with a small one, tests of the
+// failure path have a sweep give up.
+int icsf_test_sweep_limit(icsf_case* c, int polls) {
+    if (!c) return fail(ICSF_ERR_ARG, "NULL case");
+    c->wk.swLimit = polls < 0 ? kSweepPolls : polls;
+    return dropGraph(c);
 }
 
 int icsf_get_interface_blocks(icsf_case* c, double* blocks) {

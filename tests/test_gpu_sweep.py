@@ -3,12 +3,14 @@ against the oracle's sequential sweep, bit for bit: RCM and file order, chunks
 of one row and of a wavefront, a polyhedral number of levels, generator and
 block storage, FP32 vectors through the mixed solve, and repeated
 applications (the values of one must not serve the next)."""
+import ctypes
 import dataclasses
 
 import numpy as np
 import pytest
 
 from icsfoam_amd import cases, dbnsCase
+from icsfoam_amd._lib import check, lib
 from icsfoam_amd.mesh import prepare_case
 from oracle.oracle import OracleCase
 
@@ -58,3 +60,28 @@ def test_many_level_pseudo_steps(form):
     assert rel_err(g.fields()["W"], o.fields()["W"]) < tol
     if form == "fp64":
         assert abs(h - ho).max() < 1e-8 * abs(ho).max()
+
+
+def _sweep_limit(g, polls):
+    """Polls after which one wait of the sweep gives up (negative: the
+    default); a test entry beside the interface."""
+    f = lib().icsf_test_sweep_limit
+    f.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    check(f(g._h, polls))
+
+
+def test_wait_limit_is_per_wait():
+    """A chain of single-cell levels: every wavefront draws 157 of the 40 000
+    chunks and waits each time for at most the 256 chunks in flight (some 500
+    polls; the whole sweep some 80 000).  A limit of 20 000 polls per wait
+    must not end it."""
+    print("[sweep limit]", flush=True)
+    c = _case((20000, 1, 1), "file")
+    g, o = dbnsCase.from_case(c), OracleCase(c)
+    assert g.mesh.nFwdLevels == g.nCells
+    for q in (g, o):
+        q.residual()
+        q.createJacobian()
+    _sweep_limit(g, 20000)
+    x = np.random.default_rng(1).standard_normal((5, g.nCells))
+    np.testing.assert_array_equal(g.precondition(x), o.precondition(x))
