@@ -493,6 +493,17 @@ int caseErrors(icsf_case* c) {
     return flagError(e);
 }
 
+// Waits for the case's stream and reports a sweep that gave up; the other
+// flags stay for the calls that report them.
+int sweepErrors(icsf_case* c) {
+    if (c->wk.swF) HIPCHK(hipMemcpyAsync(c->hErr, c->derr, sizeof(int), hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipStreamSynchronize(c->st));
+    if (!c->wk.swF || !(*c->hErr & ERR_FLAG_SWEEP)) return ICSF_OK;
+    *c->hErr &= ~ERR_FLAG_SWEEP;
+    HIPCHK(hipMemcpy(c->derr, c->hErr, sizeof(int), hipMemcpyHostToDevice));
+    return flagError(ERR_FLAG_SWEEP);
+}
+
 // ---- settings -----------------------------------------------------------
 int readSettings(icsf_case* c, const char* thermo, const char* schemes, const char* solution) {
     Dict td, sd, fd;
@@ -2540,7 +2551,7 @@ int icsf_precondition(icsf_case* c, double* r) {
     HIPCHK(hipMemcpyAsync(c->t1, r, vs * 8, hipMemcpyHostToDevice, c->st));
     applyPrecond(c, 0, c->t1);
     HIPCHK(hipMemcpyAsync(r, c->t1, vs * 8, hipMemcpyDeviceToHost, c->st));
-    return caseErrors(c);
+    return sweepErrors(c);
 }
 
 int icsf_solve_for_incr(icsf_case* c, const double* W, const double* b, double* dW, double* residuals,
@@ -2563,7 +2574,7 @@ int icsf_solve_for_incr(icsf_case* c, const double* W, const double* b, double* 
     }
     int it = 0;
     RC(solveStage(c, dWsrc, db, it));
-    HIPCHK(hipStreamSynchronize(c->st));
+    RC(sweepErrors(c));
     if (dW) HIPCHK(hipMemcpy(dW, c->dW, vs * 8, hipMemcpyDeviceToHost));
     if (residuals) gmresReadResiduals(c->g, residuals, c->st);
     if (nIter) *nIter = it;

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from icsfoam_amd import cases, dbnsCase
-from icsfoam_amd._lib import check, lib
+from icsfoam_amd._lib import ERR_HIP, IcsfError, check, lib
 from icsfoam_amd.mesh import prepare_case
 from oracle.oracle import OracleCase
 
@@ -85,3 +85,35 @@ def test_wait_limit_is_per_wait():
     _sweep_limit(g, 20000)
     x = np.random.default_rng(1).standard_normal((5, g.nCells))
     np.testing.assert_array_equal(g.precondition(x), o.precondition(x))
+
+
+def _gives_up(call):
+    with pytest.raises(IcsfError, match="sweep") as e:
+        call()
+    assert e.value.code == ERR_HIP
+
+
+def test_sweep_that_gives_up_is_reported():
+    """A sweep whose waits may not wait (limit 0) gives up: every call that
+    ran it reports that, none hands its failure to a later call, and with the
+    limit back the same calls give the same bits as before."""
+    print("[sweep gives up]", flush=True)
+    c = _case((16, 16, 9), "file")
+    g = dbnsCase.from_case(c)
+    g.residual()
+    g.createJacobian()
+    x = np.random.default_rng(1).standard_normal((5, g.nCells))
+    p, (dW, res, _) = g.precondition(x), g.solveForIncr()
+    _sweep_limit(g, 0)
+    _gives_up(g.solveForIncr)
+    _sweep_limit(g, -1)
+    np.testing.assert_array_equal(g.precondition(x), p)
+    _sweep_limit(g, 0)
+    _gives_up(lambda: g.precondition(x))
+    _sweep_limit(g, -1)
+    d, r, _ = g.solveForIncr()
+    np.testing.assert_array_equal(d, dW)
+    np.testing.assert_array_equal(r, res)
+    _sweep_limit(g, 0)
+    _gives_up(lambda: g.pseudo_steps(4))  # the last ones replayed
+    _gives_up(lambda: g.pseudo_time_loop(2))
