@@ -474,11 +474,12 @@ __global__ void k_fill(int n, double v, double* x) {
 
 int nblk(size_t n, int b) { return (int)((n + b - 1) / b); }
 
-// Device error flags as a return code: a non-finite state first, then a
+// Device error flags as a return code: a sweep that gave up first (what
+// follows from its values may be non-finite), then a non-finite state, then a
 // diagonal whose LU-SGS coefficient fell below VSMALL (lusgs.C:119-123).
 int flagError(int any) {
-    if (any & ERR_FLAG_NONFINITE) return fail(ICSF_ERR_NONFINITE, "non-finite conserved state after the update");
     if (any & ERR_FLAG_SWEEP) return fail(ICSF_ERR_HIP, "LU-SGS sweep: a wait ended at its limit");
+    if (any & ERR_FLAG_NONFINITE) return fail(ICSF_ERR_NONFINITE, "non-finite conserved state after the update");
     if (any & ERR_FLAG_DIAG) return fail(ICSF_ERR_ZERO_DIAG, "All diagonals of coupledMatrix are zero.");
     return ICSF_OK;
 }

@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 from icsfoam_amd import cases, dbnsCase
-from icsfoam_amd._lib import ERR_HIP, IcsfError, check, lib
+from icsfoam_amd._lib import ERR_HIP, ERR_NONFINITE, IcsfError, check, lib
 from icsfoam_amd.mesh import prepare_case
 from oracle.oracle import OracleCase
 
@@ -117,3 +117,22 @@ def test_sweep_that_gives_up_is_reported():
     _sweep_limit(g, 0)
     _gives_up(lambda: g.pseudo_steps(4))  # the last ones replayed
     _gives_up(lambda: g.pseudo_time_loop(2))
+
+
+def test_sweep_that_gives_up_is_the_cause_reported():
+    """With an inflow whose |U|^2 overflows the state turns non-finite too:
+    the sweep is the cause reported, and without it the state is."""
+    print("[sweep gives up, non-finite]", flush=True)
+    c = _case((16, 16, 9), "file")
+    i = [p.name for p in c.mesh.patches].index("inlet")
+    U = np.zeros((c.mesh.patches[i].size, 3))
+    U[:, 0] = 1e200
+    bcs = list(c.bcs)
+    bcs[i] = dataclasses.replace(bcs[i], U_val=U)
+    g = dbnsCase.from_case(dataclasses.replace(c, bcs=bcs))
+    _sweep_limit(g, 0)
+    _gives_up(lambda: g.pseudo_steps(2))
+    g = dbnsCase.from_case(dataclasses.replace(c, bcs=bcs))
+    with pytest.raises(IcsfError) as e:
+        g.pseudo_steps(2)
+    assert e.value.code == ERR_NONFINITE
