@@ -204,6 +204,7 @@ struct icsf_case {
     int* derr = nullptr;
     int* hErr = nullptr;  // pinned: the error flags as read back by caseErrors
     double* hRes = nullptr;  // pinned: the residuals of up to kResBatch steps
+    int failStep = -1;       // icsf_test_fail_step
     // pseudo-time loop control (pseudotimeControl): device block [NCTL],
     // stored initial residuals [5]; criteria from fvSolution pseudoTime
     // (pseudoTol / pseudoTolRel NaN when absent)
@@ -1030,6 +1031,27 @@ int vjpDevice(icsf_case* c, const double* W, const double* v, double* gW, double
     return caseErrors(c);
 }
 
+// nSteps pseudo-steps with n residuals each into out (null: none).  queue
+// stores a step's residuals in pinned memory after its kernels, `batch` steps
+// without a wait, so that the steps follow each other on the device.  A step
+// that fails ends the run; those before it keep their residuals.
+template <typename Step, typename Queue>
+int stepHistory(int nSteps, int batch, size_t n, double* out, double* pinned, hipStream_t st, Step step,
+                Queue queue) {
+    int rc = ICSF_OK, have = 0;
+    for (int i = 0; i < nSteps && !rc; ++i) {
+        rc = step(i);
+        if (!rc && out) queue(pinned + have++ * n);
+        if (have == batch || (have && (rc || i == nSteps - 1))) {
+            const hipError_t e = hipStreamSynchronize(st);
+            if (!rc) HIPCHK(e);
+            if (e == hipSuccess) std::copy(pinned, pinned + have * n, out + (size_t)(rc ? i - have : i + 1 - have) * n);
+            have = 0;
+        }
+    }
+    return rc;
+}
+
 }  // namespace
 
 
@@ -1057,6 +1079,7 @@ struct icsf_hb {
     int* derr = nullptr;
     int* hErr = nullptr;     // pinned, as icsf_case's
     double* hRes = nullptr;  // pinned: [kResBatch][nO][10]
+    int failStep = -1;       // icsf_test_fail_step
     HBInst* dInst = nullptr;  // per-instance views, blockIdx.y of the batched launches
     GmresScalars* g = nullptr;
     std::vector<GmresScalars*> gJ;
@@ -2472,6 +2495,14 @@ int icsf_test_sweep_limit(icsf_case* c, int polls) {
     return dropGraph(c);
 }
 
+// The next icsf_pseudo_steps / icsf_hb_pseudo_steps fails at step `step`
+// (from 0).  Not part of the interface: for tests of the failure path.
+int icsf_test_fail_step(icsf_case* c, icsf_hb* h, int step) {
+    if (c) c->failStep = step;
+    if (h) h->failStep = step;
+    return ICSF_OK;
+}
+
 int icsf_get_interface_blocks(icsf_case* c, double* blocks) {
     if (!c || !blocks) return fail(ICSF_ERR_ARG, "icsf_get_interface_blocks: NULL argument");
     if (!c->assembled) return fail(ICSF_ERR_STATE, "Jacobian not assembled");
@@ -2588,22 +2619,17 @@ int icsf_pseudo_steps(icsf_case* c, int nSteps, double* residuals, int* nIter) {
     // flags left by earlier calls (e.g. a state handed to the VJP) do not
     // belong to these steps
     k_flags<<<1, 64, 0, c->st>>>(FlagPtrs{{c->derr}, 1}, nullptr);
-    for (int i = 0; i < nSteps; ++i) {
-        int it = 1;
-        if (graphable(c)) RC(graphStep(c));
-        else RC(pseudoStep(c, it));
-        if (residuals) {
-            // collected without a wait per step, so that the steps follow
-            // each other on the device
-            const int k = i % kResBatch;
-            k_store_residuals<<<1, 64, 0, c->st>>>(ResPtrs{{gmresResidualsDevice(c->g)}}, 1, c->hRes + 10 * k);
-            if (k == kResBatch - 1 || i == nSteps - 1) {
-                HIPCHK(hipStreamSynchronize(c->st));
-                std::copy(c->hRes, c->hRes + 10 * (k + 1), residuals + 10 * (size_t)(i - k));
-            }
-        }
-        if (nIter) nIter[i] = it;
-    }
+    RC(stepHistory(
+        nSteps, kResBatch, 10, residuals, c->hRes, c->st,
+        [&](int i) {
+            int it = 1;
+            if (c->failStep >= 0 && c->failStep-- == 0) return fail(ICSF_ERR_HIP, "icsf_test_fail_step");
+            if (graphable(c)) RC(graphStep(c));
+            else RC(pseudoStep(c, it));
+            if (nIter) nIter[i] = it;
+            return (int)ICSF_OK;
+        },
+        [&](double* host) { k_store_residuals<<<1, 64, 0, c->st>>>(ResPtrs{{gmresResidualsDevice(c->g)}}, 1, host); }));
     HIPCHK(hipGetLastError());
     const int rc = caseErrors(c);
     resolveEvents(c);
@@ -3072,18 +3098,13 @@ int icsf_hb_pseudo_steps(icsf_hb* h, int nSteps, double* residuals) {
     // one step's residuals may be in use by the solver's own stop test
     // (maxIter > 1, hbReadResiduals): those steps are read one by one
     const int batch = h->maxIter == 1 && h->minIter <= 1 ? kResBatch : 1;
-    for (int i = 0; i < nSteps; ++i) {
-        if (hbGraphable(h)) RC(hbGraphStep(h));
-        else RC(hbPseudoStep(h));
-        if (residuals) {
-            const int k = i % batch;
-            hbQueueResiduals(h, h->hRes + k * nr);
-            if (k == batch - 1 || i == nSteps - 1) {
-                HIPCHK(hipStreamSynchronize(h->st));
-                std::copy(h->hRes, h->hRes + (k + 1) * nr, residuals + (size_t)(i - k) * nr);
-            }
-        }
-    }
+    RC(stepHistory(
+        nSteps, batch, nr, residuals, h->hRes, h->st,
+        [&](int) {
+            if (h->failStep >= 0 && h->failStep-- == 0) return fail(ICSF_ERR_HIP, "icsf_test_fail_step");
+            return hbGraphable(h) ? hbGraphStep(h) : hbPseudoStep(h);
+        },
+        [&](double* host) { hbQueueResiduals(h, host); }));
     HIPCHK(hipGetLastError());
     return hbErrors(h);
 }

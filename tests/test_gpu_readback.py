@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from icsfoam_amd import cases, dbnsCase
-from icsfoam_amd._lib import check, lib, ptr
+from icsfoam_amd._lib import IcsfError, check, lib, ptr
 from icsfoam_amd.mesh import prepare_case
 from icsfoam_amd.solver import hbCase
 
@@ -57,3 +57,46 @@ def test_field_subsets():
         for i, k in enumerate(("rho", "U", "T", "p", "W")):
             if mask >> i & 1:
                 np.testing.assert_array_equal(out[i], full[k])
+
+
+def _fail_step(case=None, hb=None, step=0):
+    """The next pseudo_steps fails at this step; a test entry beside the
+    interface."""
+    f = lib().icsf_test_fail_step
+    f.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int]
+    check(f(case, hb, step))
+
+
+def _check_kept(kept, step, want):
+    """Residual array left by a call that failed at `step`: the steps before
+    it as asked for alone, those after it untouched."""
+    np.testing.assert_array_equal(kept[:step], want)
+    assert np.isnan(kept[step:]).all()
+
+
+@pytest.mark.parametrize("step", [0, 1, 5, 32, 33, 40])
+def test_failed_step_keeps_the_history_before_it(step):
+    print(f"[history, step {step} fails]", flush=True)
+    c = bump_small(16, 8)
+    a, b = dbnsCase.from_case(c), dbnsCase.from_case(c)
+    h = np.full((45, 10), np.nan)
+    _fail_step(case=a._h, step=step)
+    with pytest.raises(IcsfError):
+        check(lib().icsf_pseudo_steps(a._h, 45, ptr(h), None))
+    _check_kept(h, step, b.pseudo_steps(step))
+    np.testing.assert_array_equal(a.pseudo_steps(3), b.pseudo_steps(3))  # and goes on from there
+
+
+@pytest.mark.parametrize("max_iter", [1, 2])
+def test_failed_hb_step_keeps_the_history_before_it(max_iter):
+    print(f"[hb history, a step fails, {max_iter}]", flush=True)
+    insts, D, _ = cases.case_hb(n=(6, 4, 3), n_harmonics=1)
+    insts = [dataclasses.replace(prepare_case(c, permute_seed=1), fvSolution=cases.solution_dict(
+        co=20.0, nDirections=4, maxIter=max_iter, relTol=1e-6)) for c in insts]
+    a, b = hbCase.from_cases(insts, D), hbCase.from_cases(insts, D)
+    h = np.full((10, 3, 10), np.nan)
+    _fail_step(hb=a._h, step=7)
+    with pytest.raises(IcsfError):
+        check(lib().icsf_hb_pseudo_steps(a._h, 10, ptr(h)))
+    _check_kept(h, 7, b.pseudo_steps(7))
+    np.testing.assert_array_equal(a.pseudo_steps(2), b.pseudo_steps(2))
