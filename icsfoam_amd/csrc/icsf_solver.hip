@@ -2208,15 +2208,11 @@ int icsf_set_fields(icsf_case* c, const double* rho, const double* U, const doub
     return ICSF_OK;
 }
 
-int icsf_get_fields(icsf_case* c, double* rho, double* U, double* T, double* p, double* W) {
-    if (!c) return fail(ICSF_ERR_ARG, "NULL case");
+// Fields of c; q: a work vector of 5 nC entries, free between calls, in which
+// the asked-for entries of the field rows are gathered.
+static int readFields(icsf_case* c, double* q, double* rho, double* U, double* T, double* p, double* W) {
     const size_t nC = c->mv.nC;
     if (rho || p || U) {
-        // the asked-for entries of the field rows, gathered on the device
-        // (a work vector of the case, else a temporary one)
-        DevBuf tmp;
-        double* q = c->t1;
-        if (!q) RC(tmp.alloc(q, 5 * nC));
         k_pack_fields<<<nblk((int)nC, 256), 256, 0, c->st>>>((int)nC, c->sv.fld, q);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(c->st));
@@ -2227,6 +2223,11 @@ int icsf_get_fields(icsf_case* c, double* rho, double* U, double* T, double* p, 
     if (T) HIPCHK(hipMemcpy(T, c->sv.T, nC * sizeof(double), hipMemcpyDeviceToHost));
     if (W) HIPCHK(hipMemcpy(W, c->sv.W, 5 * nC * sizeof(double), hipMemcpyDeviceToHost));
     return ICSF_OK;
+}
+
+int icsf_get_fields(icsf_case* c, double* rho, double* U, double* T, double* p, double* W) {
+    if (!c) return fail(ICSF_ERR_ARG, "NULL case");
+    return readFields(c, c->t1, rho, U, T, p, W);
 }
 
 int icsf_calc_flux(icsf_case* c, double* phi, double* phiUp, double* phiEp) {
@@ -2999,7 +3000,7 @@ int icsf_hb_set_fields(icsf_hb* h, int instant, const double* rho, const double*
 
 int icsf_hb_get_fields(icsf_hb* h, int instant, double* rho, double* U, double* T, double* p, double* W) {
     RC(hbCheckInstance(h, instant));
-    return icsf_get_fields(h->inst[instant], rho, U, T, p, W);
+    return readFields(h->inst[instant], h->t1, rho, U, T, p, W);
 }
 
 // error flags of the coupled diagonal and of every instance

@@ -100,3 +100,21 @@ def test_failed_hb_step_keeps_the_history_before_it(max_iter):
         check(lib().icsf_hb_pseudo_steps(a._h, 10, ptr(h)))
     _check_kept(h, 7, b.pseudo_steps(7))
     np.testing.assert_array_equal(a.pseudo_steps(2), b.pseudo_steps(2))
+
+
+def test_hb_reads_between_steps():
+    """Field read-backs gather in the system's work vector: every instance's
+    own fields, and the steps that follow as without them."""
+    print("[hb reads]", flush=True)
+    insts, D, _ = cases.case_hb(n=(6, 4, 3), n_harmonics=1)
+    insts = [prepare_case(c, permute_seed=1) for c in insts]
+    a, b = hbCase.from_cases(insts, D), hbCase.from_cases(insts, D)
+    h = []
+    for _ in range(4):
+        for J in (2, 0, 1):
+            F = a.fields(J)
+            np.testing.assert_array_equal(F["W"][0], F["rho"])
+            np.testing.assert_allclose(F["W"][2:].T, F["rho"][:, None] * F["U"], rtol=1e-15)
+            np.testing.assert_allclose(F["p"], cases.R_GAS * F["rho"] * F["T"], rtol=1e-14)
+        h.append(a.pseudo_steps(1))
+    np.testing.assert_array_equal(np.concatenate(h), b.pseudo_steps(4))
