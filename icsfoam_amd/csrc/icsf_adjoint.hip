@@ -695,10 +695,9 @@ __device__ __forceinline__ void adjBoundaryFace(const MeshView& m, const Phys& p
     bp[2] = Uc_b.x; bp[3] = Uc_b.y; bp[4] = Uc_b.z;
 }
 
-// Face pass 2 of the geometry adjoint: Gauss-gradient face values (internal
-// faces: adjoint of w*(q_o - q_n) + q_n for the cell pull, Sf part), the
-// boundary faces, and the limiter's Cf part.
-template <bool VISC>
+// Face pass 2 of the geometry adjoint (inviscid): Gauss-gradient face values
+// (internal faces: adjoint of w*(q_o - q_n) + q_n for the cell pull, Sf part),
+// the boundary faces, and the limiter's Cf part.
 __global__ void __launch_bounds__(256) k_adj_gauss(MeshView m, Phys ph, StateView s, AdjView a,
                                                    double* __restrict__ gS, double* __restrict__ gC) {
     const int f = xcdBlock() * blockDim.x + threadIdx.x;
@@ -713,14 +712,12 @@ __global__ void __launch_bounds__(256) k_adj_gauss(MeshView m, Phys ph, StateVie
     const int o = m.own[f];
     V3 bS{0, 0, 0}, bC{0, 0, 0};
     const bool rec = ph.recon == 1;
-    constexpr bool visc = VISC;
     // fields whose Gauss gradient carries an adjoint: the reconstructed ones
-    // (second order) and, viscous, the velocity components
-    const auto grads = [&](int k) { return (used(ph.flux, k) && rec) || (visc && k >= F_UX && k <= F_UZ); };
+    // (second order)
+    const auto grads = [&](int k) { return used(ph.flux, k) && rec; };
     if (f < m.nI) {
         const int n = m.nei[f];
         const double w = m.w[f];
-        if (visc) a.qe[f] = dot(S, ld3(a.Ge + 3 * (size_t)o) - ld3(a.Ge + 3 * (size_t)n));
         // both cells' rows: field values, the limiter faces, and the
         // gradient adjoints two fields (six doubles) at a time
         double fo[NFLD], fn[NFLD], qv[NFLD];
@@ -750,7 +747,7 @@ __global__ void __launch_bounds__(256) k_adj_gauss(MeshView m, Phys ph, StateVie
             }
         }
         stRow(qf, qv);
-    } else adjBoundaryFace<VISC>(m, ph, s, a, f, bS, bC);
+    } else adjBoundaryFace<false>(m, ph, s, a, f, bS, bC);
     gS[3 * (size_t)f] += bS.x; gS[3 * (size_t)f + 1] += bS.y; gS[3 * (size_t)f + 2] += bS.z;
     gC[3 * (size_t)f] += bC.x; gC[3 * (size_t)f + 1] += bC.y; gC[3 * (size_t)f + 2] += bC.z;
 }
@@ -788,6 +785,7 @@ __global__ void __launch_bounds__(256) k_adj_state(MeshView m, Phys ph, StateVie
     V3 Ubnd{0, 0, 0};
     // viscous: direct U and e adjoints of the viscous face terms, and the
     // Gauss face values of e
+    static_assert(DIRECT || !VISC, "the geometry adjoint is inviscid");
     constexpr bool visc = VISC;
     V3 Uv{0, 0, 0}, GeC{0, 0, 0};
     double ecB = 0.0;
@@ -834,11 +832,8 @@ __global__ void __launch_bounds__(256) k_adj_state(MeshView m, Phys ph, StateVie
                 ldRow(a.vis + (size_t)f * NVIS + VS_UO, vu);
                 const int u0 = (isOwn ? VS_UO : VS_UN) - VS_UO;
                 Uv = Uv + V3{vu[u0], vu[u0 + 1], vu[u0 + 2]};
-                double qe;
-                if constexpr (DIRECT) {
-                    const V3 Gj = ld3(a.Ge + 3 * (size_t)j);
-                    qe = dot(S, isOwn ? GeC - Gj : Gj - GeC);
-                } else qe = a.qe[f];
+                const V3 Gj = ld3(a.Ge + 3 * (size_t)j);
+                const double qe = dot(S, isOwn ? GeC - Gj : Gj - GeC);
                 ecB += (isOwn ? vu[VS_EO - VS_UO] : vu[VS_EN - VS_UO]) + wt * qe;
             }
         } else {
@@ -917,8 +912,7 @@ void launchResidualVjp(const MeshView& m, const Phys& ph, const StateView& s, co
         k_adj_cell<true><<<gc2, kAdjCellBlock, 0, st>>>(m, ph, s, a);
     } else k_adj_cell<false><<<gc2, kAdjCellBlock, 0, st>>>(m, ph, s, a);
     if (geom) {
-        // inviscid residuals only
-        k_adj_gauss<false><<<gf, 256, 0, st>>>(m, ph, s, a, gS, gC);
+        k_adj_gauss<<<gf, 256, 0, st>>>(m, ph, s, a, gS, gC);
         k_adj_state<false, false><<<gc, 256, 0, st>>>(m, ph, s, a, gW);
     } else if (ph.viscous) {
         if (gb) k_adj_boundary<true><<<gb, 256, 0, st>>>(m, ph, s, a);

@@ -981,11 +981,19 @@ int adjointSupported(const icsf_case* c) {
     return ICSF_OK;
 }
 
-int adjointPrepare(icsf_case* c) {
+int adjointPrepare(icsf_case* c, bool geom) {
     RC(adjointSupported(c));
-    if (c->adjReady) return ICSF_OK;
     const size_t nC = c->mv.nC, nF = c->mv.nF, nB = std::max(c->mv.nB, 1);
     AdjView& a = c->adj;
+    if (geom && !a.qf) {
+        // with an allocation that fails the next call starts over
+        double* qf;
+        if (!c->adjGS) RC(c->buf.alloc(c->adjGS, 3 * nF));
+        if (!c->adjGC) RC(c->buf.alloc(c->adjGC, 3 * nF));
+        RC(c->buf.alloc(qf, nF * NFLD));
+        a.qf = qf;
+    }
+    if (c->adjReady) return ICSF_OK;
     if (!a.W0) RC(c->buf.alloc(a.W0, 5 * nC));
     RC(c->buf.alloc(a.gun, nC * NFLD * 3));
     RC(c->buf.alloc(a.lim, nC * NFLD));
@@ -996,13 +1004,9 @@ int adjointPrepare(icsf_case* c) {
     RC(c->buf.alloc(a.tval, nC * NFLD));
     RC(c->buf.alloc(a.fst, nC * NFLD));
     RC(c->buf.alloc(a.fext, nC * NFLD));
-    RC(c->buf.alloc(a.qf, nF * NFLD));
     RC(c->buf.alloc(a.bprim, nB * 5));
-    RC(c->buf.alloc(c->adjGS, 3 * nF));
-    RC(c->buf.alloc(c->adjGC, 3 * nF));
     if (c->ph.viscous) {
         RC(c->buf.alloc(a.vis, nF * NVIS));
-        RC(c->buf.alloc(a.qe, nF));
         RC(c->buf.alloc(a.Ge, nC * 3));
     }
     c->adjReady = true;
@@ -1022,7 +1026,7 @@ int stateFromW(icsf_case* c, const double* W, bool keep = true) {
 
 int vjpDevice(icsf_case* c, const double* W, const double* v, double* gW, double* gSf, double* gCf, bool geom) {
     if (!W && !c->haveFields) return fail(ICSF_ERR_STATE, "fields not set");
-    RC(adjointPrepare(c));
+    RC(adjointPrepare(c, geom));
     RC(uploadBC(c));
     RC(stateFromW(c, W));
     launchAdjointForward(c->mv, c->ph, c->sv, c->adj.gun, c->adj.lim, c->st);
@@ -2325,7 +2329,7 @@ int icsf_residual_records_device(icsf_case* c, const double* W, int* faceBranche
     if (!c || !faceBranches || !limiterElement || !limiterFace)
         return fail(ICSF_ERR_ARG, "icsf_residual_records_device: NULL argument");
     if (!W && !c->haveFields) return fail(ICSF_ERR_STATE, "fields not set");
-    RC(adjointPrepare(c));
+    RC(adjointPrepare(c, false));
     RC(uploadBC(c));
     RC(stateFromW(c, W));
     const size_t nC = c->mv.nC, nF = c->mv.nF;
@@ -2337,7 +2341,7 @@ int icsf_residual_records_device(icsf_case* c, const double* W, int* faceBranche
     AdjView a = c->adj;
     a.fbr = faceBranches;
     launchAdjointForward(c->mv, c->ph, c->sv, a.gun, a.lim, c->st);
-    launchResidualVjp(c->mv, c->ph, c->sv, a, v, gW, c->adjGS, c->adjGC, false, c->st);
+    launchResidualVjp(c->mv, c->ph, c->sv, a, v, gW, nullptr, nullptr, false, c->st);
     HIPCHK(hipMemcpyAsync(limiterElement, a.tgt, nC * NFLD * sizeof(int), hipMemcpyDeviceToDevice, c->st));
     HIPCHK(hipMemcpyAsync(limiterFace, a.fst, nC * NFLD * sizeof(int), hipMemcpyDeviceToDevice, c->st));
     HIPCHK(hipGetLastError());
@@ -2368,13 +2372,14 @@ int icsf_residual_vjp_device_noalloc(icsf_case* c, const double* W, const double
         a.tval = sc.take<double>(nC * NFLD);
         a.fst = sc.take<int>(nC * NFLD);
         a.fext = sc.take<double>(nC * NFLD);
-        a.qf = sc.take<double>(nF * NFLD);
         a.bprim = sc.take<double>(nB * 5);
-        gS = sc.take<double>(3 * nF);
-        gC = sc.take<double>(3 * nF);
+        if (gSf || gCf) {
+            a.qf = sc.take<double>(nF * NFLD);
+            gS = sc.take<double>(3 * nF);
+            gC = sc.take<double>(3 * nF);
+        }
         if (c->ph.viscous) {
             a.vis = sc.take<double>(nF * NVIS);
-            a.qe = sc.take<double>(nF);
             a.Ge = sc.take<double>(nC * 3);
         }
     };

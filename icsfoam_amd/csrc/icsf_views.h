@@ -178,7 +178,8 @@ struct AdjView {
     double* tval;   // [nC][NFLD] adjoint sent to that element
     int* fst;       // [nC][NFLD] face that set the limiter, -1 none
     double* fext;   // [nC][NFLD] adjoint of that face's extrapolation
-    double* qf;     // [nF][NFLD] adjoint of the Gauss face values (internal faces)
+    double* qf;     // [nF][NFLD] adjoint of the Gauss face values (internal faces;
+                    //   geometry adjoint, null without)
     double* bprim;  // [nB][5] boundary adjoint forwarded to the owner's p, T, U
     int* fbr;       // [nF] branch bits of each face's flux (records for derivative
                     //   checks; null: not written)
@@ -189,7 +190,6 @@ struct AdjView {
                     //   owner and of the neighbour; boundary faces grad(U) of the
                     //   owner (9), 0 (3), U of the owner (3), the boundary U (3), e
                     //   of the owner, the boundary e
-    double* qe;     // [nF] adjoint of the Gauss face value of e (internal faces)
     double* Ge;     // [nC][3] adjoint of the Gauss sum of grad(e), divided by V
 };
 enum { VS_Z = 0, VS_GE = 9, VS_UO = 12, VS_UN = 15, VS_EO = 18, VS_EN = 19, NVIS = 20 };

@@ -247,8 +247,9 @@ int icsf_residual_vjp_device(icsf_case* c, const double* W, const double* v, dou
 /* icsf_residual_vjp_device without any device allocation (no counterpart
  * in the reference;
  * for callers that cannot allocate: code under HIP graph capture, serving
- * loops): the adjoint's work buffers (about 750 bytes per cell and 240 per
- * face, 24 and 170 more with the viscous terms) live in one fixed 128 MiB
+ * loops): the adjoint's work buffers (about 750 bytes per cell and 130 per
+ * face; 112 per face more with gSf or gCf, 24 per cell and 160 per face more
+ * with the viscous terms) live in one fixed 128 MiB
  * array per GPU, held until the process ends; cases needing more are
  * rejected with ICSF_ERR_ARG.  The case's device must be current.  Calls on
  * one GPU share the array and must not overlap; results are those of

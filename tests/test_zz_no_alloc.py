@@ -77,3 +77,19 @@ def test_noalloc_vjp_rejects_cases_beyond_the_scratch():
     W = g.fields()["W"]
     with pytest.raises(IcsfError, match="scratch"):
         _run(L.icsf_residual_vjp_device_noalloc, g, W, np.ones_like(W), False)
+
+
+def test_noalloc_vjp_takes_the_geometry_buffers_only_when_asked():
+    """A case whose buffers fit the array without the Sf/Cf adjoint and not
+    with it; the allocating form makes them on the first call that asks."""
+    L = _bind()
+    print("[noalloc vjp 46^3]", flush=True)
+    c = _case((46, 46, 46), 6)
+    g = dbnsCase.from_case(c)
+    W = generic_state(g.fields()["W"], 6)
+    v = np.random.default_rng(6).standard_normal(W.shape)
+    ref = _run(L.icsf_residual_vjp_device, g, W, v, False)
+    np.testing.assert_array_equal(_run(L.icsf_residual_vjp_device_noalloc, g, W, v, False)[0], ref[0])
+    with pytest.raises(IcsfError, match="scratch"):
+        _run(L.icsf_residual_vjp_device_noalloc, g, W, v, True)
+    np.testing.assert_array_equal(_run(L.icsf_residual_vjp_device, g, W, v, True)[0], ref[0])
