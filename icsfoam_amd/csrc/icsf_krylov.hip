@@ -763,7 +763,7 @@ __global__ void __launch_bounds__(64) k_sweep(MeshView m, const TB* __restrict__
             unsigned miss = 0;
 #pragma unroll
             for (int u = 0; u < UN; ++u) miss |= ok && k + u < n ? 1u << u : 0u;
-            for (int polls = 0; __any(miss);) {
+            for (int polls = 0; ok;) {
 #pragma unroll
                 for (int u = 0; u < UN; ++u)
                     if (miss & (1u << u)) {
@@ -776,7 +776,8 @@ __global__ void __launch_bounds__(64) k_sweep(MeshView m, const TB* __restrict__
                         }
                         if (got) miss &= ~(1u << u);
                     }
-                if (__any(miss) && ++polls > limit) { ok = false; break; }
+                if (!__any(miss)) break;
+                ok = ++polls <= limit;
             }
 #pragma unroll
             for (int u = 0; u < UN; ++u) {
