@@ -2,7 +2,8 @@
 and state update, against the oracle: the smallest and largest instance
 counts, cell counts on both sides of where the average is formed without a
 launch of its own (32 768) and a last block with few cells.  And the time-step
-bound's kernels where some cells are out of bounds, against the single case."""
+bound's kernels where some cells are out of bounds: one instance against the
+single case, several against the oracle, with phase-lagged patches too."""
 import dataclasses
 
 import numpy as np
@@ -47,3 +48,48 @@ def test_bound_kernels_match_single_case():
     np.testing.assert_array_equal(np.concatenate([h.pseudo_steps(1)[:, 0], h.pseudo_steps(2)[:, 0]]),
                                   np.concatenate([rs, s.pseudo_steps(2)]))
     np.testing.assert_array_equal(h.fields(0)["W"], s.fields()["W"])
+
+
+@pytest.mark.parametrize("lag", [False, True])
+def test_bound_of_each_instance(lag):
+    """Three instances with different cells out of bounds (the first and the
+    last cells among them) and, with phase-lagged patches half a period
+    apart, lagged densities out of bounds in one: after a step every
+    instance's own Courant numbers show in its operator, bit for bit as the
+    oracle's (the fields given anew, so that nothing else differs)."""
+    print(f"[hb bound, instances, lag={lag}]", flush=True)
+    insts, D, t = cases.case_hb(n=(8, 6, 5), n_harmonics=1, flux="ROE", jitter=0.1)
+    m = insts[0].mesh
+    w = 2 * np.pi * 100.0
+    if lag:
+        lo = next(i for i, p in enumerate(m.patches) if p.kind == cases.PATCH_CYCLIC)
+        pair = cases.PhaseLagPair(owner=lo, ibpa=np.pi, frequencies=np.array([w]), harmonics=np.array([1]),
+                                  instants=t, cyl_coords=True)
+        insts = [dataclasses.replace(c, phase_lag=pair, rho=c.rho * (1 + 0.2 * np.sin(w * t[J])))
+                 for J, c in enumerate(insts)]
+    insts = [prepare_case(dataclasses.replace(c, fvSolution=cases.solution_dict(co=5.0, nDirections=10)),
+                          permute_seed=3) for c in insts]
+    n = m.n_cells
+    out = [np.r_[0, 3:6], np.r_[100:103], np.r_[n - 3:n]]
+    low = []
+    for J, c in enumerate(insts):
+        T, U = np.array(c.T), np.array(c.U)
+        T[out[J]], U[out[J]] = 1e-20, 0.0
+        low.append(dataclasses.replace(c, T=T, U=U))
+    g, o = hbCase.from_cases(low, D), OracleHB(low, D)
+    for patch, Dl in getattr(g, "phase_lag_sides", []):
+        o.set_phase_lag(patch, Dl, cyl=True, axis=pair.axis, origin=pair.centre)
+    g.pseudo_steps(1)
+    o.pseudo_steps(1)
+    co = [o.inst[J].pseudoCo() for J in range(3)]
+    assert all(len(np.unique(q)) == 3 for q in co)
+    if lag:  # cells on the lagged patches of one instance beside no cell out of bounds
+        assert (co[1] != 5.0).sum() > (co[0] != 5.0).sum() + 10
+    for J, c in enumerate(insts):
+        g.set_fields(J, c.rho, c.U, c.T)
+        o.inst[J].set_fields(c.rho, c.U, c.T)
+    np.testing.assert_array_equal(g.residual(), o.residual())
+    g.createJacobian()
+    o.createJacobian()
+    x = np.random.default_rng(4).standard_normal((3, 5, n))
+    np.testing.assert_array_equal(g.matrixMul(x), o.matrixMul(x))
