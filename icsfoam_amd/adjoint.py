@@ -95,7 +95,8 @@ class ResidualFunction(torch.autograd.Function):
 
 
 def residual(case, W: torch.Tensor) -> torch.Tensor:
-    """Differentiable b(W) of the inviscid AUSM+up residual."""
+    """Differentiable b(W) of the case's residual (AUSM+up, Roe or HLLC,
+    inviscid or viscous)."""
     return ResidualFunction.apply(W, case)
 
 

@@ -31,9 +31,12 @@ struct Levels {
 };
 // Largest average number of cells per level swept in one dataflow launch: a
 // launch per level costs the same up to there (its latency), while the
-// dataflow's uncached loads add up.  Pseudo-step with a launch per level / in
-// one launch: 813 cells per level 11.5 / 7.5 ms, 2600 101 / 60 ms, 3800 14.4 /
-// 10.3 ms, 13800 26.0 / 23.7 ms in FP64 but 20.3 / 20.7 ms mixed.
+// dataflow's uncached loads add up.  Boxes in random order (34 to 42 levels),
+// pseudo-step with a launch per level / in one launch: 3770 cells per level
+// FP64 14.1 / 10.5 ms, mixed 11.7 / 10.0; 8270 17.0 / 13.6, 14.1 / 12.5; 9760
+// 19.5 / 16.6, 15.9 / 14.8; 12700 21.8 / 20.0, 17.3 / 17.8; 13800 25.5 / 23.7,
+// 19.8 / 20.6; 17800 34.4 / 32.8, 26.5 / 28.5.  One line for both precisions,
+// on the side of mixed, which crosses near 11000.
 constexpr int kSweepLevelCells = 8192;
 // Fewest levels (forward and backward together) for it: the 28 059-cell LS89
 // mesh coloured (4 + 4 levels) steps in 2.36 ms with its 7 launches per

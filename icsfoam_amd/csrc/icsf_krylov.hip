@@ -1430,7 +1430,13 @@ void launchSpmv(const MeshView& m, int blkFp32, int vecFp32, const void* blk, co
 // 1.643 ms, 64^3 4.43 / 4.48 ms; mixed 48^3 1.90 / 1.74 ms, 64^3 3.08 /
 // 3.12 ms.
 constexpr size_t kOpLatencyRows = 65536;
-// Cells (instances included) from which a norm is summed by a launch of its own.
+// Cells (instances included) from which a norm is summed by a launch of its
+// own (and the update takes its large form, updateBlocks).  Pseudo-step, own
+// launch / merged: 125 000 cells FP64 2.79 / 2.66 ms, mixed 1.99 / 1.86 ms;
+// 195 000 3.78 / 3.70, 2.70 / 2.58; 262 000 4.44 / 4.43, 2.97 / 2.95; 512 000
+// 8.18 / 8.10, 4.98 / 4.97; 1 000 000 15.15 / 15.09, 8.86 / 8.80: the line lies
+// where the gain has fallen to a percent, and above it the first phase grows
+// by what the launch saves (gmresCycleT).
 constexpr int kNormMergeCells = 200000;
 
 template <typename TB, bool GEN, bool HB, int UN, int W>

@@ -743,7 +743,7 @@ int solveStage(icsf_case* c, const double* W, const double* b, int& nIter) {
 // timed with HIP events on the case stream over its candidates and the
 // fastest kept: workgroup sizes 64/128/256 of the face-terms, gradient,
 // cell-sums + Jacobian-row and Arnoldi-operator kernels, and 8/16/32
-// basis vectors per CGS projection pass.  Only scratch vectors are written
+// basis vectors per projection workgroup.  Only scratch vectors are written
 // (or state is recomputed identically); no candidate changes a result bit.
 int autotune(icsf_case* c) {
     {

@@ -32,7 +32,8 @@ extern "C" {
                                     entry above 1/VSMALL (as the reference tests it; an all-zero
                                     diagonal gives 1/SMALL there and passes) or not a number */
 #define ICSF_ERR_NONFINITE (-4)  /* non-finite input value, residual or conserved state */
-#define ICSF_ERR_HIP (-5)        /* HIP runtime failure */
+#define ICSF_ERR_HIP (-5)        /* HIP runtime failure, or an LU-SGS sweep on the device that gave up
+                                    waiting (the call's results are then not to be used) */
 #define ICSF_ERR_STATE (-6)      /* call-order error (e.g. solve before assemble) */
 #define ICSF_ERR_NODEVICE (-7)   /* no HIP device available */
 
