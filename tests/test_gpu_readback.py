@@ -59,6 +59,25 @@ def test_field_subsets():
                 np.testing.assert_array_equal(out[i], full[k])
 
 
+@pytest.mark.parametrize("nx,ny", [(102, 100), (128, 80), (128, 81), (160, 81)])
+def test_field_subsets_on_both_sides_of_the_gather(nx, ny):
+    """Cell counts around 10 240, above which the device gathers rho, p, U."""
+    print(f"[fields {nx} x {ny}]", flush=True)
+    g = dbnsCase.from_case(bump_small(nx, ny))
+    g.pseudo_steps(1)
+    n = g.nCells
+    full = g.fields()
+    np.testing.assert_array_equal(full["W"][0], full["rho"])
+    np.testing.assert_allclose(full["W"][2:].T, full["rho"][:, None] * full["U"], rtol=1e-15)
+    np.testing.assert_allclose(full["p"], cases.R_GAS * full["rho"] * full["T"], rtol=1e-14)
+    for mask in (1, 2, 8, 11, 18, 25):
+        out = [np.empty(n), np.empty((n, 3)), np.empty(n), np.empty(n), np.empty((5, n))]
+        check(lib().icsf_get_fields(g._h, *[ptr(x) if mask >> i & 1 else None for i, x in enumerate(out)]))
+        for i, k in enumerate(("rho", "U", "T", "p", "W")):
+            if mask >> i & 1:
+                np.testing.assert_array_equal(out[i], full[k])
+
+
 def _fail_step(case=None, hb=None, step=0):
     """The next pseudo_steps fails at this step; a test entry beside the
     interface."""
@@ -102,11 +121,12 @@ def test_failed_hb_step_keeps_the_history_before_it(max_iter):
     np.testing.assert_array_equal(a.pseudo_steps(2), b.pseudo_steps(2))
 
 
-def test_hb_reads_between_steps():
+@pytest.mark.parametrize("n", [(6, 4, 3), (24, 22, 20)])
+def test_hb_reads_between_steps(n):
     """Field read-backs gather in the system's work vector: every instance's
     own fields, and the steps that follow as without them."""
-    print("[hb reads]", flush=True)
-    insts, D, _ = cases.case_hb(n=(6, 4, 3), n_harmonics=1)
+    print(f"[hb reads {n}]", flush=True)
+    insts, D, _ = cases.case_hb(n=n, n_harmonics=1)
     insts = [prepare_case(c, permute_seed=1) for c in insts]
     a, b = hbCase.from_cases(insts, D), hbCase.from_cases(insts, D)
     h = []
