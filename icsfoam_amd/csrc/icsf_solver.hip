@@ -985,31 +985,29 @@ int adjointPrepare(icsf_case* c, bool geom) {
     RC(adjointSupported(c));
     const size_t nC = c->mv.nC, nF = c->mv.nF, nB = std::max(c->mv.nB, 1);
     AdjView& a = c->adj;
-    if (geom && !a.qf) {
-        // with an allocation that fails the next call starts over
-        double* qf;
+    if (!c->adjReady) {
+        if (!a.W0) RC(c->buf.alloc(a.W0, 5 * nC));
+        RC(c->buf.alloc(a.gun, nC * NFLD * 3));
+        RC(c->buf.alloc(a.lim, nC * NFLD));
+        RC(c->buf.alloc(a.fLR, nF * 2 * NFLD));
+        RC(c->buf.alloc(a.G, nC * NFLD * 3));
+        RC(c->buf.alloc(a.qc, nC * NFLD));
+        RC(c->buf.alloc(a.tgt, nC * NFLD));
+        RC(c->buf.alloc(a.tval, nC * NFLD));
+        RC(c->buf.alloc(a.fst, nC * NFLD));
+        RC(c->buf.alloc(a.fext, nC * NFLD));
+        RC(c->buf.alloc(a.bprim, nB * 5));
+        if (c->ph.viscous) {
+            RC(c->buf.alloc(a.vis, nF * NVIS));
+            RC(c->buf.alloc(a.Ge, nC * 3));
+        }
+        c->adjReady = true;
+    }
+    if (geom) {
+        if (!a.qf) RC(c->buf.alloc(a.qf, nF * NFLD));
         if (!c->adjGS) RC(c->buf.alloc(c->adjGS, 3 * nF));
         if (!c->adjGC) RC(c->buf.alloc(c->adjGC, 3 * nF));
-        RC(c->buf.alloc(qf, nF * NFLD));
-        a.qf = qf;
     }
-    if (c->adjReady) return ICSF_OK;
-    if (!a.W0) RC(c->buf.alloc(a.W0, 5 * nC));
-    RC(c->buf.alloc(a.gun, nC * NFLD * 3));
-    RC(c->buf.alloc(a.lim, nC * NFLD));
-    RC(c->buf.alloc(a.fLR, nF * 2 * NFLD));
-    RC(c->buf.alloc(a.G, nC * NFLD * 3));
-    RC(c->buf.alloc(a.qc, nC * NFLD));
-    RC(c->buf.alloc(a.tgt, nC * NFLD));
-    RC(c->buf.alloc(a.tval, nC * NFLD));
-    RC(c->buf.alloc(a.fst, nC * NFLD));
-    RC(c->buf.alloc(a.fext, nC * NFLD));
-    RC(c->buf.alloc(a.bprim, nB * 5));
-    if (c->ph.viscous) {
-        RC(c->buf.alloc(a.vis, nF * NVIS));
-        RC(c->buf.alloc(a.Ge, nC * 3));
-    }
-    c->adjReady = true;
     return ICSF_OK;
 }
 
